@@ -18,7 +18,7 @@
 //   EO driver source b_o - D_oe R^-1 b_e and even reconstruction
 //   R_ee^-1 (b_e - D_eo x_o)                  diag = 1, hop_sign = -1 [, INV]
 // (PreconditionedBiCGStab.cpp:56-86).
-#include "lym_device.h"
+#include "lym_stencil.h"
 
 // Launch shape of the stencil (swept on the device; defaults are the measured best)
 #ifndef LYM_DSLASH_THREADS
@@ -35,21 +35,6 @@
 #ifndef LYM_SWEEP_MAX_BLOCKS
 #define LYM_SWEEP_MAX_BLOCKS 1024
 #endif
-// 1: each XCD works through its own contiguous range of site blocks;
-// 0: all XCDs advance together through the lattice in block order
-#ifndef LYM_XCD_MAP
-#define LYM_XCD_MAP 1
-#endif
-// 1: within its block range an XCD takes the x-slices as the fastest index of
-// its sweep (block j of every x-slice of the range, then block j + 1, ...), so
-// the workgroups in flight together hold x-adjacent planes and the neighbour
-// spinors and backward links of the x hops are read while still in L2;
-// 0: plain block order within the range (one whole x-slice after the other).
-// Measured on the 16^3x32 FP64 clover apply: L2 misses 277 -> 236-250 MB per
-// apply, 49.5 -> 47.2 us; even-odd applies and solves gain alike.
-#ifndef LYM_XSWEEP
-#define LYM_XSWEEP 1
-#endif
 // 1: single-RHS FP32/FP16 applies of at most LYM_SPLIT_MAX_SITES sites per
 // parity run two threads per site (k_dslash_split).  Measured: mixed CG on
 // 16^3x32 (65536 sites) 5 % faster, on 24^3x48 (331776) 4 % slower
@@ -58,14 +43,6 @@
 #endif
 #ifndef LYM_SPLIT_MAX_SITES
 #define LYM_SPLIT_MAX_SITES 131072
-#endif
-// 1: XCDs 2i and 2i+1 share the x-slices of both their ranges, each taking half
-// of every slice's site blocks, so an XCD's domain is 4 x-slices by half the
-// (y, z) blocks instead of 2 whole x-slices: 3/4 of the halo spinors and
-// links.  Measured on the 16^3x32 FP64 clover apply: 252 -> 221 MB read,
-// 47.1 -> 44.6 us; even-odd launches 68.4 -> 65.8 us.
-#ifndef LYM_XCD_PAIRS
-#define LYM_XCD_PAIRS 1
 #endif
 // Full-lattice applies: odd-parity sites take each direction's backward hop
 // before its forward hop, so the two reads of a link U_mu(y) -- by y (forward)
@@ -110,80 +87,6 @@
 #endif
 
 namespace lym {
-
-template <int MU>
-struct Dir;
-// (1 - gamma_mu) keeps h_a = psi_a + c_a psi_{P_a} for a = 0, 1; c = i^C.
-template <>
-struct Dir<0> { static constexpr int P0 = 3, C0 = 1, P1 = 2, C1 = 1; };
-template <>
-struct Dir<1> { static constexpr int P0 = 3, C0 = 0, P1 = 2, C1 = 2; };
-template <>
-struct Dir<2> { static constexpr int P0 = 2, C0 = 1, P1 = 3, C1 = 3; };
-template <>
-struct Dir<3> { static constexpr int P0 = 2, C0 = 2, P1 = 3, C1 = 2; };
-
-// forward:  h_a = psi_a + c_a psi_P, acc_a += U h_a, acc_P += conj(c_a) U h_a
-// backward: h_a = psi_a - c_a psi_P, acc_a += U^+ h_a, acc_P -= conj(c_a) U^+ h_a
-// SCALED: psi is an unscaled FP16 spinor and sc its site scale, applied (with
-// the boundary sign) to the two colour vectors after the link multiply
-template <int MU, bool FWD, int LK, class T, bool SCALED = false>
-__device__ __forceinline__ void hop_dir(cplx<T> acc[12], const cplx<T> psi[12], const LinkMat<LK, T>& L, bool flip,
-                                        T sc = (T)1) {
-    using D = Dir<MU>;
-    constexpr int PH0 = FWD ? D::C0 : D::C0 + 2;
-    constexpr int PH1 = FWD ? D::C1 : D::C1 + 2;
-    constexpr int Q0 = FWD ? 4 - D::C0 : 6 - D::C0;
-    constexpr int Q1 = FWD ? 4 - D::C1 : 6 - D::C1;
-    cplx<T> h0[3], h1[3], r0[3], r1[3];
-    if constexpr (SCALED) {
-        // FP16 operands: each component of h = psi_a + c psi_P as a fused
-        // multiply-add by a unit the compiler cannot see through, so that the
-        // conversions of both FP16 operands fold into one mixed-precision
-        // instruction instead of two conversions and an add.  The value is
-        // the same: the product by one is exact and the sum rounds once.
-        T one = (T)1;
-        asm volatile("" : "+v"(one));
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const cplx<T> m0 = mulph<PH0>(psi[3 * D::P0 + c]), m1 = mulph<PH1>(psi[3 * D::P1 + c]);
-            h0[c] = mk(fmadd(m0.re, one, psi[c].re), fmadd(m0.im, one, psi[c].im));
-            h1[c] = mk(fmadd(m1.re, one, psi[3 + c].re), fmadd(m1.im, one, psi[3 + c].im));
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            h0[c] = psi[c] + mulph<PH0>(psi[3 * D::P0 + c]);
-            h1[c] = psi[3 + c] + mulph<PH1>(psi[3 * D::P1 + c]);
-            if (flip) {
-                h0[c] = -h0[c];
-                h1[c] = -h1[c];
-            }
-        }
-    }
-    if constexpr (FWD) {
-        matvec<LK, T>(L, h0, r0);
-        matvec<LK, T>(L, h1, r1);
-    } else {
-        matvec_dag<LK, T>(L, h0, r0);
-        matvec_dag<LK, T>(L, h1, r1);
-    }
-    if constexpr (SCALED) {
-        const T f = flip ? -sc : sc;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            r0[c] = f * r0[c];
-            r1[c] = f * r1[c];
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        acc[c] = acc[c] + r0[c];
-        acc[3 + c] = acc[3 + c] + r1[c];
-        acc[3 * D::P0 + c] = acc[3 * D::P0 + c] + mulph<Q0>(r0[c]);
-        acc[3 * D::P1 + c] = acc[3 * D::P1 + c] + mulph<Q1>(r1[c]);
-    }
-}
 
 // Empty asm that reads and writes the accumulator and clobbers memory: the
 // hop of one direction must finish before the next direction's loads are
@@ -336,7 +239,7 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
         herm6_packed<PR>(Ab_, 4 * (size_t)ST, (size_t)(2 * p) * ST, site, sc, s, t);
         herm6_packed<PR>(Ab_, 4 * (size_t)ST, (size_t)(2 * p + 1) * ST, site, sc, s + 6, t + 6);
 #pragma unroll
-        for (int k = 0; k < 12; ++k) v[k] = t[k] + hk * acc[k];
+        for (int k = 0; k < 12; ++k) v[k] = axpy1(hk, acc[k], t[k]);
     } else {
         cplx<T> s[12];
         load_spinor<PR>(SpinorRef<PR>{reinterpret_cast<const S*>(a.diag_in[p]), a.diag_sc[p]}, ST, a.nr, site, r, s);
@@ -346,10 +249,10 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
             herm6<PR>(Ab, ST, site, (T)1, s, t);
             herm6<PR>(Ab + (size_t)18 * ST, ST, site, (T)1, s + 6, t + 6);
 #pragma unroll
-            for (int k = 0; k < 12; ++k) v[k] = t[k] + hk * acc[k];
+            for (int k = 0; k < 12; ++k) v[k] = axpy1(hk, acc[k], t[k]);
         } else {
 #pragma unroll
-            for (int k = 0; k < 12; ++k) v[k] = s[k] + hk * acc[k];
+            for (int k = 0; k < 12; ++k) v[k] = axpy1(hk, acc[k], s[k]);
         }
     }
     if constexpr (INV) {
@@ -375,7 +278,7 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
         load_spinor<PR, true>(SpinorRef<PR>{reinterpret_cast<const S*>(a.v2[p]), a.v2_sc[p]}, ST, a.nr, site, r, w);
         const cplx<T> al = mk((T)a.alpha.re, (T)a.alpha.im);
 #pragma unroll
-        for (int k = 0; k < 12; ++k) v[k] = v[k] + al * w[k];
+        for (int k = 0; k < 12; ++k) cfma(v[k], al, w[k]);
     }
     if constexpr (BM == 2) {
         // batch lane r: x_s += alpha_r p, r_s -= alpha_r v (v in FP32, never
@@ -387,18 +290,15 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
         cplx<float>* xs = reinterpret_cast<cplx<float>*>(a.upd_xs[p]);
         cplx<float>* rs = reinterpret_cast<cplx<float>*>(a.upd_rs[p]);
         const size_t o = (size_t)site * a.nr + r, ks = (size_t)ST * a.nr;
-        double n2 = 0;
+        double n2[6] = {0, 0, 0, 0, 0, 0};  // per pair of components, as the one-wave-per-direction form sums them
 #pragma unroll
         for (int k = 0; k < 12; ++k) {
-            cplx<float> x = xs[k * ks + o];
-            cplx<float> rr = rs[k * ks + o];
-            x = x + al * pv[k];
-            rr = rr - al * v[k];
-            xs[k * ks + o] = x;
+            const cplx<float> rr = axpy1(-al, v[k], rs[k * ks + o]);
+            xs[k * ks + o] = axpy1(al, pv[k], xs[k * ks + o]);
             rs[k * ks + o] = rr;
-            n2 += (double)rr.re * rr.re + (double)rr.im * rr.im;
+            n2[k / 2] = norm_acc(mk((double)rr.re, (double)rr.im), n2[k / 2]);
         }
-        a.bsite[p][o] = n2;
+        a.bsite[p][o] = ((((n2[0] + n2[1]) + n2[2]) + n2[3]) + n2[4]) + n2[5];
         return 0;
     }
     if constexpr (UPD) {
@@ -423,10 +323,10 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
     }
     store_spinor<PR>(SpinorOut<PR>{reinterpret_cast<S*>(a.out[p]), a.out_sc[p]}, ST, a.nr, site, r, v);
     if constexpr (BM == 1) {  // lane r's |v|^2 at this site: the 24 squares in FP32
-        float n2 = 0.f;
+        float n2[2] = {0.f, 0.f};
 #pragma unroll
-        for (int k = 0; k < 12; ++k) n2 += v[k].re * v[k].re + v[k].im * v[k].im;
-        a.bsite[p][(size_t)site * a.nr + r] = (double)n2;
+        for (int k = 0; k < 12; ++k) n2[k / 6] = norm_acc(v[k], n2[k / 6]);
+        a.bsite[p][(size_t)site * a.nr + r] = (double)(n2[0] + n2[1]);
     }
     if constexpr (NORM) {  // the site's 24 squares in FP32, the sum over sites in FP64
         float n2 = 0.f;
@@ -453,91 +353,6 @@ __device__ __forceinline__ void block_sum_store(double v, double* out) {
     }
 }
 
-// Grid: gridDim.x workgroups dealt round-robin over the 8 XCDs.  XCD x owns a
-// contiguous range of logical site blocks (x-major lattice order, the two
-// parities of a block range interleaved) and its workgroups sweep that range
-// in order, so at any time an XCD works on one compact slab and the
-// neighbour spinors and links of that slab are reused from its L2.  A
-// workgroup holds `spb` sites x `nr` right-hand sides, rhs fastest.
-// (The mapping functions take the workgroup index and grid size as arguments so
-// that the host can evaluate the same mapping: lym_launch_plan below.)
-struct BlockSweep {
-    int lo, hi, k, nphys;
-};
-__host__ __device__ __forceinline__ BlockSweep block_sweep_at(const DslashParams& a, int bx, int gdim) {
-    const int nbt = a.nblocks_per_parity * (a.parity >= 0 ? 1 : 2);
-    BlockSweep b;
-#if LYM_XCD_MAP
-    const int nx = 8;
-    const int xcd = bx % nx;
-    b.k = bx / nx;
-    b.nphys = (gdim - xcd + nx - 1) / nx;  // workgroups on this XCD
-    const int q = nbt / nx, rr = nbt % nx;
-    b.lo = xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q;
-    b.hi = b.lo + (xcd < rr ? q + 1 : q);
-#else
-    // plain order: consecutive workgroups (dealt round-robin over the XCDs) take
-    // consecutive site blocks, so all XCDs advance one front through the lattice
-    // and the neighbour slices they re-read are recent in the shared Infinity Cache
-    b.k = bx;
-    b.nphys = gdim;
-    b.lo = 0;
-    b.hi = nbt;
-#endif
-    return b;
-}
-
-// Which renumbering block_of_at applied (reported by lym_launch_plan)
-enum { MAP_PLAIN = 0, MAP_XSLICE = 1, MAP_XCD_PAIRS = 2 };
-
-// logical block lb of the sweep of workgroup bx -> parity p and site block bi
-// of that parity; returns the MAP_* branch taken
-__host__ __device__ __forceinline__ int block_of_at(const DslashParams& a, const BlockSweep& b, int lb, int bx, int& p,
-                                                    int& bi) {
-    (void)bx;
-    if (a.parity >= 0) {
-        p = a.parity;
-        bi = lb;
-    } else {
-        p = lb & 1;
-        bi = lb >> 1;
-    }
-#if LYM_XSWEEP && LYM_XCD_MAP
-    {
-        // the range holds whole x-slices: renumber its blocks x-slice fastest
-        const int W = a.xslice_blocks;
-        const int b0 = a.parity >= 0 ? b.lo : b.lo >> 1;
-        const int D = a.parity >= 0 ? b.hi - b.lo : (b.hi - b.lo) >> 1;
-        const bool whole = a.parity >= 0 || ((b.lo | b.hi) & 1) == 0;
-#if LYM_XCD_PAIRS
-        // XCDs 2i and 2i+1 share the x-slices of both their ranges, each taking
-        // half of every slice's blocks (a 2-D domain: shorter x halo)
-        const int nbt = a.nblocks_per_parity * (a.parity >= 0 ? 1 : 2);
-        if (W > 0 && whole && W % 2 == 0 && nbt % 16 == 0 && b0 % W == 0 && D % W == 0) {
-            const int x1 = (bx % 8) & 1;
-            const int b0p = b0 - x1 * D, nxs2 = 2 * D / W, Wh = W / 2;
-            const int u = bi - b0, j = u / nxs2;
-            bi = b0p + (u - j * nxs2) * W + x1 * Wh + j;
-            return MAP_XCD_PAIRS;
-        }
-#endif
-        if (W > 0 && whole && b0 % W == 0 && D % W == 0 && D > W) {
-            const int u = bi - b0, nxs = D / W;
-            const int j = u / nxs;
-            bi = b0 + (u - j * nxs) * W + j;
-            return MAP_XSLICE;
-        }
-    }
-#endif
-    return MAP_PLAIN;
-}
-
-__device__ __forceinline__ BlockSweep block_sweep(const DslashParams& a) {
-    return block_sweep_at(a, (int)blockIdx.x, (int)gridDim.x);
-}
-__device__ __forceinline__ void block_of(const DslashParams& a, const BlockSweep& b, int lb, int& p, int& bi) {
-    (void)block_of_at(a, b, lb, (int)blockIdx.x, p, bi);
-}
 
 // The fused update's step: alpha = rr_s / (sum of the n <p, Ap> partials),
 // folded by every workgroup in one fixed order (so all get the same alpha);
@@ -1184,20 +999,56 @@ static int plan_dslash(DslashParams& a) {
     return nblocks;
 }
 
+// Launches of at most this many (site, RHS) lanes take the one-wave-per-direction
+// form (dslash_hop.hip).  Measured, that form against the other: half-lattice
+// launches, time of an FP64 even-odd CG / FP16 mixed CG iteration: 83 against
+// 91 us / 48 against 57 us at 32768 lanes, 147 against 141 us / 78 against 67 us
+// at 65536; batched FP16 solves of 4 RHS 5.9 against 7.0 ms at 41472 lanes, 10.9
+// against 9.9 ms at 131072.  Full-lattice FP64 applies: 10.2 against 13.6 us at
+// 20736 lanes (clover), 14.3 against 12.5 us at 41472 (Wilson).
+#ifndef LYM_HOP_MAX_HALF
+#define LYM_HOP_MAX_HALF 49152
+#endif
+#ifndef LYM_HOP_MAX_FULL
+#define LYM_HOP_MAX_FULL 32768
+#endif
+
+// The launch geometry of that form: sites per workgroup and site blocks per
+// parity; returns the number of workgroups, or 0 when the launch takes another.
+static int plan_hop(DslashParams& a) {
+    const int par = a.parity >= 0 ? 1 : 2;
+    const long lanes = (long)a.g.Vh * a.nr * par;
+    if (LYM_T_SLOW || a.mfma || a.nr > 64 || lanes > (par == 1 ? LYM_HOP_MAX_HALF : LYM_HOP_MAX_FULL)) return 0;
+    a.spb = 64 / a.nr;
+    // tiny launches: fewer sites per workgroup, so that more CUs share the loads
+    while (a.spb > 1 && a.spb * a.nr > 16 && (a.g.Vh + a.spb - 1) / a.spb * par < 256) a.spb = (a.spb + 1) / 2;
+    a.nblocks_per_parity = (a.g.Vh + a.spb - 1) / a.spb;
+    a.inv_ext[0] = 1.0 / a.g.L[1];
+    a.inv_ext[1] = 1.0 / a.g.L[2];
+    a.inv_ext[2] = 1.0 / a.g.Lth;
+    return a.nblocks_per_parity * par;
+}
+
 int launch_dslash(DslashParams a, int link_kind, int diag, bool inv, hipStream_t st) {
     const int threads = (a.threads > 0 && a.threads <= LYM_DSLASH_THREADS) ? a.threads : LYM_DSLASH_THREADS;
-    const int nblocks = plan_dslash(a);
+    if (a.nr < 1) a.nr = 1;
+    const int hop_blocks = plan_hop(a);
+    const int nblocks = hop_blocks ? hop_blocks : plan_dslash(a);
     // output norm partials: low precision only, one per workgroup, and only
     // when the caller's buffer holds one per workgroup of this launch
     // (the workgroup sum shuffles over whole 64-lane waves)
-    if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || threads % 64 != 0 ||
-        nblocks > a.norm_max)
+    const bool whole_waves = hop_blocks || threads % 64 == 0;
+    if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || !whole_waves || nblocks > a.norm_max)
         a.norm_partials = nullptr;
     // the fused update: under the same conditions (the caller checks the return
     // value and runs the separate update when it is 0)
-    if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || a.lane_ops || threads % 64 != 0 ||
+    if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || a.lane_ops || !whole_waves ||
         nblocks > a.norm_max || a.norm_partials)
         a.upd_state = nullptr;
+    if (hop_blocks) {
+        launch_dslash_hop(a, link_kind, diag, inv, nblocks, st);
+        return (a.norm_partials || a.upd_state) ? nblocks : 0;
+    }
     switch (a.prec) {
         case 0: launch_pr<0>(a, link_kind, diag, inv, nblocks, st); break;
         case 1: launch_pr<1>(a, link_kind, diag, inv, nblocks, st); break;

@@ -80,9 +80,18 @@ __host__ __device__ __forceinline__ cplx<T> cmulc(cplx<T> a, cplx<T> b) {
 }
 template <class T>
 __host__ __device__ __forceinline__ cplx<T> conj(cplx<T> a) { return {a.re, -a.im}; }
-// one fused multiply-add (a single rounding)
-__host__ __device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__host__ __device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
+// one fused multiply-add (a single rounding), and nothing merged into it: with
+// contraction allowed the compiler turns pairs of FP16-operand multiply-adds into
+// two-product instructions in some kernels and not in others, and a site's bits
+// would depend on the kernel
+__host__ __device__ __forceinline__ float fmadd(float a, float b, float c) {
+#pragma clang fp contract(off)
+    return __builtin_fmaf(a, b, c);
+}
+__host__ __device__ __forceinline__ double fmadd(double a, double b, double c) {
+#pragma clang fp contract(off)
+    return __builtin_fma(a, b, c);
+}
 // a += b * c, as two fused multiply-adds per real component: four
 // instructions per complex product instead of six (a multiply, a fused
 // multiply-add and an add per component), and one rounding fewer
@@ -100,6 +109,27 @@ __host__ __device__ __forceinline__ void cfmac(cplx<T>& a, cplx<T> b, cplx<T> c)
     a.re = fmadd(b.im, c.im, a.re);
     a.im = fmadd(b.re, c.im, a.im);
     a.im = fmadd(-b.im, c.re, a.im);
+}
+
+// a * b and y + s * x with their roundings written out, so that every kernel
+// that uses them computes the same bits (left to itself the compiler fuses a
+// product into either addend, differently from kernel to kernel)
+template <class T>
+__host__ __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) {
+    return {fmadd(-a.im, b.im, a.re * b.re), fmadd(a.im, b.re, a.re * b.im)};
+}
+template <class T>
+__host__ __device__ __forceinline__ cplx<T> cmulcj(cplx<T> a, cplx<T> b) {  // conj(a) * b
+    return {fmadd(a.im, b.im, a.re * b.re), fmadd(-a.im, b.re, a.re * b.im)};
+}
+template <class T>
+__host__ __device__ __forceinline__ cplx<T> axpy1(T s, cplx<T> x, cplx<T> y) {
+    return {fmadd(s, x.re, y.re), fmadd(s, x.im, y.im)};
+}
+// n + |a|^2, likewise
+template <class T>
+__host__ __device__ __forceinline__ T norm_acc(cplx<T> a, T n) {
+    return fmadd(a.im, a.im, fmadd(a.re, a.re, n));
 }
 
 // multiply by the phase i^PH (PH = 0: 1, 1: i, 2: -1, 3: -i)

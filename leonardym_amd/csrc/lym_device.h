@@ -462,6 +462,26 @@ __device__ __forceinline__ void load_link_rows(const void* base, int stride, int
     __builtin_memcpy(e, buf, P::BYTES);
 }
 
+// row 2 from rows 0 and 1: conj(row0 x row1), for real links row0 x row1
+template <class T>
+__device__ __forceinline__ void rebuild_row2(cplx<T> m[9]) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int i = (k + 1) % 3, j = (k + 2) % 3;
+        cplx<T> t = cmul(m[i], m[3 + j]);
+        cfma(t, -m[j], m[3 + i]);
+        m[6 + k] = conj(t);
+    }
+}
+template <class T>
+__device__ __forceinline__ void rebuild_row2(T m[9]) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int i = (k + 1) % 3, j = (k + 2) % 3;
+        m[6 + k] = fmadd(-m[j], m[3 + i], m[i] * m[3 + j]);
+    }
+}
+
 template <int PR, int LK>
 __device__ __forceinline__ void load_link(const void* base, int stride, int p, int mu, int idx,
                                           LinkMat<LK, typename Prec<PR>::T>& L) {
@@ -476,13 +496,9 @@ __device__ __forceinline__ void load_link(const void* base, int stride, int p, i
             else L.m[k] = to_c<PR>(e[k]);
         }
         if constexpr (REAL) {
-            L.m[6] = L.m[1] * L.m[5] - L.m[2] * L.m[4];
-            L.m[7] = L.m[2] * L.m[3] - L.m[0] * L.m[5];
-            L.m[8] = L.m[0] * L.m[4] - L.m[1] * L.m[3];
+            rebuild_row2(L.m);
         } else {
-            L.m[6] = conj(L.m[1] * L.m[5] - L.m[2] * L.m[4]);
-            L.m[7] = conj(L.m[2] * L.m[3] - L.m[0] * L.m[5]);
-            L.m[8] = conj(L.m[0] * L.m[4] - L.m[1] * L.m[3]);
+            rebuild_row2(L.m);
         }
     } else if constexpr (LK == 0 || LK == 1) {
         constexpr int NC = (LK == 0) ? 9 : 6;
@@ -493,9 +509,7 @@ __device__ __forceinline__ void load_link(const void* base, int stride, int p, i
             L.m[k] = to_c<PR>(fld<typename Prec<PR>::S, LYM_NT_LINKS != 0>(b + (size_t)k * stride, (unsigned)idx));
         }
         if constexpr (LK == 1) {
-            L.m[6] = conj(L.m[1] * L.m[5] - L.m[2] * L.m[4]);
-            L.m[7] = conj(L.m[2] * L.m[3] - L.m[0] * L.m[5]);
-            L.m[8] = conj(L.m[0] * L.m[4] - L.m[1] * L.m[3]);
+            rebuild_row2(L.m);
         }
     } else {
         constexpr int NC = (LK == 2) ? 9 : 6;
@@ -504,9 +518,7 @@ __device__ __forceinline__ void load_link(const void* base, int stride, int p, i
 #pragma unroll
         for (int k = 0; k < NC; ++k) L.m[k] = (T)fld<typename Prec<PR>::R, LYM_NT_LINKS != 0>(b + (size_t)k * stride, (unsigned)idx);
         if constexpr (LK == 3) {
-            L.m[6] = L.m[1] * L.m[5] - L.m[2] * L.m[4];
-            L.m[7] = L.m[2] * L.m[3] - L.m[0] * L.m[5];
-            L.m[8] = L.m[0] * L.m[4] - L.m[1] * L.m[3];
+            rebuild_row2(L.m);
         }
     }
 }
@@ -516,13 +528,12 @@ __device__ __forceinline__ void matvec(const LinkMat<LK, T>& L, const cplx<T> h[
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         if constexpr (LK <= 1) {
-            cplx<T> s = L.m[3 * i] * h[0];
+            cplx<T> s = cmul(L.m[3 * i], h[0]);
             cfma(s, L.m[3 * i + 1], h[1]);
             cfma(s, L.m[3 * i + 2], h[2]);
             o[i] = s;
         } else {
-            o[i] = mk(L.m[3 * i] * h[0].re + L.m[3 * i + 1] * h[1].re + L.m[3 * i + 2] * h[2].re,
-                      L.m[3 * i] * h[0].im + L.m[3 * i + 1] * h[1].im + L.m[3 * i + 2] * h[2].im);
+            o[i] = axpy1(L.m[3 * i + 2], h[2], axpy1(L.m[3 * i + 1], h[1], L.m[3 * i] * h[0]));
         }
     }
 }
@@ -532,13 +543,12 @@ __device__ __forceinline__ void matvec_dag(const LinkMat<LK, T>& L, const cplx<T
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         if constexpr (LK <= 1) {
-            cplx<T> s = cmulc(L.m[i], h[0]);
+            cplx<T> s = cmulcj(L.m[i], h[0]);
             cfmac(s, L.m[3 + i], h[1]);
             cfmac(s, L.m[6 + i], h[2]);
             o[i] = s;
         } else {
-            o[i] = mk(L.m[i] * h[0].re + L.m[3 + i] * h[1].re + L.m[6 + i] * h[2].re,
-                      L.m[i] * h[0].im + L.m[3 + i] * h[1].im + L.m[6 + i] * h[2].im);
+            o[i] = axpy1(L.m[6 + i], h[2], axpy1(L.m[3 + i], h[1], L.m[i] * h[0]));
         }
     }
 }
@@ -616,14 +626,12 @@ struct PackedBlock {
     static constexpr bool H8 = BYTES - 16 * N16 >= 8;
 };
 
-// o = sc * A v for the block at plane_off = plane * stride of a packed field
-// whose group arrays hold ngroup vectors each
+// the 18 entries (unscaled) of the block at plane_off = plane * stride of a
+// packed field whose group arrays hold ngroup vectors each
 template <int PR>
-__device__ __forceinline__ void herm6_packed(const void* base, size_t ngroup, size_t plane_off, int idx,
-                                             typename Prec<PR>::T sc, const cplx<typename Prec<PR>::T> v[6],
-                                             cplx<typename Prec<PR>::T> o[6]) {
+__device__ __forceinline__ void load_block_packed(const void* base, size_t ngroup, size_t plane_off, int idx,
+                                                  cplx<typename Prec<PR>::T> a[18]) {
     typedef PackedBlock<PR> P;
-    typedef typename Prec<PR>::T T;
     const char* gb = reinterpret_cast<const char*>(base);
     unsigned char buf[P::BYTES];
     int off = 0;
@@ -640,10 +648,18 @@ __device__ __forceinline__ void herm6_packed(const void* base, size_t ngroup, si
     }
     typename P::E e[18];
     __builtin_memcpy(e, buf, P::BYTES);
-    cplx<T> a[18];
 #pragma unroll
     for (int k = 0; k < 18; ++k) a[k] = to_c<PR>(e[k]);
-    herm6_mul<T>(a, v, o);
+}
+
+// o = sc * A v for that block
+template <int PR>
+__device__ __forceinline__ void herm6_packed(const void* base, size_t ngroup, size_t plane_off, int idx,
+                                             typename Prec<PR>::T sc, const cplx<typename Prec<PR>::T> v[6],
+                                             cplx<typename Prec<PR>::T> o[6]) {
+    cplx<typename Prec<PR>::T> a[18];
+    load_block_packed<PR>(base, ngroup, plane_off, idx, a);
+    herm6_mul<typename Prec<PR>::T>(a, v, o);
     if constexpr (PR == 2) {
         // the block's scale on the 6 outputs instead of its 18 entries
 #pragma unroll

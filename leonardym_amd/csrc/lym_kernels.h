@@ -44,6 +44,7 @@ struct DslashParams {
     int allow_split;       // the caller allows the two-threads-per-site form (low precision)
     int mfma;              // the caller allows the matrix-core form (FP16 SU(3) multi-RHS, nr 2, 4 or 8)
     int split;             // set by the launcher: threads per half of that form, or 0
+    double inv_ext[3];     // set by the launcher (the one-wave-per-direction form): 1 / Ly, 1 / Lz, 1 / Lth
     double* norm_partials; // optional (FP32/FP16 only): workgroup b writes the sum of |out|^2 over
     int norm_max;          //   its sites to norm_partials[b], when the launch has at most norm_max workgroups
     // Per-lane operators (multi-RHS launches of the serving engine): lane r uses
@@ -98,6 +99,9 @@ struct UpdArgs {
 // link_kind: 0 complex 18, 1 complex 12, 2 real 9, 3 real 6; diag: 0 none, 1 identity, 2 clover.
 // Returns the number of output-norm partials written (0: none were asked for or they did not fit).
 int launch_dslash(DslashParams a, int link_kind, int diag, bool inv, hipStream_t st);
+// the one-wave-per-direction form (dslash_hop.hip) of a launch whose spb, blocks per
+// parity and inv_ext launch_dslash has set
+void launch_dslash_hop(const DslashParams& a, int link_kind, int diag, bool inv, int nblocks, hipStream_t st);
 
 // ---------------------------------------------------------------- layout (layout.hip)
 void launch_spinor_to_eo(const Geom& g, const zd* aos, zd* eo, hipStream_t st);
