@@ -240,8 +240,28 @@ lym::DslashParams base_params(const lym_op* op) {
 inline zd* par(zd* f, const lym_ctx* c, int p) { return f + (size_t)p * 12 * c->g.stride; }
 inline const zd* par(const zd* f, const lym_ctx* c, int p) { return f + (size_t)p * 12 * c->g.stride; }
 
-// full-lattice single power: out = Op in (+ alpha v2); Wilson or clover
-void apply_full1(lym_op* op, zd* out, const zd* in, const zd* v2, zd alpha, int gamma5, const int* skip) {
+// a fused step of the FP64 solvers on a launch: vectors of nparity parities (1:
+// odd halves, on the odd-parity launch)
+void set_fuse64(lym::DslashParams& a, const lym::Fuse64& f, const lym_ctx* c, int nparity) {
+    a.fmode = f.mode;
+    a.upd_state = f.state;
+    a.upd_dot = f.dot;
+    a.upd_ndot = f.ndot;
+    a.upd_rpart = f.part;
+    a.part_stride = f.part_stride;
+    for (int q = 0; q < 2; ++q) {
+        const size_t o = nparity == 2 ? (size_t)q * 12 * c->g.stride : 0;
+        a.dotw[q] = f.w ? f.w + o : nullptr;
+        a.upd_p[q] = f.p ? f.p + o : nullptr;
+        a.upd_xs[q] = f.x ? f.x + o : nullptr;
+        a.upd_rs[q] = f.r ? f.r + o : nullptr;
+    }
+}
+
+// full-lattice single power: out = Op in (+ alpha v2); Wilson or clover.  Returns
+// the number of partials of the fused step (0: none asked for or not taken)
+int apply_full1(lym_op* op, zd* out, const zd* in, const zd* v2, zd alpha, int gamma5, const int* skip,
+                const lym::Fuse64* fuse = nullptr) {
     lym_ctx* c = op->ctx;
     lym::DslashParams a = base_params(op);
     for (int p = 0; p < 2; ++p) {
@@ -254,11 +274,13 @@ void apply_full1(lym_op* op, zd* out, const zd* in, const zd* v2, zd alpha, int 
     a.gamma5 = gamma5;
     a.parity = c->g.tsh ? -1 : 0;  // both parities, or the one class of a lattice with an odd extent
     a.skip = skip;
-    lym::launch_dslash(a, link_kind(op->gauge), op_has_clover(op) ? 2 : 1, false, c->stream);
+    if (fuse) set_fuse64(a, *fuse, c, 2);
+    return lym::launch_dslash(a, link_kind(op->gauge), op_has_clover(op) ? 2 : 1, false, c->stream);
 }
 
 // Schur complement on odd half fields: out_o = gamma5^g (A_o in_o - D_oe Ainv_e D_eo in_o)
-void apply_schur1(lym_op* op, zd* out_o, const zd* in_o, int gamma5, const int* skip) {
+int apply_schur1(lym_op* op, zd* out_o, const zd* in_o, int gamma5, const int* skip,
+                 const lym::Fuse64* fuse = nullptr) {
     lym_ctx* c = op->ctx;
     int lk = link_kind(op->gauge);
     lym::DslashParams a = base_params(op);
@@ -275,7 +297,8 @@ void apply_schur1(lym_op* op, zd* out_o, const zd* in_o, int gamma5, const int* 
     b.out[1] = out_o;
     b.hop_sign = -1.0;
     b.gamma5 = gamma5;
-    lym::launch_dslash(b, lk, op->csw != 0.0 ? 2 : 1, false, c->stream);
+    if (fuse) set_fuse64(b, *fuse, c, 1);
+    return lym::launch_dslash(b, lk, op->csw != 0.0 ? 2 : 1, false, c->stream);
 }
 
 int ensure_op_scratch(lym_op* op) {
@@ -329,14 +352,15 @@ int op_ready(lym_op* op, bool force_blocks) {
     if (rc) return rc;
     return ensure_op_scratch(op);
 }
-void apply_schur(lym_op* op, zd* out_o, const zd* in_o, int gamma5, const int* skip) {
-    apply_schur1(op, out_o, in_o, gamma5, skip);
+int apply_schur(lym_op* op, zd* out_o, const zd* in_o, int gamma5, const int* skip, const lym::Fuse64* fuse) {
+    return apply_schur1(op, out_o, in_o, gamma5, skip, fuse);
 }
-void apply_full(lym_op* op, zd* out, const zd* in, int gamma5, const int* skip) {
-    apply_full1(op, out, in, nullptr, lym::mk(0.0, 0.0), gamma5, skip);
+int apply_full(lym_op* op, zd* out, const zd* in, int gamma5, const int* skip, const lym::Fuse64* fuse) {
+    return apply_full1(op, out, in, nullptr, lym::mk(0.0, 0.0), gamma5, skip, fuse);
 }
-void apply_full_add(lym_op* op, zd* out, const zd* in, const zd* v2, zd alpha, int gamma5, const int* skip) {
-    apply_full1(op, out, in, v2, alpha, gamma5, skip);
+int apply_full_add(lym_op* op, zd* out, const zd* in, const zd* v2, zd alpha, int gamma5, const int* skip,
+                   const lym::Fuse64* fuse) {
+    return apply_full1(op, out, in, v2, alpha, gamma5, skip, fuse);
 }
 int link_kind_of(const lym_gauge* g) { return link_kind(g); }
 

@@ -29,9 +29,9 @@ __device__ __forceinline__ void wave_sum(double v[NV]) {
         for (int k = 0; k < NV; ++k) v[k] += __shfl_xor(v[k], off, 64);
 }
 
-// block of RB_THREADS threads -> partials[k * RED_BLOCKS + blockIdx.x]
+// block of RB_THREADS threads -> partials[k * stride + blockIdx.x]
 template <int NV>
-__device__ __forceinline__ void block_store(double v[NV], double* partials) {
+__device__ __forceinline__ void block_store(double v[NV], double* partials, int stride = RED_BLOCKS) {
     __shared__ double sh[NV][RB_THREADS / 64];
     wave_sum<NV>(v);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -45,7 +45,7 @@ __device__ __forceinline__ void block_store(double v[NV], double* partials) {
             double s = 0;
 #pragma unroll
             for (int j = 0; j < RB_THREADS / 64; ++j) s += sh[k][j];
-            partials[k * RED_BLOCKS + blockIdx.x] = s;
+            partials[(size_t)k * stride + blockIdx.x] = s;
         }
     }
 }
@@ -73,29 +73,25 @@ __device__ __forceinline__ void final_sum(const double* partials, double out[NV]
         }
 }
 
-// The total of final_sum, folded by every workgroup of RB_THREADS threads that
-// needs it (the same fixed order in each, so all get the same value): the
+// The totals of NV sums of n <= FOLD_MAX partials each (sum k of workgroup b at
+// partials[k * stride + b]), folded by every workgroup of RB_THREADS threads that
+// needs them (the same fixed order in each, so all get the same values): the
 // partials are loaded first (fold_load), the caller may then issue its own
 // loads, and fold_block folds across the workgroup (result in every thread).
-constexpr int FOLD_PER_THREAD = RED_BLOCKS / RB_THREADS;
-static_assert(RED_BLOCKS % RB_THREADS == 0, "partials per thread");
 template <int NV>
-__device__ __forceinline__ void fold_load(const double* partials, double pl[NV][FOLD_PER_THREAD]) {
+__device__ __forceinline__ void fold_load(const double* partials, int stride, int n, double pl[NV]) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k)
+    for (int k = 0; k < NV; ++k) pl[k] = 0;
+    for (int i = (int)threadIdx.x; i < n; i += RB_THREADS)
 #pragma unroll
-        for (int i = 0; i < FOLD_PER_THREAD; ++i) pl[k][i] = partials[k * RED_BLOCKS + threadIdx.x + i * RB_THREADS];
+        for (int k = 0; k < NV; ++k) pl[k] += partials[(size_t)k * stride + i];
 }
 template <int NV>
-__device__ __forceinline__ void fold_block(const double pl[NV][FOLD_PER_THREAD], double out[NV]) {
+__device__ __forceinline__ void fold_block(const double pl[NV], double out[NV]) {
     __shared__ double sh[NV][RB_THREADS / 64];
     double v[NV];
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        v[k] = 0;
-#pragma unroll
-        for (int i = 0; i < FOLD_PER_THREAD; ++i) v[k] += pl[k][i];
-    }
+    for (int k = 0; k < NV; ++k) v[k] = pl[k];
     wave_sum<NV>(v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -109,6 +105,40 @@ __device__ __forceinline__ void fold_block(const double pl[NV][FOLD_PER_THREAD],
         out[k] = t;
     }
     __syncthreads();
+}
+
+// more than FOLD_MAX partials: one workgroup folds each sum into one
+template <int NV>
+__global__ __launch_bounds__(1024) void k_fold(const double* partials, int stride, int n, double* out,
+                                               const int* skip) {
+    if (skip && *skip) return;
+    __shared__ double sh[NV][16];
+    double v[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] = 0;
+    for (int i = (int)threadIdx.x; i < n; i += 1024)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] += partials[(size_t)k * stride + i];
+    wave_sum<NV>(v);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) sh[k][threadIdx.x >> 6] = v[k];
+    __syncthreads();
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            double t = 0;
+            for (int j = 0; j < 16; ++j) t += sh[k][j];
+            out[(size_t)k * stride] = t;
+        }
+}
+
+void launch_fold(int nv, const double*& part, int stride, int& npart, double* out, const int* skip, hipStream_t st) {
+    if (npart <= FOLD_MAX) return;
+    if (nv == 1) hipLaunchKernelGGL(k_fold<1>, dim3(1), dim3(1024), 0, st, part, stride, npart, out, skip);
+    else hipLaunchKernelGGL(k_fold<3>, dim3(1), dim3(1024), 0, st, part, stride, npart, out, skip);
+    part = out;
+    npart = 1;
 }
 
 #define GRID_LOOP(i, n) for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += (long)gridDim.x * blockDim.x)
@@ -278,8 +308,8 @@ __global__ __launch_bounds__(RB_THREADS) void k_cg_update(CGState* s, zd* __rest
                                                           const zd* __restrict__ p, const zd* __restrict__ Ap, long n,
                                                           const double* dot_partials, double* partials) {
     if (s->done) return;
-    double pl[2][FOLD_PER_THREAD];
-    fold_load<2>(dot_partials, pl);
+    double pl[2];
+    fold_load<2>(dot_partials, RED_BLOCKS, RED_BLOCKS, pl);
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long istep = (long)gridDim.x * blockDim.x;
     zd xv, rv, pv, av;
@@ -329,13 +359,13 @@ void launch_cg_update(CGState* s, zd* x, zd* r, const zd* p, const zd* Ap, long 
 // start (read once per workgroup: after a stop decided here p may be left
 // partly updated, which nothing reads).
 __global__ __launch_bounds__(RB_THREADS) void k_cg_p(CGState* s, zd* __restrict__ p, const zd* __restrict__ r, long n,
-                                                     const double* rpart) {
+                                                     const double* rpart, int npart) {
     __shared__ int stop;
     if (threadIdx.x == 0) stop = s->done;
     __syncthreads();
     if (stop) return;
-    double pl[1][FOLD_PER_THREAD];
-    fold_load<1>(rpart, pl);
+    double pl[1];
+    fold_load<1>(rpart, 0, npart, pl);
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long istep = (long)gridDim.x * blockDim.x;
     zd pv, rv;
@@ -368,8 +398,8 @@ __global__ __launch_bounds__(RB_THREADS) void k_cg_p(CGState* s, zd* __restrict_
     }
 }
 
-void launch_cg_p(CGState* s, zd* p, const zd* r, long n, double* partials, hipStream_t st) {
-    hipLaunchKernelGGL(k_cg_p, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, p, r, n, partials + 2 * RED_BLOCKS);
+void launch_cg_p(CGState* s, zd* p, const zd* r, long n, const double* part, int npart, hipStream_t st) {
+    hipLaunchKernelGGL(k_cg_p, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, p, r, n, part, npart);
 }
 
 // ---------------------------------------------------------------- BiCGStab
@@ -390,6 +420,7 @@ __global__ void k_bicg_init(BiCGState* s, double precision, int max_steps) {
     s->converged = 0;
     s->breakdown = 0;
     s->copy_b = 0;
+    s->phase = BICG_FIRST;
     s->done = max_steps <= 0 ? 1 : 0;
 }
 
@@ -397,65 +428,86 @@ void launch_bicg_init(BiCGState* s, double precision, int max_steps, hipStream_t
     hipLaunchKernelGGL(k_bicg_init, dim3(1), dim3(1), 0, st, s, precision, max_steps);
 }
 
-__global__ void k_bicg_setup(zd* __restrict__ r, zd* __restrict__ rh, zd* __restrict__ p, zd* __restrict__ nu,
-                             const zd* __restrict__ b, const zd* __restrict__ Ax, long n) {
+// v += <rh, r> and |r|^2 of one element
+__device__ __forceinline__ void bicg_terms(zd rh, zd r, double v[3]) {
+    v[0] += rh.re * r.re + rh.im * r.im;
+    v[1] += rh.re * r.im - rh.im * r.re;
+    v[2] += r.re * r.re + r.im * r.im;
+}
+
+__global__ __launch_bounds__(RB_THREADS) void k_bicg_setup(zd* __restrict__ r, zd* __restrict__ rh,
+                                                           zd* __restrict__ p, zd* __restrict__ nu,
+                                                           const zd* __restrict__ b, const zd* __restrict__ Ax,
+                                                           long n, double* partials, int stride) {
+    double v[3] = {0, 0, 0};
     GRID_LOOP(i, n) {
-        zd bb = b[i], ax = Ax[i];
-        r[i] = bb - ax;
-        rh[i] = bb + ax;
+        const zd bb = b[i], ax = Ax[i], ri = bb - ax, hi = bb + ax;
+        r[i] = ri;
+        rh[i] = hi;
         p[i] = mk(0.0, 0.0);
         nu[i] = mk(0.0, 0.0);
+        bicg_terms(hi, ri, v);
     }
+    block_store<3>(v, partials, stride);
 }
 
-void launch_bicg_setup(zd* r, zd* rh, zd* p, zd* nu, const zd* b, const zd* Ax, long n, hipStream_t st) {
-    hipLaunchKernelGGL(k_bicg_setup, dim3(ew_blocks(n)), dim3(256), 0, st, r, rh, p, nu, b, Ax, n);
+void launch_bicg_setup(zd* r, zd* rh, zd* p, zd* nu, const zd* b, const zd* Ax, long n, double* partials, int stride,
+                       hipStream_t st) {
+    hipLaunchKernelGGL(k_bicg_setup, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, r, rh, p, nu, b, Ax, n, partials,
+                       stride);
 }
 
-template <class S>
-__global__ __launch_bounds__(RB_THREADS) void k_state_dot(const S* s, const zd* __restrict__ a,
-                                                          const zd* __restrict__ b, long n, double* partials) {
-    if (s->done) return;
-    double v[2] = {0, 0};
-    GRID_LOOP(i, n) {
-        zd x = a[i], y = b[i];
-        v[0] += x.re * y.re + x.im * y.im;
-        v[1] += x.re * y.im - x.im * y.re;
-    }
-    block_store<2>(v, partials);
-}
-
-void launch_bicg_rho(BiCGState* s, const zd* rh, const zd* r, long n, double* partials, hipStream_t st) {
-    hipLaunchKernelGGL(k_state_dot<BiCGState>, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, rh, r, n, partials);
-}
-
-// Each of the p, s and x/r updates below folds the partial sums of the dot
-// product before it in every workgroup (a fixed order, so all get the same
-// value); workgroup 0 writes the state, and no workgroup reads what it
-// writes except `done` at the start (read once per workgroup: after a stop
-// decided there a vector may be left partly updated, which nothing reads).
+// Each of the p, s and x/r updates below folds the partial sums of the step
+// before it in every workgroup (a fixed order, so all get the same value);
+// workgroup 0 writes the state, and no workgroup reads what it writes except
+// `done` at the start (read once per workgroup: after a stop decided there a
+// vector may be left partly updated, which nothing reads).
 #define BICG_STOP_CHECK()                        \
     __shared__ int stop_;                        \
     if (threadIdx.x == 0) stop_ = s->done;      \
     __syncthreads();                             \
     if (stop_) return
 
-// rho_next = <rh, r>; breakdown if zero; beta = (rho_next / rho)(alpha / omega);
-// p = r + beta (p - omega nu)
+// |r|^2 < precision after the last update: converged at its step; else that step
+// is over, at most max_steps of them (BiConjugateGradient.cpp:480-501).  Returns
+// whether the solve stops; wr: this thread writes the state.
+__device__ __forceinline__ bool bicg_stop(BiCGState* s, double norm, int step, bool wr) {
+    const bool conv = norm < s->precision, last = step + 1 >= s->max_steps;
+    if (wr) {
+        s->norm = norm;
+        if (conv) {
+            s->converged = 1;
+            s->done = 1;
+        } else if (last) {
+            s->step = step + 1;
+            s->done = 1;
+        }
+    }
+    return conv || last;
+}
+
+// The last update's stopping rule, then rho_next = <rh, r>; breakdown if zero;
+// beta = (rho_next / rho)(alpha / omega); p = r + beta (p - omega nu)
 __global__ __launch_bounds__(RB_THREADS) void k_bicg_p(BiCGState* s, zd* __restrict__ p, const zd* __restrict__ r,
-                                                       const zd* __restrict__ nu, long n, const double* partials) {
+                                                       const zd* __restrict__ nu, long n, const double* partials,
+                                                       int stride, int npart) {
     BICG_STOP_CHECK();
-    double pl[2][FOLD_PER_THREAD];
-    fold_load<2>(partials, pl);
-    double out[2];
-    fold_block<2>(pl, out);
+    const bool wr = blockIdx.x == 0 && threadIdx.x == 0;
+    const int phase = s->phase, step = s->step;
+    double pl[3];
+    fold_load<3>(partials, stride, npart, pl);
+    double out[3];
+    fold_block<3>(pl, out);
+    if (phase == BICG_FOLD && bicg_stop(s, out[2], step, wr)) return;
     const zd rn = mk(out[0], out[1]);
     const bool brk = rn.re * rn.re + rn.im * rn.im == 0.0;
-    const zd beta = zdiv(rn, mk(s->rho_re, s->rho_im)) * zdiv(mk(s->alpha_re, s->alpha_im), mk(s->omega_re, s->omega_im));
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const zd om = mk(s->omega_re, s->omega_im);
+    const zd beta = zdiv(rn, mk(s->rho_re, s->rho_im)) * zdiv(mk(s->alpha_re, s->alpha_im), om);
+    if (wr) {
         s->rhon_re = rn.re;
         s->rhon_im = rn.im;
         if (brk) {
+            if (phase == BICG_FOLD) s->step = step + 1;
             s->done = 1;
             s->breakdown = 1;
             s->converged = 0;
@@ -465,66 +517,55 @@ __global__ __launch_bounds__(RB_THREADS) void k_bicg_p(BiCGState* s, zd* __restr
         }
     }
     if (brk) return;
-    const zd om = mk(s->omega_re, s->omega_im);
     GRID_LOOP(i, n) { p[i] = r[i] + beta * (p[i] - om * nu[i]); }
 }
 
-void launch_bicg_p(BiCGState* s, zd* p, const zd* r, const zd* nu, long n, const double* partials, hipStream_t st) {
-    hipLaunchKernelGGL(k_bicg_p, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, p, r, nu, n, partials);
+void launch_bicg_p(BiCGState* s, zd* p, const zd* r, const zd* nu, long n, const double* partials, int stride,
+                   hipStream_t st) {
+    hipLaunchKernelGGL(k_bicg_p, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, p, r, nu, n, partials, stride,
+                       RED_BLOCKS);
 }
 
-void launch_bicg_alpha(BiCGState* s, const zd* rh, const zd* nu, long n, double* partials, hipStream_t st) {
-    hipLaunchKernelGGL(k_state_dot<BiCGState>, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, rh, nu, n, partials);
-}
-
-// alpha = rho_next / <rh, nu>; s = r - alpha nu
+// alpha = rho_next / <rh, nu>; s = r - alpha nu.  Workgroup 0 also moves rho_next
+// to rho and counts the step the p update has closed.
 __global__ __launch_bounds__(RB_THREADS) void k_bicg_s(BiCGState* s, zd* __restrict__ sv, const zd* __restrict__ r,
-                                                       const zd* __restrict__ nu, long n, const double* partials) {
+                                                       const zd* __restrict__ nu, long n, const double* part,
+                                                       int stride, int npart) {
     BICG_STOP_CHECK();
-    double pl[2][FOLD_PER_THREAD];
-    fold_load<2>(partials, pl);
+    double pl[2];
+    fold_load<2>(part, stride, npart, pl);
     double out[2];
     fold_block<2>(pl, out);
-    const zd al = zdiv(mk(s->rhon_re, s->rhon_im), mk(out[0], out[1]));
+    const zd rhon = mk(s->rhon_re, s->rhon_im), al = zdiv(rhon, mk(out[0], out[1]));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         s->alpha_re = al.re;
         s->alpha_im = al.im;
+        s->rho_re = rhon.re;
+        s->rho_im = rhon.im;
+        if (s->phase == BICG_FOLD) s->step += 1;
+        s->phase = BICG_FOLD;
     }
     GRID_LOOP(i, n) { sv[i] = r[i] - al * nu[i]; }
 }
 
-void launch_bicg_s(BiCGState* s, zd* sv, const zd* r, const zd* nu, long n, const double* partials, hipStream_t st) {
-    hipLaunchKernelGGL(k_bicg_s, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, sv, r, nu, n, partials);
+void launch_bicg_s(BiCGState* s, zd* sv, const zd* r, const zd* nu, long n, const double* part, int stride, int npart,
+                   hipStream_t st) {
+    hipLaunchKernelGGL(k_bicg_s, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, sv, r, nu, n, part, stride, npart);
 }
 
-__global__ __launch_bounds__(RB_THREADS) void k_bicg_ts(const BiCGState* s, const zd* __restrict__ t,
-                                                        const zd* __restrict__ sv, long n, double* partials) {
-    if (s->done) return;
-    double v[4] = {0, 0, 0, 0};
-    GRID_LOOP(i, n) {
-        zd x = t[i], y = sv[i];
-        v[0] += x.re * y.re + x.im * y.im;
-        v[1] += x.re * y.im - x.im * y.re;
-        v[2] += x.re * x.re + x.im * x.im;
-    }
-    block_store<4>(v, partials);
-}
-
-void launch_bicg_omega(BiCGState* s, const zd* t, const zd* sv, long n, double* partials, hipStream_t st) {
-    hipLaunchKernelGGL(k_bicg_ts, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, t, sv, n, partials);
-}
-
-// omega = <t,s>/<t,t>; <t,t> == 0 -> solution = source (BiConjugateGradient.cpp:449-458);
-// x += alpha p + omega s, r = s - omega t, partial |r|^2 (into rpart)
+// omega = <t,s>/<t,t> from <s,t> and |t|^2; <t,t> == 0 -> solution = source
+// (BiConjugateGradient.cpp:449-458); x += alpha p + omega s, r = s - omega t,
+// partial <rh, r> and |r|^2
 __global__ __launch_bounds__(RB_THREADS) void k_bicg_update(BiCGState* s, zd* __restrict__ x, zd* __restrict__ r,
-                                                            const zd* __restrict__ p, const zd* __restrict__ sv,
-                                                            const zd* __restrict__ t, const zd* __restrict__ b,
-                                                            long n, const double* partials, double* rpart) {
+                                                            const zd* __restrict__ rh, const zd* __restrict__ p,
+                                                            const zd* __restrict__ sv, const zd* __restrict__ t,
+                                                            const zd* __restrict__ b, long n, const double* part,
+                                                            int stride, int npart, double* partials) {
     BICG_STOP_CHECK();
-    double pl[4][FOLD_PER_THREAD];
-    fold_load<4>(partials, pl);
-    double out[4];
-    fold_block<4>(pl, out);
+    double pl[3];
+    fold_load<3>(part, stride, npart, pl);
+    double out[3];
+    fold_block<3>(pl, out);
     if (out[2] == 0.0) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             s->copy_b = 1;
@@ -534,48 +575,43 @@ __global__ __launch_bounds__(RB_THREADS) void k_bicg_update(BiCGState* s, zd* __
         GRID_LOOP(i, n) { x[i] = b[i]; }
         return;
     }
-    const zd om = mk(out[0] / out[2], out[1] / out[2]);
+    const zd om = mk(out[0] / out[2], -out[1] / out[2]);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         s->omega_re = om.re;
         s->omega_im = om.im;
     }
     const zd al = mk(s->alpha_re, s->alpha_im);
-    double v[1] = {0};
+    double v[3] = {0, 0, 0};
     GRID_LOOP(i, n) {
-        zd sv_i = sv[i];
+        const zd sv_i = sv[i];
         x[i] = x[i] + al * p[i] + om * sv_i;
-        zd rn = sv_i - om * t[i];
+        const zd rn = sv_i - om * t[i];
         r[i] = rn;
-        v[0] += rn.re * rn.re + rn.im * rn.im;
+        bicg_terms(rh[i], rn, v);
     }
-    block_store<1>(v, rpart);
+    block_store<3>(v, partials, stride);
 }
 
-__global__ __launch_bounds__(RED_BLOCKS) void k_bicg_update_final(BiCGState* s, const double* partials) {
-    if (s->done) return;
-    double out[1];
-    final_sum<1>(partials, out);
-    if (threadIdx.x == 0) {
-        s->norm = out[0];
-        if (out[0] < s->precision) {
-            s->done = 1;
-            s->converged = 1;
-            return;
-        }
-        s->rho_re = s->rhon_re;
-        s->rho_im = s->rhon_im;
+void launch_bicg_update(BiCGState* s, zd* x, zd* r, const zd* rh, const zd* p, const zd* sv, const zd* t, const zd* b,
+                        long n, const double* part, int stride, int npart, double* partials, hipStream_t st) {
+    hipLaunchKernelGGL(k_bicg_update, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, x, r, rh, p, sv, t, b, n, part,
+                       stride, npart, partials);
+}
+
+__global__ __launch_bounds__(RB_THREADS) void k_bicg_check(BiCGState* s, const double* partials, int stride,
+                                                           int npart) {
+    if (s->done || s->phase != BICG_FOLD) return;
+    double pl[3], out[3];
+    fold_load<3>(partials, stride, npart, pl);
+    fold_block<3>(pl, out);
+    if (threadIdx.x == 0 && !bicg_stop(s, out[2], s->step, true)) {
         s->step += 1;
-        if (s->step >= s->max_steps) s->done = 1;
+        s->phase = BICG_CHECKED;
     }
 }
 
-void launch_bicg_update(BiCGState* s, zd* x, zd* r, const zd* p, const zd* sv, const zd* t, const zd* b, long n,
-                        double* partials, hipStream_t st) {
-    // <t,s>, <t,t> partials (launch_bicg_omega) in slots 0..3, |r|^2 in slot 4
-    double* rpart = partials + 4 * RED_BLOCKS;
-    hipLaunchKernelGGL(k_bicg_update, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, x, r, p, sv, t, b, n, partials,
-                       rpart);
-    hipLaunchKernelGGL(k_bicg_update_final, dim3(1), dim3(RED_BLOCKS), 0, st, s, rpart);
+void launch_bicg_check(BiCGState* s, const double* partials, int stride, hipStream_t st) {
+    hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(RB_THREADS), 0, st, s, partials, stride, RED_BLOCKS);
 }
 
 }  // namespace lym

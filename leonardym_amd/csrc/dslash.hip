@@ -166,9 +166,10 @@ __device__ __forceinline__ void hop_pair(const DslashParams& a, int p, int site,
     if constexpr (pin_end) pin(acc);
 }
 
-template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD = false, int BM = 0>
+template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD = false, int BM = 0, int FM = 0>
 __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, int site, int r,
-                                                  const cplx<typename Prec<PR>::T> acc[12], float ual = 0.f);
+                                                  const cplx<typename Prec<PR>::T> acc[12], float ual = 0.f,
+                                                  double al = 0.0, double* sums = nullptr);
 
 // NORM (low precision only): returns |v|^2 of the site's output as computed,
 // before rounding to the storage precision; else 0.  A template parameter, so
@@ -176,9 +177,12 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
 // own kappa and clover blocks (a.lane_ops); also a template parameter.  UPD:
 // the fused mixed-CG update with step ual (a.upd_*): returns the site's
 // |r_s|^2 after it, and stores no output.
-template <int PR, int LK, int DIAG, bool INV, bool NORM = false, bool LO = false, bool UPD = false, int BM = 0>
+// FM: a fused step of the FP64 solvers (F64_*), with step al, its terms added to sums.
+template <int PR, int LK, int DIAG, bool INV, bool NORM = false, bool LO = false, bool UPD = false, int BM = 0,
+          int FM = 0>
 __device__ __forceinline__ double dslash_site(const DslashParams& a, int p, int site, int r, float ual = 0.f,
-                                              const cplx<double>* lds = nullptr, int lbase = 0) {
+                                              const cplx<double>* lds = nullptr, int lbase = 0, double al = 0.0,
+                                              double* sums = nullptr) {
     typedef typename Prec<PR>::T T;
     int c[4];
     eo_coords(a.g, p, site, c);
@@ -196,15 +200,16 @@ __device__ __forceinline__ double dslash_site(const DslashParams& a, int p, int 
         hop_pair<2, PR, LK>(a, p, site, r, c, acc, lds, lbase);
         hop_pair<3, PR, LK>(a, p, site, r, c, acc, lds, lbase);
     }
-    return dslash_epilogue<PR, DIAG, INV, NORM, LO, UPD, BM>(a, p, site, r, acc, ual);
+    return dslash_epilogue<PR, DIAG, INV, NORM, LO, UPD, BM, FM>(a, p, site, r, acc, ual, al, sums);
 }
 
 // The site's output from its hopping sum acc: v = diag(psi_x) + hop_sign
 // (-kappa acc), then R^-1, gamma5, the axpy and the store (the value
 // returned is as for dslash_site)
-template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD, int BM>
+template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD, int BM, int FM>
 __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, int site, int r,
-                                                  const cplx<typename Prec<PR>::T> acc[12], float ual) {
+                                                  const cplx<typename Prec<PR>::T> acc[12], float ual, double al64,
+                                                  double* sums) {
     typedef typename Prec<PR>::T T;
     typedef typename Prec<PR>::S S;
     const int ST = a.g.stride;
@@ -321,6 +326,12 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
         }
         return n2;
     }
+    if constexpr (FM != F64_STORE) {
+        static_assert(PR == 0 && !NORM && !LO && !UPD && BM == 0, "the FP64 solvers' fused steps: one RHS");
+#pragma unroll
+        for (int k = 0; k < 12; ++k) f64_step<FM>(a, p, k, (unsigned)site, al64, v[k], sums);
+        if constexpr (FM == F64_CG) return 0;
+    }
     store_spinor<PR>(SpinorOut<PR>{reinterpret_cast<S*>(a.out[p]), a.out_sc[p]}, ST, a.nr, site, r, v);
     if constexpr (BM == 1) {  // lane r's |v|^2 at this site: the 24 squares in FP32
         float n2[2] = {0.f, 0.f};
@@ -337,28 +348,37 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
     return 0;
 }
 
-// Sum of v over the workgroup (blockDim.x a multiple of 64, at most 1024), in
-// one fixed order; the total is written by thread 0 to out[blockIdx.x].  Every
-// thread of the workgroup must call it.
-__device__ __forceinline__ void block_sum_store(double v, double* out) {
-    __shared__ double sh[16];
+// Sums of N values over the workgroup (blockDim.x a multiple of 64, at most
+// 1024), in one fixed order; thread 0 writes total k to out[k * stride + blockIdx.x].
+// Every thread of the workgroup must call it.
+template <int N>
+__device__ __forceinline__ void block_sums_store(const double v[N], double* out, size_t stride) {
+    __shared__ double sh[N][16];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    for (int k = 0; k < N; ++k) {
+        double t = v[k];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+        if ((threadIdx.x & 63) == 0) sh[k][threadIdx.x >> 6] = t;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double t = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sh[w];
-        out[blockIdx.x] = t;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            double t = 0;
+            for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sh[k][w];
+            out[k * stride + blockIdx.x] = t;
+        }
     }
 }
+__device__ __forceinline__ void block_sum_store(double v, double* out) { block_sums_store<1>(&v, out, 0); }
 
-
-// The fused update's step: alpha = rr_s / (sum of the n <p, Ap> partials),
-// folded by every workgroup in one fixed order (so all get the same alpha);
-// workgroup 0 stores alpha and rr_prev = rr_s in the state.  Every thread of
-// the workgroup must call it.
-__device__ __forceinline__ float upd_alpha(const DslashParams& a) {
+// The fused update's step: alpha = rr / (sum of the n <p, Ap> partials), folded
+// by every workgroup in one fixed order (so all get the same alpha); workgroup 0
+// stores alpha and rr_prev = rr in the state (ST: MCGState, or CGState for the
+// FP64 CG).  Every thread of the workgroup must call it.
+template <class ST>
+__device__ __forceinline__ double upd_alpha(const DslashParams& a) {
     __shared__ double sh[16];
     double v = 0;
     for (int k = (int)threadIdx.x; k < a.upd_ndot; k += (int)blockDim.x) v += a.upd_dot[k];
@@ -368,15 +388,12 @@ __device__ __forceinline__ float upd_alpha(const DslashParams& a) {
     __syncthreads();
     double t = 0;
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sh[w];
-    MCGState* st = reinterpret_cast<MCGState*>(a.upd_state);
-    const double rr = st->rr_s;
+    ST* st = reinterpret_cast<ST*>(a.upd_state);
+    const double rr = state_rr(st);
     const double alpha = rr / t;
-    __syncthreads();  // every thread has read rr_s before workgroup 0 moves it to rr_prev
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->alpha = alpha;
-        st->rr_prev = rr;
-    }
-    return (float)alpha;
+    __syncthreads();  // every thread has read rr before workgroup 0 moves it to rr_prev
+    if (blockIdx.x == 0 && threadIdx.x == 0) set_alpha(st, alpha, rr);
+    return alpha;
 }
 
 // NORM: also the per-workgroup output norms (a.norm_partials); LO: per-lane
@@ -390,7 +407,7 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash(DslashPar
     const int ls = (int)threadIdx.x / a.nr, r = (int)threadIdx.x - ls * a.nr;
     if constexpr (UPD) {
         // one RHS, no lane flags: every thread holds a site slot and reaches the sums
-        const float ual = upd_alpha(a);
+        const float ual = (float)upd_alpha<MCGState>(a);
         double n2 = 0;
         for (int lb = b.lo + b.k; lb < b.hi; lb += b.nphys) {
             int p, bi;
@@ -428,12 +445,16 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash(DslashPar
 // with t fastest, the z and t neighbours of most of the block's sites -- into
 // LDS, coalesced, once; those hops then read LDS instead of issuing four
 // reads of every such spinor to L2.
-template <int LK, int DIAG, bool INV>
+// FM: a fused step of the FP64 solvers; its terms' per-workgroup sums go to
+// a.upd_rpart.
+template <int LK, int DIAG, bool INV, int FM = 0>
 __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash_stg(DslashParams a) {
     __shared__ cplx<double> stg[12 * LYM_DSLASH_THREADS];
     if (a.skip && *a.skip) return;
     const BlockSweep b = block_sweep(a);
     const int t = (int)threadIdx.x;
+    double al = 0, sums[3] = {0, 0, 0};
+    if constexpr (FM == F64_CG) al = upd_alpha<CGState>(a);
     for (int lb = b.lo + b.k; lb < b.hi; lb += b.nphys) {
         int p, bi;
         block_of(a, b, lb, p, bi);
@@ -447,8 +468,11 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash_stg(Dslas
         }
         __syncthreads();
         const int site = base + t;
-        if (site < a.g.Vh) dslash_site<0, LK, DIAG, INV>(a, p, site, 0, 0.f, stg, base);
+        if (site < a.g.Vh)
+            dslash_site<0, LK, DIAG, INV, false, false, false, 0, FM>(a, p, site, 0, 0.f, stg, base, al, sums);
     }
+    if constexpr (FM == F64_DOT) block_sums_store<3>(sums, a.upd_rpart, a.part_stride);
+    else if constexpr (FM != F64_STORE) block_sums_store<1>(sums, a.upd_rpart, 0);
 }
 
 #endif
@@ -536,7 +560,7 @@ __global__ __launch_bounds__(2 * LYM_DSLASH_THREADS) LYM_OCC void k_dslash_split
     const size_t ks = (size_t)a.g.stride * a.nr;
     [[maybe_unused]] double n2 = 0;
     [[maybe_unused]] float ual = 0.f;
-    if constexpr (UPD) ual = upd_alpha(a);
+    if constexpr (UPD) ual = (float)upd_alpha<MCGState>(a);
     for (int lb = b.lo + b.k; lb < b.hi; lb += b.nphys) {
         int p, bi;
         block_of(a, b, lb, p, bi);
@@ -944,6 +968,15 @@ static void launch_one(const DslashParams& a, int nblocks, hipStream_t st) {
 #if LYM_STAGE_ZT
     if constexpr (PR == 0) {
         if (a.nr == 1 && a.spb == LYM_DSLASH_THREADS && !a.lane_flags) {
+            if constexpr (DIAG >= 1 && !INV) {
+                const dim3 g(nblocks), th(LYM_DSLASH_THREADS);
+                switch (a.fmode) {
+                    case F64_NORM: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_NORM>), g, th, 0, st, a); return;
+                    case F64_CG: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_CG>), g, th, 0, st, a); return;
+                    case F64_DOT: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_DOT>), g, th, 0, st, a); return;
+                    default: break;
+                }
+            }
             hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV>), dim3(nblocks), dim3(LYM_DSLASH_THREADS), 0, st, a);
             return;
         }
@@ -1044,17 +1077,23 @@ int launch_dslash(DslashParams a, int link_kind, int diag, bool inv, hipStream_t
     // value and runs the separate update when it is 0)
     if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || a.lane_ops || !whole_waves ||
         nblocks > a.norm_max || a.norm_partials)
-        a.upd_state = nullptr;
+        if (!a.fmode) a.upd_state = nullptr;
+    // the FP64 solvers' fused steps: one RHS, a diagonal and no R^-1, and room for
+    // one partial per workgroup
+    if (a.prec != 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || a.lane_ops || a.threads ||
+        nblocks > a.part_stride || !LYM_STAGE_ZT)
+        a.fmode = F64_STORE;
+    const bool fused = a.norm_partials || a.upd_state || a.fmode;
     if (hop_blocks) {
         launch_dslash_hop(a, link_kind, diag, inv, nblocks, st);
-        return (a.norm_partials || a.upd_state) ? nblocks : 0;
+        return fused ? nblocks : 0;
     }
     switch (a.prec) {
         case 0: launch_pr<0>(a, link_kind, diag, inv, nblocks, st); break;
         case 1: launch_pr<1>(a, link_kind, diag, inv, nblocks, st); break;
         default: launch_pr<2>(a, link_kind, diag, inv, nblocks, st); break;
     }
-    return (a.norm_partials || a.upd_state) ? nblocks : 0;
+    return fused ? nblocks : 0;
 }
 
 }  // namespace lym

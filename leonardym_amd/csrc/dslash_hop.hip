@@ -177,6 +177,32 @@ struct UpdPair {
     }
 };
 
+// The same for the FP64 CG (F64_CG).
+struct UpdPair64 {
+    zd p[2], x[2], r[2];
+    __device__ __forceinline__ void load(const DslashParams& a, int par, unsigned o, int w) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const size_t c = (size_t)(2 * w + k) * a.g.stride;
+            p[k] = fld<zd>(reinterpret_cast<const zd*>(a.upd_p[par]) + c, o);
+            x[k] = fld<zd>(reinterpret_cast<const zd*>(a.upd_xs[par]) + c, o);
+            r[k] = fld<zd>(reinterpret_cast<const zd*>(a.upd_rs[par]) + c, o);
+        }
+    }
+    __device__ __forceinline__ double step(const DslashParams& a, int par, unsigned o, int w, double al, zd v0, zd v1) {
+        double n2 = 0;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const size_t c = (size_t)(2 * w + k) * a.g.stride;
+            const zd rn = axpy1(-al, k ? v1 : v0, r[k]);
+            fst<zd, false>(reinterpret_cast<zd*>(a.upd_xs[par]) + c, o, axpy1(al, p[k], x[k]));
+            fst<zd, false>(reinterpret_cast<zd*>(a.upd_rs[par]) + c, o, rn);
+            n2 = norm_acc(rn, n2);
+        }
+        return n2;
+    }
+};
+
 // sum over a wave, in every lane
 __device__ __forceinline__ double wave_total(double v) {
 #pragma unroll
@@ -185,19 +211,22 @@ __device__ __forceinline__ double wave_total(double v) {
 }
 
 // One workgroup: the spb sites of one block x nr right-hand sides (rhs
-// fastest, spb * nr <= 64).  LO: per-lane operators.
-template <int PR, int LK, int DIAG, bool INV, int MODE, bool LO>
+// fastest, spb * nr <= 64).  LO: per-lane operators.  FM: a fused step of the FP64
+// solvers (F64_*).
+template <int PR, int LK, int DIAG, bool INV, int MODE, bool LO, int FM = F64_STORE>
 __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void k_dslash_hop(DslashParams a) {
     typedef typename Prec<PR>::T T;
     typedef typename Prec<PR>::S S;
     static_assert(MODE == HOP_STORE || (PR >= 1 && DIAG >= 1 && !INV), "fused steps: low precision, last launch");
+    static_assert(FM == F64_STORE || (PR == 0 && DIAG >= 1 && !INV && !LO), "the FP64 solvers' fused steps");
     __shared__ cplx<T> xch[8][6 * HOP_LANES];
     __shared__ float fsc[PR == 2 ? 8 : 1][HOP_LANES];
     constexpr bool UPDATE = MODE == HOP_UPD || MODE == HOP_BM2;
     __shared__ double half_sum[MODE == HOP_STORE || UPDATE ? 1 : HOP_LANES];
-    __shared__ cplx<T> vout[UPDATE ? 12 : 1][HOP_LANES];
+    __shared__ cplx<T> vout[UPDATE || FM == F64_CG ? 12 : 1][HOP_LANES];
     __shared__ double pair_sum[UPDATE ? HOP_WAVES + 2 : 1][HOP_LANES];
     __shared__ float al_sh[1];
+    __shared__ double al64[1], wsum[3][HOP_WAVES + 2];
     __shared__ float half_max[PR == 2 ? 2 : 1][HOP_LANES];
     if (a.skip && *a.skip) return;
     const int lane = (int)threadIdx.x & 63;
@@ -244,8 +273,27 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
                 if constexpr (PR == 2) fsc[2 * w + i][lane] = f[i];
             }
         }
+        if constexpr (FM == F64_CG) {
+            // (its operands are on their way while the workgroup gathers)
+            UpdPair64 u64;
+            if (ok) u64.load(a, p, o, w);
+            __syncthreads();
+            __syncthreads();
+            const double t =
+                wave_total(ok ? u64.step(a, p, o, w, al64[0], vout[2 * w][lane], vout[2 * w + 1][lane]) : 0.0);
+            if (lane == 0) wsum[0][w] = t;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                double n2 = 0;
+                for (int k = 0; k < HOP_WAVES + 2; ++k) n2 += wsum[0][k];
+                a.upd_rpart[blockIdx.x] = n2;
+            }
+            return;
+        }
         __syncthreads();
-        if constexpr (UPDATE) {
+        if constexpr (FM != F64_STORE) {
+            __syncthreads();
+        } else if constexpr (UPDATE) {
             __syncthreads();
             pair_sum[w][lane] = ok ? up.step(a, p, ks, o, w, MODE == HOP_BM2 ? (float)a.balpha[r] : al_sh[0],
                                              vout[2 * w][lane], vout[2 * w + 1][lane])
@@ -314,6 +362,23 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
         }
         const double kap = LO ? a.kappa_dev[r] : (a.kappa_dev ? *a.kappa_dev : a.kappa);
         hk = (T)(-kap * a.hop_sign);
+    }
+    [[maybe_unused]] UpdPair64 u64;
+    [[maybe_unused]] cplx<T> dw[6];
+    if constexpr (FM == F64_CG) {
+        if (ok) u64.load(a, p, o, w);
+        if (h == 0) {
+            double d = 0;
+            for (int k = lane; k < a.upd_ndot; k += 64) d += a.upd_dot[k];
+            CGState* st = reinterpret_cast<CGState*>(a.upd_state);
+            const double rr = st->rr, alpha = rr / wave_total(d);
+            if (lane == 0) {
+                al64[0] = alpha;
+                if (blockIdx.x == 0) set_alpha(st, alpha, rr);
+            }
+        }
+    } else if constexpr (FM == F64_DOT) {
+        if (ok) load_half<PR>(a.dotw[p], ks, o, h, dw);
     }
     if constexpr (MODE == HOP_UPD) {
         // alpha = rr_s / <p, Ap>, folded by every workgroup in one order
@@ -387,7 +452,16 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
             }
         }
     }
-    if constexpr (UPDATE) {
+    if constexpr (FM == F64_CG) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) vout[6 * h + k][lane] = v[k];
+        __syncthreads();
+        const double t =
+            wave_total(ok ? u64.step(a, p, o, w, al64[0], vout[2 * w][lane], vout[2 * w + 1][lane]) : 0.0);
+        if (lane == 0) wsum[0][w] = t;
+        __syncthreads();
+        return;
+    } else if constexpr (UPDATE) {
         // v in FP32 to every wave, never rounded to storage
 #pragma unroll
         for (int k = 0; k < 6; ++k) vout[6 * h + k][lane] = v[k];
@@ -431,6 +505,32 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
                 if (PR == 2 && h == 0) fst<float, false>(a.out_sc[p], o, m);
             }
         }
+        if constexpr (FM != F64_STORE) {
+            // (lanes without a site hold zeros in v)
+            double sums[3] = {0, 0, 0};
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                if constexpr (FM == F64_DOT) {
+                    const zd wv = ok ? dw[k] : mk(0.0, 0.0);
+                    sums[0] = fmadd(wv.im, v[k].im, fmadd(wv.re, v[k].re, sums[0]));
+                    sums[1] = fmadd(-wv.im, v[k].re, fmadd(wv.re, v[k].im, sums[1]));
+                    sums[2] = norm_acc(v[k], sums[2]);
+                } else {
+                    sums[0] = norm_acc(v[k], sums[0]);
+                }
+            }
+            constexpr int NS = FM == F64_DOT ? 3 : 1;
+#pragma unroll
+            for (int k = 0; k < NS; ++k) {
+                sums[k] = wave_total(sums[k]);
+                if (h == 1 && lane == 0) wsum[k][0] = sums[k];
+            }
+            __syncthreads();
+            if (h == 0 && lane == 0)
+#pragma unroll
+                for (int k = 0; k < NS; ++k)
+                    a.upd_rpart[(size_t)k * a.part_stride + blockIdx.x] = sums[k] + wsum[k][0];
+        }
         if constexpr (MODE != HOP_STORE) {
             if (h == 0) {
                 n2 += (float)half_sum[lane];
@@ -457,6 +557,23 @@ static void hop_go(const DslashParams& a, int nblocks, hipStream_t st) {
     hipLaunchKernelGGL((k_dslash_hop<PR, LK, DIAG, INV, MODE, false>), dim3(nblocks), dim3(HOP_THREADS), 0, st, a);
 }
 
+// the FP64 solvers' fused steps
+template <int LK, int DIAG>
+static void hop_f64(const DslashParams& a, int nblocks, hipStream_t st) {
+    const dim3 g(nblocks), t(HOP_THREADS);
+    switch (a.fmode) {
+        case F64_NORM:
+            hipLaunchKernelGGL((k_dslash_hop<0, LK, DIAG, false, HOP_STORE, false, F64_NORM>), g, t, 0, st, a);
+            break;
+        case F64_CG:
+            hipLaunchKernelGGL((k_dslash_hop<0, LK, DIAG, false, HOP_STORE, false, F64_CG>), g, t, 0, st, a);
+            break;
+        default:
+            hipLaunchKernelGGL((k_dslash_hop<0, LK, DIAG, false, HOP_STORE, false, F64_DOT>), g, t, 0, st, a);
+            break;
+    }
+}
+
 template <int PR, int LK>
 static void hop_lk(const DslashParams& a, int diag, bool inv, int nblocks, hipStream_t st) {
     if (diag == 0) {
@@ -477,6 +594,13 @@ static void hop_lk(const DslashParams& a, int diag, bool inv, int nblocks, hipSt
                 else if (a.upd_state) hop_go<PR, LK, 2, false, HOP_UPD>(a, nblocks, st);
                 else hop_go<PR, LK, 2, false, HOP_NORM>(a, nblocks, st);
             }
+            return;
+        }
+    }
+    if constexpr (PR == 0) {
+        if (a.fmode) {
+            if (diag == 1) hop_f64<LK, 1>(a, nblocks, st);
+            else hop_f64<LK, 2>(a, nblocks, st);
             return;
         }
     }

@@ -7,6 +7,9 @@ namespace lym {
 
 typedef cplx<double> zd;
 
+// Fused steps of the FP64 solvers on a stencil launch (DslashParams::fmode)
+enum { F64_STORE = 0, F64_NORM = 1, F64_CG = 2, F64_DOT = 3 };
+
 // Parameters of one stencil launch.  Field pointers are per parity; the
 // storage element type follows `prec` (0 FP64, 1 FP32, 2 FP16 + per-site
 // scales); multi-RHS fields hold `nr` right-hand sides, rhs fastest.
@@ -79,6 +82,27 @@ struct DslashParams {
     int bmode;
     double* bsite[2];
     const double* balpha;
+    // A fused step of the FP64 solvers (single RHS), from the output v before it
+    // is stored: F64_NORM |v|^2; F64_CG x += alpha p, r -= alpha v and |r|^2, as
+    // the fused update above (upd_state a CGState, upd_p / upd_xs / upd_rs the FP64
+    // p, x, r; v is not stored); F64_DOT <w, v> (dotw) and |v|^2.  Workgroup b
+    // writes its sum k to upd_rpart[k * part_stride + b].
+    int fmode;
+    const void* dotw[2];
+    int part_stride;
+};
+// The arguments of such a step for vectors of one parity (an odd half) or two
+struct Fuse64 {
+    int mode;
+    double* part;     // sums: part[k * part_stride + workgroup]
+    int part_stride;  // most workgroups it holds
+    const zd* w;      // F64_DOT
+    void* state;      // F64_CG: CGState, the <p, Ap> partials, p, x, r
+    const double* dot;
+    int ndot;
+    const zd* p;
+    zd* x;
+    zd* r;
 };
 
 // Arguments of the fused mixed-CG update (DslashParams::upd_*) for one vector
@@ -142,34 +166,48 @@ struct CGState {
     double rr_prev;  // rr at the start of the iteration (set by the update, read by the p update)
 };
 
+enum { BICG_FOLD = 0, BICG_CHECKED = 1, BICG_FIRST = 2 };
 struct BiCGState {
     int done, converged, step, max_steps, breakdown, copy_b;
+    int phase;  // what the next p update finds: BICG_FOLD the last update's partials, BICG_CHECKED
+                // those already folded by launch_bicg_check, BICG_FIRST the start's <rh, r> only
     double rho_re, rho_im, rhon_re, rhon_im;
     double alpha_re, alpha_im, omega_re, omega_im, beta_re, beta_im;
     double norm, precision;
 };
 
 void launch_cg_init(CGState* s, const zd* r, long n, double* partials, double eps, int max_steps, hipStream_t st);
-// one CG iteration after Ap = A p: <p, Ap> partials (slots 0, 1 of partials),
-// the update folding them into alpha (|r|^2 partials into slot 2), the p update
-// folding those into beta and the stopping rule
+// The steps of an iteration that are not fused into the stencil fold npart
+// partial sums of the step before (sum k of workgroup b at part[k * stride + b]).
+// launch_fold folds more than FOLD_MAX of them into one; npart and part then
+// describe the result.
+constexpr int FOLD_MAX = 2048;
+void launch_fold(int nv, const double*& part, int stride, int& npart, double* out, const int* skip, hipStream_t st);
+// one CG iteration after Ap = A p, for maps whose <p, Ap> is not |Q p|^2: <p, Ap>
+// partials (slots 0, 1 of partials), the update folding them into alpha (|r|^2
+// partials into slot 2)
 void launch_cg_alpha(CGState* s, const zd* p, const zd* Ap, long n, double* partials, hipStream_t st);
 void launch_cg_update(CGState* s, zd* x, zd* r, const zd* p, const zd* Ap, long n, double* partials,
                       hipStream_t st);
-void launch_cg_p(CGState* s, zd* p, const zd* r, long n, double* partials, hipStream_t st);
+// the p update, folding the |r|^2 partials into beta and the stopping rule
+void launch_cg_p(CGState* s, zd* p, const zd* r, long n, const double* part, int npart, hipStream_t st);
 
 void launch_bicg_init(BiCGState* s, double precision, int max_steps, hipStream_t st);
-// r = b - Ax, rh = b + Ax, p = nu = 0
-void launch_bicg_setup(zd* r, zd* rh, zd* p, zd* nu, const zd* b, const zd* Ax, long n, hipStream_t st);
-void launch_bicg_rho(BiCGState* s, const zd* rh, const zd* r, long n, double* partials, hipStream_t st);
-// the p, s and x/r updates fold the partials of the dot launched before them
-// (rho, alpha, omega) into their scalars
-void launch_bicg_p(BiCGState* s, zd* p, const zd* r, const zd* nu, long n, const double* partials, hipStream_t st);
-void launch_bicg_alpha(BiCGState* s, const zd* rh, const zd* nu, long n, double* partials, hipStream_t st);
-void launch_bicg_s(BiCGState* s, zd* sv, const zd* r, const zd* nu, long n, const double* partials, hipStream_t st);
-void launch_bicg_omega(BiCGState* s, const zd* t, const zd* sv, long n, double* partials, hipStream_t st);
-void launch_bicg_update(BiCGState* s, zd* x, zd* r, const zd* p, const zd* sv, const zd* t, const zd* b, long n,
-                        double* partials, hipStream_t st);
+// r = b - Ax, rh = b + Ax, p = nu = 0, and <rh, r> into the partials of launch_bicg_update
+void launch_bicg_setup(zd* r, zd* rh, zd* p, zd* nu, const zd* b, const zd* Ax, long n, double* partials, int stride,
+                       hipStream_t st);
+// One iteration: the p update (folding the last update's <rh, r> and |r|^2: the
+// stopping rule and beta), the stencil of nu with <rh, nu> fused (npart partials),
+// the s update, the stencil of t with <s, t> and |t|^2 fused, the x and r update
+// (leaving <rh, r> and |r|^2 partials at partials[k * stride + workgroup]).
+void launch_bicg_p(BiCGState* s, zd* p, const zd* r, const zd* nu, long n, const double* partials, int stride,
+                   hipStream_t st);
+void launch_bicg_s(BiCGState* s, zd* sv, const zd* r, const zd* nu, long n, const double* part, int stride, int npart,
+                   hipStream_t st);
+void launch_bicg_update(BiCGState* s, zd* x, zd* r, const zd* rh, const zd* p, const zd* sv, const zd* t, const zd* b,
+                        long n, const double* part, int stride, int npart, double* partials, hipStream_t st);
+// the stopping rule of the last update, before the host reads the state
+void launch_bicg_check(BiCGState* s, const double* partials, int stride, hipStream_t st);
 
 }  // namespace lym
 

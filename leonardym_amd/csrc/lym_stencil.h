@@ -128,6 +128,53 @@ __device__ __forceinline__ void hop_dir(cplx<T> acc[12], const cplx<T> psi[12], 
     }
 }
 
+// ---------------------------------------------------------------- fused steps of the FP64 solvers
+// On small lattices an FP64 Krylov iteration is bound by its launches (a launch
+// that does nothing takes 1.7 us in a replayed graph, a dot or a vector update of
+// a few thousand elements 3 to 4 us): with the dots and the CG update on the
+// launches that write Q p, A p, nu and t, a CG iteration on Q^2 is 5 launches
+// (even-odd; 3 on the full lattice) instead of 7 (5) and a BiCGStab one 3 and its
+// stencils instead of 8.  8^4 Wilson CG 3.35 -> 2.80 ms, BiCGStab of the 8^3x16
+// fermion force 28.7 -> 23.2 ms; on 16^3x32 the dot costs the stencil 4.3 us of
+// the 5.9 us it took alone and a solve gains 0.5 %.
+__device__ __forceinline__ double state_rr(const MCGState* s) { return s->rr_s; }
+__device__ __forceinline__ double state_rr(const CGState* s) { return s->rr; }
+__device__ __forceinline__ void set_alpha(MCGState* s, double alpha, double rr) {
+    s->alpha = alpha;
+    s->rr_prev = rr;
+}
+__device__ __forceinline__ void set_alpha(CGState* s, double alpha, double rr) {
+    s->alpha_re = alpha;
+    s->alpha_im = 0;
+    s->rr_prev = rr;
+}
+
+// The step's work on component k of a site, from its output v (in registers):
+//   F64_NORM  sums[0] += |v|^2
+//   F64_CG    x += al p, r -= al v, sums[0] += |r|^2 (the output is not stored)
+//   F64_DOT   sums[0], [1] += conj(w) v, sums[2] += |v|^2
+template <int FM>
+__device__ __forceinline__ void f64_step(const DslashParams& a, int p, int k, unsigned site, double al, zd v,
+                                         double* sums) {
+    const size_t o = (size_t)k * a.g.stride;
+    if constexpr (FM == F64_NORM) {
+        sums[0] = norm_acc(v, sums[0]);
+    } else if constexpr (FM == F64_CG) {
+        const zd pv = fld<zd>(reinterpret_cast<const zd*>(a.upd_p[p]) + o, site);
+        zd* xp = reinterpret_cast<zd*>(a.upd_xs[p]) + o;
+        zd* rp = reinterpret_cast<zd*>(a.upd_rs[p]) + o;
+        const zd rn = axpy1(-al, v, fld<zd>(rp, site));
+        fst<zd, false>(xp, site, axpy1(al, pv, fld<zd>(xp, site)));
+        fst<zd, false>(rp, site, rn);
+        sums[0] = norm_acc(rn, sums[0]);
+    } else if constexpr (FM == F64_DOT) {
+        const zd w = fld<zd>(reinterpret_cast<const zd*>(a.dotw[p]) + o, site);
+        sums[0] = fmadd(w.im, v.im, fmadd(w.re, v.re, sums[0]));
+        sums[1] = fmadd(-w.im, v.re, fmadd(w.re, v.im, sums[1]));
+        sums[2] = norm_acc(v, sums[2]);
+    }
+}
+
 // Grid: gridDim.x workgroups dealt round-robin over the 8 XCDs.  XCD x owns a
 // contiguous range of logical site blocks (x-major lattice order, the two
 // parities of a block range interleaved) and its workgroups sweep that range

@@ -35,9 +35,13 @@ using lym::zd;
 namespace lym_internal {
 int fail(int code, const char* fmt, ...);
 int op_ready(lym_op* op, bool force_blocks);
-void apply_schur(lym_op* op, zd* out_o, const zd* in_o, int gamma5, const int* skip);
-void apply_full(lym_op* op, zd* out, const zd* in, int gamma5, const int* skip);
-void apply_full_add(lym_op* op, zd* out, const zd* in, const zd* v2, zd alpha, int gamma5, const int* skip);
+// fuse: a fused step on the last launch; the return value is its number of
+// partials (one per workgroup)
+int apply_schur(lym_op* op, zd* out_o, const zd* in_o, int gamma5, const int* skip,
+                const lym::Fuse64* fuse = nullptr);
+int apply_full(lym_op* op, zd* out, const zd* in, int gamma5, const int* skip, const lym::Fuse64* fuse = nullptr);
+int apply_full_add(lym_op* op, zd* out, const zd* in, const zd* v2, zd alpha, int gamma5, const int* skip,
+                   const lym::Fuse64* fuse = nullptr);
 int link_kind_of(const lym_gauge* g);
 int op_sloppy(lym_op* op, int prec, bool full_rows = false);
 // the sloppy applies can also write per-workgroup partial sums of |out|^2
@@ -78,6 +82,9 @@ struct lym_solver {
     unsigned max_steps;
     int even_odd;
     zd* w[8];
+    double* dot_part;       // partials of the FP64 solvers' steps, three of [3][dot_stride]: the
+    int dot_stride;         //   stencils' fused ones, those folded, the vector updates'
+
     void* state;
     void* host_state;
     // mixed precision
@@ -148,23 +155,25 @@ struct LinOp {
     zd* scratch;  // one vector of the map's domain
     zd shift{0.0, 0.0};  // full-lattice maps only: apply A + shift (fused into the last stencil launch)
     bool shifted() const { return shift.re != 0.0 || shift.im != 0.0; }
-    void last(zd* out, const zd* in, const zd* v, const int* skip) const {
-        if (shifted()) lym_internal::apply_full_add(op, out, in, v, shift, gamma5, skip);
-        else lym_internal::apply_full(op, out, in, gamma5, skip);
+    int last(zd* out, const zd* in, const zd* v, const int* skip, const lym::Fuse64* f) const {
+        if (shifted()) return lym_internal::apply_full_add(op, out, in, v, shift, gamma5, skip, f);
+        return lym_internal::apply_full(op, out, in, gamma5, skip, f);
     }
-    void apply(zd* out, const zd* in, const int* skip) const {
-        if (power == 1) {
-            if (half) lym_internal::apply_schur(op, out, in, gamma5, skip);
-            else last(out, in, in, skip);
-        } else {
-            if (half) {
-                lym_internal::apply_schur(op, scratch, in, gamma5, skip);
-                lym_internal::apply_schur(op, out, scratch, gamma5, skip);
-            } else {
-                lym_internal::apply_full(op, scratch, in, gamma5, skip);
-                last(out, scratch, in, skip);
-            }
-        }
+    // out = A in.  f: a fused step on the last stencil launch; the return value is
+    // its number of partials
+    int apply(zd* out, const zd* in, const int* skip, const lym::Fuse64* f = nullptr) const {
+        if (power == 1) return half ? lym_internal::apply_schur(op, out, in, gamma5, skip, f) : last(out, in, in, skip, f);
+        first(in, skip, nullptr);
+        return second(out, in, skip, f);
+    }
+    // the two factors of A = Q^2: scratch = Q in, then out = Q scratch (+ shift in)
+    int first(const zd* in, const int* skip, const lym::Fuse64* f) const {
+        if (half) return lym_internal::apply_schur(op, scratch, in, gamma5, skip, f);
+        return lym_internal::apply_full(op, scratch, in, gamma5, skip, f);
+    }
+    int second(zd* out, const zd* in, const int* skip, const lym::Fuse64* f) const {
+        if (half) return lym_internal::apply_schur(op, out, scratch, gamma5, skip, f);
+        return last(out, scratch, in, skip, f);
     }
 };
 
@@ -175,6 +184,10 @@ int ensure_work(lym_solver* s) {
         if (hipMalloc((void**)&s->w[i], bytes) != hipSuccess) return fail(LYM_ERR_NOMEM, "solver work vectors");
         if (hipMemsetAsync(s->w[i], 0, bytes, s->ctx->stream) != hipSuccess) return fail(LYM_ERR_DEVICE, "hipMemsetAsync");
     }
+    // one partial per workgroup of a stencil launch of both parities, however split
+    s->dot_stride = (int)std::max<long>(8192, 2 * (((long)s->ctx->g.Vh + 255) / 256));
+    if (hipMalloc((void**)&s->dot_part, 9 * sizeof(double) * (size_t)s->dot_stride) != hipSuccess)
+        return fail(LYM_ERR_NOMEM, "solver partials");
     if (hipMalloc(&s->state, 256) != hipSuccess) return fail(LYM_ERR_NOMEM, "solver state");
     if (hipHostMalloc(&s->host_state, 256, hipHostMallocDefault) != hipSuccess)
         return fail(LYM_ERR_DEVICE, "hipHostMalloc");
@@ -352,11 +365,29 @@ int run_cg(lym_solver* s, const LinOp& L, const zd* b, zd* xout, const zd* x0, l
     key << 1 << s << n << b;
     key_op(key, L.op);
     key << L.half << L.gamma5 << L.power << L.scratch;
+    // A = Q^2 with Q hermitian: <p, A p> = |Q p|^2, summed by the launch that writes
+    // Q p, and the update x += alpha p, r -= alpha A p runs on the last launch of
+    // A p, which then does not store it
+    const bool fused = L.power == 2 && L.gamma5 && !L.shifted();
+    const int* done = &S->done;
     auto body = [&](unsigned) {
-        L.apply(Ap, p, &S->done);
-        lym::launch_cg_alpha(S, p, Ap, n, c->red_partials, st);
-        lym::launch_cg_update(S, x, r, p, Ap, n, c->red_partials, st);
-        lym::launch_cg_p(S, p, r, n, c->red_partials, st);
+        const double* part = c->red_partials + 2 * lym::RED_BLOCKS;
+        int npart = lym::RED_BLOCKS;
+        if (fused) {
+            lym::Fuse64 f{lym::F64_NORM, s->dot_part, s->dot_stride};
+            int nd = L.first(p, done, &f);
+            const double* dot = s->dot_part;
+            lym::launch_fold(1, dot, s->dot_stride, nd, s->dot_part + 3 * (size_t)s->dot_stride, done, st);
+            f = {lym::F64_CG, s->dot_part + s->dot_stride, s->dot_stride, nullptr, S, dot, nd, p, x, r};
+            npart = L.second(Ap, p, done, &f);
+            part = f.part;
+            lym::launch_fold(1, part, s->dot_stride, npart, s->dot_part + 4 * (size_t)s->dot_stride, done, st);
+        } else {
+            L.apply(Ap, p, done);
+            lym::launch_cg_alpha(S, p, Ap, n, c->red_partials, st);
+            lym::launch_cg_update(S, x, r, p, Ap, n, c->red_partials, st);
+        }
+        lym::launch_cg_p(S, p, r, n, part, npart, st);
     };
     while (!H->done && queued <= s->max_steps) {
         unsigned k = next_chunk(r0, H->rr, (unsigned)H->step, s->precision, s->max_steps + 1 - queued);
@@ -395,7 +426,10 @@ int run_bicgstab(lym_solver* s, const LinOp& L, const zd* b, zd* xout, const zd*
                                  st);
     }
     L.apply(t, x, nullptr);
-    lym::launch_bicg_setup(r, rh, p, nu, b, t, n, st);
+    // <rh, r> and |r|^2 partials of the setup and of every update
+    const int ds = s->dot_stride;
+    double* part = s->dot_part + 6 * (size_t)ds;
+    lym::launch_bicg_setup(r, rh, p, nu, b, t, n, part, ds, st);
     lym::launch_bicg_init(S, s->precision, (int)s->max_steps, st);
     HIPCHECK(hipMemcpyAsync(H, S, sizeof(lym::BiCGState), hipMemcpyDeviceToHost, st));
     HIPCHECK(hipStreamSynchronize(st));
@@ -406,21 +440,27 @@ int run_bicgstab(lym_solver* s, const LinOp& L, const zd* b, zd* xout, const zd*
     key << 2 << s << n << b;
     key_op(key, L.op);
     key << L.half << L.gamma5 << L.power << L.scratch << L.shift.re << L.shift.im;
+    const int* done = &S->done;
     auto body = [&](unsigned) {
-        lym::launch_bicg_rho(S, rh, r, n, c->red_partials, st);
-        lym::launch_bicg_p(S, p, r, nu, n, c->red_partials, st);
-        L.apply(nu, p, &S->done);
-        lym::launch_bicg_alpha(S, rh, nu, n, c->red_partials, st);
-        lym::launch_bicg_s(S, sv, r, nu, n, c->red_partials, st);
-        L.apply(t, sv, &S->done);
-        lym::launch_bicg_omega(S, t, sv, n, c->red_partials, st);
-        lym::launch_bicg_update(S, x, r, p, sv, t, b, n, c->red_partials, st);
+        lym::launch_bicg_p(S, p, r, nu, n, part, ds, st);
+        // <rh, nu>, then <s, t> and |t|^2, summed by the launches that write nu and t
+        lym::Fuse64 f{lym::F64_DOT, s->dot_part, ds, rh};
+        const double* dot = s->dot_part;
+        int nd = L.apply(nu, p, done, &f);
+        lym::launch_fold(3, dot, ds, nd, s->dot_part + 3 * (size_t)ds, done, st);
+        lym::launch_bicg_s(S, sv, r, nu, n, dot, ds, nd, st);
+        f.w = sv;
+        dot = s->dot_part;
+        nd = L.apply(t, sv, done, &f);
+        lym::launch_fold(3, dot, ds, nd, s->dot_part + 3 * (size_t)ds, done, st);
+        lym::launch_bicg_update(S, x, r, rh, p, sv, t, b, n, dot, ds, nd, part, st);
     };
     while (!H->done && queued <= s->max_steps) {
         unsigned k = next_chunk(r0, rnow, (unsigned)H->step, s->precision, s->max_steps + 1 - queued);
         int rc = queue_iterations(s, key.h, L.op->uid, k, body, &queued);
         if (rc) return rc;
         HIPCHECK(hipGetLastError());
+        lym::launch_bicg_check(S, part, ds, st);
         HIPCHECK(hipMemcpyAsync(H, S, sizeof(lym::BiCGState), hipMemcpyDeviceToHost, st));
         HIPCHECK(hipStreamSynchronize(st));
         rnow = H->norm;
@@ -1190,6 +1230,7 @@ void lym_solver_destroy(lym_solver* s) {
     if (s->ctx && s->ctx->stream) (void)hipStreamSynchronize(s->ctx->stream);
     for (int i = 0; i < 8; ++i)
         if (s->w[i]) (void)hipFree(s->w[i]);
+    if (s->dot_part) (void)hipFree(s->dot_part);
     if (s->state) (void)hipFree(s->state);
     for (int i = 0; i < 4; ++i) {
         if (s->sv[i]) (void)hipFree(s->sv[i]);
