@@ -427,18 +427,29 @@ static void set_bfuse(lym::DslashParams& a, const lym::BFuse& f, const lym_ctx* 
     }
 }
 
-// full lattice, nr right-hand sides, storage precision prec: out = Op in
+// FP64 launch over nr lane fields with these lane strides
+static void set_lanes(lym::DslashParams& a, int nr, long in_lane, long diag_lane, long out_lane) {
+    a.nr = 1;
+    a.lanes = nr;
+    a.in_lane = in_lane;
+    a.diag_lane = diag_lane;
+    a.out_lane = out_lane;
+}
+
+// full lattice, nr right-hand sides, storage precision prec (FP64: lane fields): out = Op in
 int apply_full_nr(lym_op* op, int prec, int nr, int threads, void* out, float* out_sc, const void* in,
                   const float* in_sc, int gamma5, const int* skip, const int* lane_flags, int lane_skip_value,
                   bool batch_links, double* norm_partials, int norm_max, int mfma, const lym::UpdArgs* upd,
                   const lym::BFuse* bf) {
     lym_ctx* c = op->ctx;
-    const size_t po = 12 * (size_t)c->g.stride * nr * selem(prec);
+    // FP64: lane fields of 24 strides each; else one field with nr interleaved RHS
+    const size_t po = 12 * (size_t)c->g.stride * (prec ? nr : 1) * selem(prec);
     const size_t so = (size_t)c->g.stride * nr;
     lym::DslashParams a = base_params(op);
     const int lk = set_op_data(a, op, prec, batch_links);
     a.allow_split = !batch_links;  // batches keep one form for every width (same bits)
     a.nr = nr;
+    if (prec == 0) set_lanes(a, nr, full_n(c), full_n(c), full_n(c));
     a.threads = threads;
     for (int p = 0; p < 2; ++p) {
         a.in[p] = (const char*)in + p * po;
@@ -473,6 +484,7 @@ int apply_schur_nr(lym_op* op, int prec, int nr, int threads, void* out_o, float
     const int lk = set_op_data(a, op, prec, batch_links);
     a.allow_split = !batch_links;  // batches keep one form for every width (same bits)
     a.nr = nr;
+    if (prec == 0) set_lanes(a, nr, half_n(c), half_n(c), half_n(c));
     a.threads = threads;
     a.mfma = mfma;
     a.skip = skip;
@@ -514,30 +526,33 @@ int apply_schur_sloppy(lym_op* op, int prec, void* out_o, float* out_sc, const v
                           norm_partials, norm_max, 0, upd, nullptr);
 }
 
-// the EO driver's source and reconstruction steps on nr-fields (FP64)
+// the EO driver's source and reconstruction steps on nr FP64 lane fields: b full
+// fields (even half b_e, odd half b_o at its lane), te, src_o and x_e lanes of
+// their own strides
 // src_o = b_o - D_oe Ainv b_e  (te: even scratch)
-void eo_source_nr(lym_op* op, int nr, const zd* b_e, const zd* b_o, zd* te, zd* src_o) {
+void eo_source_nr(lym_op* op, int nr, const zd* b, zd* te, zd* src_o) {
     lym_ctx* c = op->ctx;
-    lym::launch_clover_apply_nr(c->g, reinterpret_cast<const zd*>(op->Ainv), b_e, te, nr, c->stream);
+    lym::launch_clover_apply_lanes(c->g, reinterpret_cast<const zd*>(op->Ainv), 0, nullptr, nullptr, b, full_n(c), te,
+                                   half_n(c), nr, c->stream);
     lym::DslashParams a = base_params(op);
-    a.nr = nr;
+    set_lanes(a, nr, half_n(c), full_n(c), half_n(c));
     a.hop_sign = -1.0;
     a.parity = 1;
     a.in[0] = te;
-    a.diag_in[1] = b_o;
+    a.diag_in[1] = par(b, c, 1);
     a.out[1] = src_o;
     lym::launch_dslash(a, link_kind(op->gauge), 1, false, c->stream);
 }
-// x_e = Ainv (b_e - D_eo x_o)
-void eo_reconstruct_nr(lym_op* op, int nr, const zd* b_e, const zd* x_o, zd* x_e) {
+// the even halves of full fields X from their odd halves: x_e = Ainv (b_e - D_eo x_o)
+void eo_reconstruct_nr(lym_op* op, int nr, const zd* b, zd* X) {
     lym_ctx* c = op->ctx;
     lym::DslashParams a = base_params(op);
-    a.nr = nr;
+    set_lanes(a, nr, full_n(c), full_n(c), full_n(c));
     a.hop_sign = -1.0;
     a.parity = 0;
-    a.in[1] = x_o;
-    a.diag_in[0] = b_e;
-    a.out[0] = x_e;
+    a.in[1] = par(X, c, 1);
+    a.diag_in[0] = b;
+    a.out[0] = X;
     lym::launch_dslash(a, link_kind(op->gauge), 1, true, c->stream);
 }
 }  // namespace lym_internal

@@ -122,6 +122,20 @@ __device__ __forceinline__ void bs_store(typename Prec<PR>::S* d, float* sc, int
     }
 }
 
+// FP64 lane fields: lane r holds [nparity][12][stride] of its own (nsites = nparity * stride)
+__device__ __forceinline__ void ld_lane(const zd* d, long nsites, int stride, long j, int r, zd s[12]) {
+    const long p = j / stride, i = j - p * stride;
+    const zd* b = d + (r * nsites + p * stride) * 12 + i;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) s[k] = b[(long)k * stride];
+}
+__device__ __forceinline__ void st_lane(zd* d, long nsites, int stride, long j, int r, const zd s[12]) {
+    const long p = j / stride, i = j - p * stride;
+    zd* b = d + (r * nsites + p * stride) * 12 + i;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) b[(long)k * stride] = s[k];
+}
+
 template <class E, int NR>
 __device__ __forceinline__ void bg_load(const E* d, int stride, long j, int r, E s[12]) {
 #pragma unroll
@@ -147,7 +161,7 @@ __global__ __launch_bounds__(BC * NR) void k_bcg_init(const zd* r, cplx<float>* 
     if (chunk_pair<NR>(nsites, j, q) && (!mask || mask[q])) {
         zd a[12];
         cplx<float> f[12], z[12];
-        bg_load<zd, NR>(r, stride, j, q, a);
+        ld_lane(r, nsites, stride, j, q, a);
 #pragma unroll
         for (int k = 0; k < 12; ++k) {
             v += a[k].re * a[k].re + a[k].im * a[k].im;
@@ -300,14 +314,14 @@ __global__ void k_brel_accum(const BState* s, zd* x, cplx<float>* xs, long nsite
         if (!s->rel[q]) continue;
         zd a[12];
         cplx<float> f[12];
-        bg_load<zd, NR>(x, stride, j, (int)q, a);
+        ld_lane(x, nsites, stride, j, (int)q, a);
         bg_load<cplx<float>, NR>(xs, stride, j, (int)q, f);
 #pragma unroll
         for (int k = 0; k < 12; ++k) {
             a[k] = a[k] + mk((double)f[k].re, (double)f[k].im);
             f[k] = mk(0.f, 0.f);
         }
-        bg_store<zd, NR>(x, stride, j, (int)q, a);
+        st_lane(x, nsites, stride, j, (int)q, a);
         bg_store<cplx<float>, NR>(xs, stride, j, (int)q, f);
     }
 }
@@ -324,15 +338,15 @@ __global__ __launch_bounds__(BC * NR) void k_brel_resid(const BState* s, zd* r, 
     if (chunk_pair<NR>(nsites, j, q) && s->rel[q]) {
         zd bb[12], ax[12];
         cplx<float> f[12];
-        bg_load<zd, NR>(b, stride, j, q, bb);
-        bg_load<zd, NR>(Ax, stride, j, q, ax);
+        ld_lane(b, nsites, stride, j, q, bb);
+        ld_lane(Ax, nsites, stride, j, q, ax);
 #pragma unroll
         for (int k = 0; k < 12; ++k) {
             bb[k] = bb[k] - ax[k];
             v += bb[k].re * bb[k].re + bb[k].im * bb[k].im;
             f[k] = mk((float)bb[k].re, (float)bb[k].im);
         }
-        bg_store<zd, NR>(r, stride, j, q, bb);
+        st_lane(r, nsites, stride, j, q, bb);
         bg_store<cplx<float>, NR>(rs, stride, j, q, f);
     }
     chunk_store<NR>(v, partials, nchunks);
@@ -390,11 +404,11 @@ __global__ void k_baccum(const BState* s, zd* x, const cplx<float>* xs, long nsi
         if (s->conv[q] || (mask && !mask[q])) continue;
         zd a[12];
         cplx<float> f[12];
-        bg_load<zd, NR>(x, stride, j, (int)q, a);
+        ld_lane(x, nsites, stride, j, (int)q, a);
         bg_load<cplx<float>, NR>(xs, stride, j, (int)q, f);
 #pragma unroll
         for (int k = 0; k < 12; ++k) a[k] = a[k] + mk((double)f[k].re, (double)f[k].im);
-        bg_store<zd, NR>(x, stride, j, (int)q, a);
+        st_lane(x, nsites, stride, j, (int)q, a);
     }
 }
 
@@ -413,20 +427,29 @@ __global__ void k_unpack(const zd* multi, int nr, zd* const* dsts, long n) {
     }
 }
 
-// ---------------------------------------------------------------- lanes of an nr-field
-// An nr-field is rows x nr elements, lane fastest.  These act on the lanes
-// with mask[q] != 0 only, or move every lane to another width.
-template <class E>
-__global__ void k_lane_copy(E* dst, const E* src, long rows, int nr, const int* mask) {
-    BSITE_LOOP(t, rows * nr) {
-        if (mask[t % nr]) dst[t] = src[t];
-    }
+// ---------------------------------------------------------------- lanes
+// FP64 lane fields: one grid row per lane
+__global__ void k_lane_copy(zd* dst, long dst_lane, const zd* src, long src_lane, long n, const int* mask) {
+    const int l = blockIdx.y;
+    if (mask && !mask[l]) return;
+    BSITE_LOOP(i, n) { dst[l * dst_lane + i] = src[l * src_lane + i]; }
 }
-__global__ void k_lane_sub(zd* out, const zd* a, const zd* b, long rows, int nr, const int* mask) {
-    BSITE_LOOP(t, rows * nr) {
-        if (mask[t % nr]) out[t] = a[t] - b[t];
-    }
+__global__ void k_lane_sub(zd* out, const zd* a, const zd* b, long lane, long n, const int* mask) {
+    const int l = blockIdx.y;
+    if (mask && !mask[l]) return;
+    BSITE_LOOP(i, n) { out[l * lane + i] = a[l * lane + i] - b[l * lane + i]; }
 }
+__global__ void k_lane_gather(const zd* const* srcs, zd* dst, long n) {
+    const zd* s = srcs[blockIdx.y];
+    if (!s) return;
+    BSITE_LOOP(i, n) { dst[blockIdx.y * n + i] = s[i]; }
+}
+__global__ void k_lane_scatter(const zd* src, zd* const* dsts, long n) {
+    zd* d = dsts[blockIdx.y];
+    if (!d) return;
+    BSITE_LOOP(i, n) { d[i] = src[blockIdx.y * n + i]; }
+}
+// An interleaved field is rows x nr elements, lane fastest.
 // out (width w_new) from in (width w_old): lane j keeps its index, lanes
 // j >= w_old are zero
 template <class E>
@@ -441,34 +464,18 @@ __global__ void k_relayout(const E* in, E* out, long rows, int w_old, int w_new)
     }
 }
 
-__global__ void k_clover_apply_nr(Geom g, const zd* __restrict__ blocks, const zd* __restrict__ in,
-                                  zd* __restrict__ out, int nr) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)g.Vh * nr) return;
-    const int idx = (int)(t / nr), r = (int)(t % nr);
+__global__ void k_clover_apply_lanes(Geom g, const zd* __restrict__ blocks, long set_elems, const int* lane_set,
+                                     const int* mask, const zd* __restrict__ in, long in_lane, zd* __restrict__ out,
+                                     long out_lane) {
+    const int l = blockIdx.y, idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (idx >= g.Vh || (mask && !mask[l])) return;
+    const zd* B = blocks + (lane_set ? lane_set[l] * set_elems : 0);
     zd s[12], o[12];
-#pragma unroll
-    for (int k = 0; k < 12; ++k) s[k] = in[((long)k * g.stride + idx) * nr + r];
-    herm6(blocks, g.stride, idx, s, o);
-    herm6(blocks + (size_t)18 * g.stride, g.stride, idx, s + 6, o + 6);
-#pragma unroll
-    for (int k = 0; k < 12; ++k) out[((long)k * g.stride + idx) * nr + r] = o[k];
-}
-
-__global__ void k_clover_apply_lanes(Geom g, const zd* __restrict__ blocks, long lane_elems, const int* lane_set,
-                                     const int* mask, const zd* __restrict__ in, zd* __restrict__ out, int nr) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)g.Vh * nr) return;
-    const int idx = (int)(t / nr), r = (int)(t % nr);
-    if (!mask[r]) return;
-    const zd* B = blocks + (lane_set ? lane_set[r] : r) * lane_elems;
-    zd s[12], o[12];
-#pragma unroll
-    for (int k = 0; k < 12; ++k) s[k] = in[((long)k * g.stride + idx) * nr + r];
+    load_spinor(in + l * in_lane, g.stride, idx, s);
     herm6(B, g.stride, idx, s, o);
     herm6(B + (size_t)18 * g.stride, g.stride, idx, s + 6, o + 6);
 #pragma unroll
-    for (int k = 0; k < 12; ++k) out[((long)k * g.stride + idx) * nr + r] = o[k];
+    for (int k = 0; k < 12; ++k) out[l * out_lane + (long)k * g.stride + idx] = o[k];
 }
 
 // ---------------------------------------------------------------- launchers
@@ -561,21 +568,19 @@ void launch_unpack(const zd* multi, int nr, zd* const* dsts_dev, long n, hipStre
     hipLaunchKernelGGL(k_unpack, dim3(bsite_blocks(n)), dim3(256), 0, st, multi, nr, dsts_dev, n);
 }
 
-void launch_lane_copy(int esize, void* dst, const void* src, long rows, int nr, const int* mask, hipStream_t st) {
-    const dim3 g(bsite_blocks(rows * nr)), b(256);
-    switch (esize) {
-        case 16: hipLaunchKernelGGL(k_lane_copy<zd>, g, b, 0, st, (zd*)dst, (const zd*)src, rows, nr, mask); break;
-        case 8:
-            hipLaunchKernelGGL(k_lane_copy<cplx<float>>, g, b, 0, st, (cplx<float>*)dst, (const cplx<float>*)src,
-                               rows, nr, mask);
-            break;
-        default:
-            hipLaunchKernelGGL(k_lane_copy<float>, g, b, 0, st, (float*)dst, (const float*)src, rows, nr, mask);
-            break;
-    }
+static inline dim3 lane_dim(long n, int lanes) { return dim3((unsigned)bsite_blocks(n), (unsigned)lanes); }
+void launch_lane_copy(zd* dst, long dst_lane, const zd* src, long src_lane, long n, int lanes, const int* mask,
+                      hipStream_t st) {
+    hipLaunchKernelGGL(k_lane_copy, lane_dim(n, lanes), dim3(256), 0, st, dst, dst_lane, src, src_lane, n, mask);
 }
-void launch_lane_sub(zd* out, const zd* a, const zd* b, long rows, int nr, const int* mask, hipStream_t st) {
-    hipLaunchKernelGGL(k_lane_sub, dim3(bsite_blocks(rows * nr)), dim3(256), 0, st, out, a, b, rows, nr, mask);
+void launch_lane_sub(zd* out, const zd* a, const zd* b, long lane, long n, int lanes, const int* mask, hipStream_t st) {
+    hipLaunchKernelGGL(k_lane_sub, lane_dim(n, lanes), dim3(256), 0, st, out, a, b, lane, n, mask);
+}
+void launch_lane_gather(const zd* const* srcs_dev, zd* dst, long n, int lanes, hipStream_t st) {
+    hipLaunchKernelGGL(k_lane_gather, lane_dim(n, lanes), dim3(256), 0, st, srcs_dev, dst, n);
+}
+void launch_lane_scatter(const zd* src, zd* const* dsts_dev, long n, int lanes, hipStream_t st) {
+    hipLaunchKernelGGL(k_lane_scatter, lane_dim(n, lanes), dim3(256), 0, st, src, dsts_dev, n);
 }
 void launch_relayout(int esize, const void* in, void* out, long rows, int w_old, int w_new, hipStream_t st) {
     const dim3 g(bsite_blocks(rows * w_new)), b(256);
@@ -614,15 +619,10 @@ void launch_zero_padding(int esize, void* buf, long groups, int stride, int vh, 
         default: hipLaunchKernelGGL(k_zero_padding<float>, g, b, 0, st, (float*)buf, groups, stride, vh, nr); break;
     }
 }
-void launch_clover_apply_lanes(const Geom& g, const zd* blocks, long lane_elems, const int* lane_set, const int* mask,
-                               const zd* in, zd* out, int nr, hipStream_t st) {
-    long n = (long)g.Vh * nr;
-    hipLaunchKernelGGL(k_clover_apply_lanes, dim3((n + 255) / 256), dim3(256), 0, st, g, blocks, lane_elems, lane_set,
-                       mask, in, out, nr);
-}
-void launch_clover_apply_nr(const Geom& g, const zd* blocks, const zd* in, zd* out, int nr, hipStream_t st) {
-    long n = (long)g.Vh * nr;
-    hipLaunchKernelGGL(k_clover_apply_nr, dim3((n + 255) / 256), dim3(256), 0, st, g, blocks, in, out, nr);
+void launch_clover_apply_lanes(const Geom& g, const zd* blocks, long set_elems, const int* lane_set, const int* mask,
+                               const zd* in, long in_lane, zd* out, long out_lane, int lanes, hipStream_t st) {
+    hipLaunchKernelGGL(k_clover_apply_lanes, dim3((g.Vh + 255) / 256, lanes), dim3(256), 0, st, g, blocks, set_elems,
+                       lane_set, mask, in, in_lane, out, out_lane);
 }
 
 }  // namespace lym

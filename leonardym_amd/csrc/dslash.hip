@@ -68,18 +68,6 @@
 #ifndef LYM_PIN_HOPS_LOWP
 #define LYM_PIN_HOPS_LOWP 4
 #endif
-// 1: single-RHS FP64 launches of 256-site blocks stage the other parity's
-// spinors of their site block in LDS (k_dslash_stg); the z and t hops whose
-// neighbour falls inside the block read it from there instead of from L2.
-// Measured: 16^3x32 full apply 3 % faster, even-odd launches 2 %, 32^3x64
-// full apply 5 % (same bits: only where the operands come from changes).
-// Filling the copy with direct global-to-LDS loads instead of through
-// registers, and a second copy filled for the next block while the current
-// one computes, were measured too: the first the same, the second 15 %
-// slower on 16^3x32.
-#ifndef LYM_STAGE_ZT
-#define LYM_STAGE_ZT 1
-#endif
 #ifdef LYM_WAVES_PER_EU
 #define LYM_OCC __attribute__((amdgpu_waves_per_eu(LYM_WAVES_PER_EU, LYM_WAVES_PER_EU)))
 #else
@@ -135,7 +123,8 @@ __device__ __forceinline__ void hop_pair(const DslashParams& a, int p, int site,
     const int iu = eo_index(g, cu[0], cu[1], cu[2], cu[3]);
     const int id = eo_index(g, cd[0], cd[1], cd[2], cd[3]);
     const bool anti = MU == 3 && g.bc_t < 0;
-    const SpinorRef<PR> src{reinterpret_cast<const typename Prec<PR>::S*>(a.in[q]), a.in_sc[q]};
+    const SpinorRef<PR> src{lane_base<PR>(a.in[q], a.in_lane, r), a.in_sc[q]};
+    const int rr = field_rhs<PR>(r);
     constexpr bool SC = PR == 2;
     cplx<T> psi[12];
     T sc;
@@ -144,7 +133,7 @@ __device__ __forceinline__ void hop_pair(const DslashParams& a, int p, int site,
     constexpr bool pin_mid = PH == 1;
     constexpr bool pin_end = PH <= 2 || (PH == 4 && (MU & 1));
     if constexpr (!BWD_FIRST) {
-        load_nb<MU, PR>(src, g.stride, a.nr, iu, r, psi, sc, lds, lbase);
+        load_nb<MU, PR>(src, g.stride, a.nr, iu, rr, psi, sc, lds, lbase);
         load_link<PR, LK>(a.links, g.stride, p, MU, site, L);
         hop_dir<MU, true, LK, T, SC>(acc, psi, L, anti && c[3] == g.L[3] - 1, sc);
         if constexpr (pin_mid) pin(acc);
@@ -153,20 +142,21 @@ __device__ __forceinline__ void hop_pair(const DslashParams& a, int p, int site,
         cplx<T> psi2[12];
         T sc2;
         LinkMat<LK, T> L2;
-        load_nb<MU, PR>(src, g.stride, a.nr, id, r, psi2, sc2, lds, lbase);
+        load_nb<MU, PR>(src, g.stride, a.nr, id, rr, psi2, sc2, lds, lbase);
         load_link<PR, LK>(a.links, g.stride, q, MU, id, L2);
         hop_dir<MU, false, LK, T, SC>(acc, psi2, L2, anti && c[3] == 0, sc2);
     }
     if constexpr (BWD_FIRST) {
         if constexpr (pin_mid) pin(acc);
-        load_nb<MU, PR>(src, g.stride, a.nr, iu, r, psi, sc, lds, lbase);
+        load_nb<MU, PR>(src, g.stride, a.nr, iu, rr, psi, sc, lds, lbase);
         load_link<PR, LK>(a.links, g.stride, p, MU, site, L);
         hop_dir<MU, true, LK, T, SC>(acc, psi, L, anti && c[3] == g.L[3] - 1, sc);
     }
     if constexpr (pin_end) pin(acc);
 }
 
-template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD = false, int BM = 0, int FM = 0>
+template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD = false, int BM = 0, int FM = 0,
+          bool NT = true>
 __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, int site, int r,
                                                   const cplx<typename Prec<PR>::T> acc[12], float ual = 0.f,
                                                   double al = 0.0, double* sums = nullptr);
@@ -177,9 +167,10 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
 // own kappa and clover blocks (a.lane_ops); also a template parameter.  UPD:
 // the fused mixed-CG update with step ual (a.upd_*): returns the site's
 // |r_s|^2 after it, and stores no output.
-// FM: a fused step of the FP64 solvers (F64_*), with step al, its terms added to sums.
+// FM: a fused step of the FP64 solvers (F64_*), with step al, its terms added to
+// sums.  NT: FP64 blocks stream past the caches (no other lane reads them).
 template <int PR, int LK, int DIAG, bool INV, bool NORM = false, bool LO = false, bool UPD = false, int BM = 0,
-          int FM = 0>
+          int FM = 0, bool NT = true>
 __device__ __forceinline__ double dslash_site(const DslashParams& a, int p, int site, int r, float ual = 0.f,
                                               const cplx<double>* lds = nullptr, int lbase = 0, double al = 0.0,
                                               double* sums = nullptr) {
@@ -200,13 +191,13 @@ __device__ __forceinline__ double dslash_site(const DslashParams& a, int p, int 
         hop_pair<2, PR, LK>(a, p, site, r, c, acc, lds, lbase);
         hop_pair<3, PR, LK>(a, p, site, r, c, acc, lds, lbase);
     }
-    return dslash_epilogue<PR, DIAG, INV, NORM, LO, UPD, BM, FM>(a, p, site, r, acc, ual, al, sums);
+    return dslash_epilogue<PR, DIAG, INV, NORM, LO, UPD, BM, FM, NT>(a, p, site, r, acc, ual, al, sums);
 }
 
 // The site's output from its hopping sum acc: v = diag(psi_x) + hop_sign
 // (-kappa acc), then R^-1, gamma5, the axpy and the store (the value
 // returned is as for dslash_site)
-template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD, int BM, int FM>
+template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD, int BM, int FM, bool NT>
 __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, int site, int r,
                                                   const cplx<typename Prec<PR>::T> acc[12], float ual, double al64,
                                                   double* sums) {
@@ -247,12 +238,13 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
         for (int k = 0; k < 12; ++k) v[k] = axpy1(hk, acc[k], t[k]);
     } else {
         cplx<T> s[12];
-        load_spinor<PR>(SpinorRef<PR>{reinterpret_cast<const S*>(a.diag_in[p]), a.diag_sc[p]}, ST, a.nr, site, r, s);
+        load_spinor<PR>(SpinorRef<PR>{lane_base<PR>(a.diag_in[p], a.diag_lane, r), a.diag_sc[p]}, ST, a.nr,
+                        site, field_rhs<PR>(r), s);
         if constexpr (DIAG == 2) {
             cplx<T> t[12];
             const S* Ab = reinterpret_cast<const S*>(Ab_) + (size_t)p * 36 * ST;
-            herm6<PR>(Ab, ST, site, (T)1, s, t);
-            herm6<PR>(Ab + (size_t)18 * ST, ST, site, (T)1, s + 6, t + 6);
+            herm6<PR, NT>(Ab, ST, site, (T)1, s, t);
+            herm6<PR, NT>(Ab + (size_t)18 * ST, ST, site, (T)1, s + 6, t + 6);
 #pragma unroll
             for (int k = 0; k < 12; ++k) v[k] = axpy1(hk, acc[k], t[k]);
         } else {
@@ -264,8 +256,8 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
         cplx<T> t[12];
         if constexpr (PR == 0) {
             const S* Ai = reinterpret_cast<const S*>(Ai_);
-            herm6<PR>(Ai, ST, site, (T)1, v, t);
-            herm6<PR>(Ai + (size_t)18 * ST, ST, site, (T)1, v + 6, t + 6);
+            herm6<PR, NT>(Ai, ST, site, (T)1, v, t);
+            herm6<PR, NT>(Ai + (size_t)18 * ST, ST, site, (T)1, v + 6, t + 6);
         } else {
             const T sc = PR == 2 ? (T)Aisc_[site] : (T)1;
             herm6_packed<PR>(Ai_, 2 * (size_t)ST, 0, site, sc, v, t);
@@ -280,7 +272,8 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
     }
     if (a.v2[p]) {
         cplx<T> w[12];
-        load_spinor<PR, true>(SpinorRef<PR>{reinterpret_cast<const S*>(a.v2[p]), a.v2_sc[p]}, ST, a.nr, site, r, w);
+        load_spinor<PR, true>(SpinorRef<PR>{reinterpret_cast<const S*>(a.v2[p]), a.v2_sc[p]}, ST, a.nr, site,
+                              field_rhs<PR>(r), w);
         const cplx<T> al = mk((T)a.alpha.re, (T)a.alpha.im);
 #pragma unroll
         for (int k = 0; k < 12; ++k) cfma(v[k], al, w[k]);
@@ -332,7 +325,8 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
         for (int k = 0; k < 12; ++k) f64_step<FM>(a, p, k, (unsigned)site, al64, v[k], sums);
         if constexpr (FM == F64_CG) return 0;
     }
-    store_spinor<PR>(SpinorOut<PR>{reinterpret_cast<S*>(a.out[p]), a.out_sc[p]}, ST, a.nr, site, r, v);
+    store_spinor<PR>(SpinorOut<PR>{const_cast<S*>(lane_base<PR>(a.out[p], a.out_lane, r)), a.out_sc[p]}, ST,
+                     a.nr, site, field_rhs<PR>(r), v);
     if constexpr (BM == 1) {  // lane r's |v|^2 at this site: the 24 squares in FP32
         float n2[2] = {0.f, 0.f};
 #pragma unroll
@@ -439,29 +433,37 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash(DslashPar
     }
 }
 
-#if LYM_STAGE_ZT
-// FP64, one RHS, one thread per site (spb == LYM_DSLASH_THREADS): each site
+// FP64, one thread per site (spb == LYM_DSLASH_THREADS): each site
 // block first copies the other parity's spinors of the same block index --
 // with t fastest, the z and t neighbours of most of the block's sites -- into
 // LDS, coalesced, once; those hops then read LDS instead of issuing four
-// reads of every such spinor to L2.
+// reads of every such spinor to L2.  Measured against reading them from L2:
+// 16^3x32 full apply 3 % faster, even-odd launches 2 %, 32^3x64 full apply 5 %
+// (same bits: only where the operands come from changes).  Filling the copy with
+// direct global-to-LDS loads instead of through registers, and a second copy
+// filled for the next block while the current one computes, were measured too:
+// the first the same, the second 15 % slower on 16^3x32.
 // FM: a fused step of the FP64 solvers; its terms' per-workgroup sums go to
-// a.upd_rpart.
-template <int LK, int DIAG, bool INV, int FM = 0>
+// a.upd_rpart.  LN: over lanes; LO: per-lane operators.
+template <int LK, int DIAG, bool INV, int FM = 0, bool LN = false, bool LO = false>
 __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash_stg(DslashParams a) {
     __shared__ cplx<double> stg[12 * LYM_DSLASH_THREADS];
     if (a.skip && *a.skip) return;
-    const BlockSweep b = block_sweep(a);
+    int bx = (int)blockIdx.x, gd = (int)gridDim.x, lane = 0;
+    if constexpr (LN) {
+        if (!lane_of_block(a, bx, gd, lane)) return;
+    }
+    const BlockSweep b = block_sweep_at(a, bx, gd);
     const int t = (int)threadIdx.x;
     double al = 0, sums[3] = {0, 0, 0};
     if constexpr (FM == F64_CG) al = upd_alpha<CGState>(a);
     for (int lb = b.lo + b.k; lb < b.hi; lb += b.nphys) {
         int p, bi;
-        block_of(a, b, lb, p, bi);
+        (void)block_of_at(a, b, lb, bx, p, bi);
         const int base = bi * LYM_DSLASH_THREADS;
         __syncthreads();  // the previous block's reads of stg are done
         if (base + t < a.g.Vh) {
-            const zd* src = reinterpret_cast<const zd*>(a.in[p ^ a.g.tsh]);
+            const zd* src = lane_base<0>(a.in[p ^ a.g.tsh], a.in_lane, LN ? lane : 0);
 #pragma unroll
             for (int k = 0; k < 12; ++k)
                 stg[k * LYM_DSLASH_THREADS + t] = fld<zd>(src + (size_t)k * a.g.stride, (unsigned)(base + t));
@@ -469,13 +471,12 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash_stg(Dslas
         __syncthreads();
         const int site = base + t;
         if (site < a.g.Vh)
-            dslash_site<0, LK, DIAG, INV, false, false, false, 0, FM>(a, p, site, 0, 0.f, stg, base, al, sums);
+            dslash_site<0, LK, DIAG, INV, false, LO, false, 0, FM, !LN>(a, p, site, LN ? lane : 0, 0.f, stg, base, al,
+                                                                      sums);
     }
     if constexpr (FM == F64_DOT) block_sums_store<3>(sums, a.upd_rpart, a.part_stride);
     else if constexpr (FM != F64_STORE) block_sums_store<1>(sums, a.upd_rpart, 0);
 }
-
-#endif
 
 // ---------------------------------------------------------------- two threads per site (FP32/FP16)
 // Split form of the single-RHS low-precision stencil: a workgroup holds its
@@ -895,8 +896,40 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) void k_dslash_mfma(DslashParams
     }
 }
 
+template <int LK, int DIAG, bool INV>
+static void launch_f64(const DslashParams& a, int nblocks, hipStream_t st) {
+    const dim3 g(lane_grid(a, nblocks)), th(LYM_DSLASH_THREADS);
+    if (a.lane_ops) {
+        hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_STORE, true, true>), g, th, 0, st, a);
+        return;
+    }
+    if (a.lanes > 1 || a.lane_flags) {
+        hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_STORE, true>), g, th, 0, st, a);
+        return;
+    }
+    if constexpr (DIAG >= 1 && !INV) {
+        switch (a.fmode) {
+            case F64_NORM: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_NORM>), g, th, 0, st, a); return;
+            case F64_CG: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_CG>), g, th, 0, st, a); return;
+            case F64_DOT: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_DOT>), g, th, 0, st, a); return;
+            default: break;
+        }
+    }
+    hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV>), g, th, 0, st, a);
+}
+
+template <int PR, int LK, int DIAG, bool INV>
+static void launch_lp(const DslashParams& a, int nblocks, hipStream_t st);
 template <int PR, int LK, int DIAG, bool INV>
 static void launch_one(const DslashParams& a, int nblocks, hipStream_t st) {
+    if constexpr (PR == 0) {
+        launch_f64<LK, DIAG, INV>(a, nblocks, st);
+    } else {
+        launch_lp<PR, LK, DIAG, INV>(a, nblocks, st);
+    }
+}
+template <int PR, int LK, int DIAG, bool INV>
+static void launch_lp(const DslashParams& a, int nblocks, hipStream_t st) {
     if constexpr (PR == 2 && LK == 0) {
         // matrix-core form: FP16 SU(3) batches of 2, 4 or 8 RHS in whole waves
         if (a.mfma && !a.bmode && (a.nr == 2 || a.nr == 4 || a.nr == 8) && (a.spb * a.nr) % 64 == 0) {
@@ -965,23 +998,6 @@ static void launch_one(const DslashParams& a, int nblocks, hipStream_t st) {
             return;
         }
     }
-#if LYM_STAGE_ZT
-    if constexpr (PR == 0) {
-        if (a.nr == 1 && a.spb == LYM_DSLASH_THREADS && !a.lane_flags) {
-            if constexpr (DIAG >= 1 && !INV) {
-                const dim3 g(nblocks), th(LYM_DSLASH_THREADS);
-                switch (a.fmode) {
-                    case F64_NORM: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_NORM>), g, th, 0, st, a); return;
-                    case F64_CG: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_CG>), g, th, 0, st, a); return;
-                    case F64_DOT: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_DOT>), g, th, 0, st, a); return;
-                    default: break;
-                }
-            }
-            hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV>), dim3(nblocks), dim3(LYM_DSLASH_THREADS), 0, st, a);
-            return;
-        }
-    }
-#endif
     hipLaunchKernelGGL((k_dslash<PR, LK, DIAG, INV>), dim3(nblocks), dim3(a.spb * a.nr), 0, st, a);
 }
 
@@ -1065,8 +1081,10 @@ static int plan_hop(DslashParams& a) {
 int launch_dslash(DslashParams a, int link_kind, int diag, bool inv, hipStream_t st) {
     const int threads = (a.threads > 0 && a.threads <= LYM_DSLASH_THREADS) ? a.threads : LYM_DSLASH_THREADS;
     if (a.nr < 1) a.nr = 1;
+    if (a.prec == 0) a.threads = 0;
     const int hop_blocks = plan_hop(a);
     const int nblocks = hop_blocks ? hop_blocks : plan_dslash(a);
+    a.grid1 = nblocks;
     // output norm partials: low precision only, one per workgroup, and only
     // when the caller's buffer holds one per workgroup of this launch
     // (the workgroup sum shuffles over whole 64-lane waves)
@@ -1080,8 +1098,7 @@ int launch_dslash(DslashParams a, int link_kind, int diag, bool inv, hipStream_t
         if (!a.fmode) a.upd_state = nullptr;
     // the FP64 solvers' fused steps: one RHS, a diagonal and no R^-1, and room for
     // one partial per workgroup
-    if (a.prec != 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || a.lane_ops || a.threads ||
-        nblocks > a.part_stride || !LYM_STAGE_ZT)
+    if (a.prec != 0 || diag == 0 || inv || a.lanes > 1 || a.lane_flags || a.lane_ops || nblocks > a.part_stride)
         a.fmode = F64_STORE;
     const bool fused = a.norm_partials || a.upd_state || a.fmode;
     if (hop_blocks) {

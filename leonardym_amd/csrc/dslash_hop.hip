@@ -59,8 +59,8 @@ __device__ __forceinline__ typename Prec<PR>::T one_hop(const DslashParams& a, i
     cplx<T> psi[12];
     T sc;
     LinkMat<LK, T> L;
-    load_spinor_unscaled<PR>(SpinorRef<PR>{reinterpret_cast<const typename Prec<PR>::S*>(a.in[q]), a.in_sc[q]},
-                             g.stride, a.nr, in, r, psi, sc);
+    load_spinor_unscaled<PR>(SpinorRef<PR>{lane_base<PR>(a.in[q], a.in_lane, r), a.in_sc[q]}, g.stride,
+                             a.nr, in, field_rhs<PR>(r), psi, sc);
     load_link<PR, LK>(a.links, g.stride, FWD ? p : q, MU, FWD ? site : in, L);
     hop_mul<MU, FWD, LK, T, PR == 2>(psi, L, o, o + 3);
     const bool flip = MU == 3 && g.bc_t < 0 && c[3] == (FWD ? g.L[3] - 1 : 0);
@@ -231,18 +231,21 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
     if (a.skip && *a.skip) return;
     const int lane = (int)threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    int p, bi;
-    {
-        const int lb = xcd_block((int)blockIdx.x, (int)gridDim.x);
-        p = a.parity >= 0 ? a.parity : lb & 1;
-        bi = a.parity >= 0 ? lb : lb >> 1;
+    int bx = (int)blockIdx.x, gd = (int)gridDim.x, ls, r;
+    if constexpr (PR == 0) {
+        if (!lane_of_block(a, bx, gd, r)) return;
+        ls = lane;
+    } else {
+        ls = lane / a.nr;
+        r = lane - ls * a.nr;
     }
-    const int ls = lane / a.nr, r = lane - ls * a.nr;
+    const int lb = xcd_block(bx, gd);
+    const int p = a.parity >= 0 ? a.parity : lb & 1, bi = a.parity >= 0 ? lb : lb >> 1;
     const int site = bi * a.spb + ls;
-    const bool ok = ls < a.spb && site < a.g.Vh && !(a.lane_flags && a.lane_flags[r] == a.lane_skip_value);
+    const bool ok = ls < a.spb && site < a.g.Vh && (PR == 0 || !(a.lane_flags && a.lane_flags[r] == a.lane_skip_value));
     const int ST = a.g.stride;
     const size_t ks = (size_t)ST * a.nr;
-    const unsigned o = (unsigned)site * (unsigned)a.nr + (unsigned)r;
+    const unsigned o = (unsigned)site * (unsigned)a.nr + (unsigned)field_rhs<PR>(r);
 
     [[maybe_unused]] UpdPair<PR> up;
     if constexpr (UPDATE) {
@@ -344,7 +347,7 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
         if constexpr (DIAG == 2) {
             cplx<T> blk[18], t[6];
             T sc = (T)1;
-            load_half<PR>(a.diag_in[p], ks, o, h, t);
+            load_half<PR>(lane_base<PR>(a.diag_in[p], a.diag_lane, r), ks, o, h, t);
             load_block<PR>(Ab, 2, ST, p, h, site, blk);
             if constexpr (PR == 2) sc = Asc[(size_t)p * ST + site] * fld<float>(a.diag_sc[p], o);
             herm6_mul<T>(blk, t, s);
@@ -353,7 +356,7 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
                 for (int k = 0; k < 6; ++k) s[k] = sc * s[k];
             }
         } else if constexpr (DIAG == 1) {
-            load_half<PR>(a.diag_in[p], ks, o, h, s);
+            load_half<PR>(lane_base<PR>(a.diag_in[p], a.diag_lane, r), ks, o, h, s);
             if constexpr (PR == 2) {
                 const T sc = fld<float>(a.diag_sc[p], o);
 #pragma unroll
@@ -497,7 +500,7 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
         }
         if (ok) {
             if constexpr (PR == 0) {
-                zd* b = reinterpret_cast<zd*>(a.out[p]) + (size_t)(6 * h) * ks;
+                zd* b = const_cast<zd*>(lane_base<0>(a.out[p], a.out_lane, r)) + (size_t)(6 * h) * ks;
 #pragma unroll
                 for (int k = 0; k < 6; ++k) fst(b + k * ks, o, e[k]);
             } else {
@@ -549,12 +552,13 @@ template <int PR, int LK, int DIAG, bool INV, int MODE = HOP_STORE>
 static void hop_go(const DslashParams& a, int nblocks, hipStream_t st) {
     if constexpr (MODE != HOP_NORM && MODE != HOP_UPD) {
         if (a.lane_ops) {
-            hipLaunchKernelGGL((k_dslash_hop<PR, LK, DIAG, INV, MODE, true>), dim3(nblocks), dim3(HOP_THREADS), 0, st,
-                               a);
+            hipLaunchKernelGGL((k_dslash_hop<PR, LK, DIAG, INV, MODE, true>),
+                               dim3(PR == 0 ? lane_grid(a, nblocks) : nblocks), dim3(HOP_THREADS), 0, st, a);
             return;
         }
     }
-    hipLaunchKernelGGL((k_dslash_hop<PR, LK, DIAG, INV, MODE, false>), dim3(nblocks), dim3(HOP_THREADS), 0, st, a);
+    hipLaunchKernelGGL((k_dslash_hop<PR, LK, DIAG, INV, MODE, false>), dim3(PR == 0 ? lane_grid(a, nblocks) : nblocks),
+                       dim3(HOP_THREADS), 0, st, a);
 }
 
 // the FP64 solvers' fused steps

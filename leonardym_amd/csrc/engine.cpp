@@ -6,11 +6,12 @@
 // the stencil reads them through per-lane strides (DslashParams::lane_ops).
 // The links and the kappa-independent blocks B are the lattice's, shared.
 //
-// Fields are multi-RHS nr-fields (batch.hip) of the current width w, lane
-// fastest, stored in buffers sized for wmax lanes.  Growing the batch
-// relayouts the fields that carry a lane's state from one iteration to the
-// next (sources, right-hand side, x, r, x_s, r_s, p) to the new width; a lane
-// keeps its index, so its operator data never moves.
+// The FP64 fields (sources, right-hand side, x, r and scratch) hold each lane as a
+// field of its own; the low-precision ones interleave the lanes of the current
+// width w, lane fastest, in buffers sized for wmax lanes.  Growing the batch
+// relayouts those that carry a lane's state from one iteration to the next (x_s,
+// r_s, p) to the new width; a lane keeps its index, so its operator data and its
+// FP64 fields never move.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -74,7 +75,7 @@ struct LaneEngine {
     zd *A = nullptr, *Ainv = nullptr;
     void *As = nullptr, *Ainvs = nullptr, *Us = nullptr;
     float *As_sc = nullptr, *Ainvs_sc = nullptr;
-    // nr-fields (FP64: B full, X full, the rest odd halves)
+    // FP64 lane fields (B and X full, the rest odd or even halves)
     zd *B = nullptr, *X = nullptr, *x = nullptr, *r = nullptr, *Ax = nullptr, *mid = nullptr, *tmp = nullptr,
        *rhs = nullptr, *src = nullptr, *te = nullptr;
     void* sv[4] = {};  // sloppy p, Ap, Q^2 intermediate, even Schur intermediate
@@ -157,6 +158,11 @@ lym::DslashParams base(LaneEngine* e, int prec) {
     std::memset(&a, 0, sizeof(a));
     a.g = e->ctx->g;
     a.nr = e->width;
+    if (prec == 0) {  // lane fields, by default odd or even halves
+        a.nr = 1;
+        a.lanes = e->width;
+        a.in_lane = a.diag_lane = a.out_lane = 12 * e->S;
+    }
     a.hop_sign = 1.0;
     lane_ops(e, a, prec);
     return a;
@@ -249,8 +255,8 @@ int write_state(LaneEngine* e) {
     return LYM_OK;
 }
 
-// Relayout of every field that carries lane state from width e->width to w
-// (X, a scratch field of wmax lanes, holds each new layout before it is copied back).
+// Relayout of every interleaved field that carries lane state from width e->width
+// to w (the FP64 fields hold each lane apart; X, a scratch field of wmax lanes, holds each new layout before it is copied back).
 int set_width(LaneEngine* e, int w) {
     const int w0 = e->width;
     if (w == w0) return LYM_OK;
@@ -262,7 +268,6 @@ int set_width(LaneEngine* e, int w) {
         int esize;
         long rows;
     } fields[] = {
-        {e->B, 16, 24 * S},  {e->rhs, 16, 12 * S}, {e->x, 16, 12 * S},  {e->r, 16, 12 * S},
         {e->xs, 8, 12 * S},  {e->rs, 8, 12 * S},   {e->sv[0], 16, G * S}, {e->svsc[0], 4, S},
     };
     for (const F& f : fields) {
@@ -281,10 +286,7 @@ int set_width(LaneEngine* e, int w) {
     e->width = w;
     // padding slots of the new layout to zero (no launch writes them)
     const int vh = e->ctx->g.Vh;
-    zd* full[] = {e->B, e->X};
-    zd* half[] = {e->x, e->r, e->Ax, e->mid, e->tmp, e->rhs, e->src, e->te};
-    for (zd* f : full) lym::launch_zero_padding(16, f, 24, (int)S, vh, w, st);
-    for (zd* f : half) lym::launch_zero_padding(16, f, 12, (int)S, vh, w, st);
+    if (w0 > 0) lym::launch_zero_padding(16, e->X, 24L * e->wcap, (int)S, vh, 1, st);  // (it was the scratch)
     for (int i = 0; i < 4; ++i) {
         lym::launch_zero_padding(16, e->sv[i], G, (int)S, vh, w, st);
         lym::launch_zero_padding(4, e->svsc[i], 1, (int)S, vh, w, st);
@@ -592,27 +594,26 @@ int engine_admit(LaneEngine* e, int n, const LaneRequest* reqs, std::vector<Lane
     // pack the admitted sources into their lanes of B
     for (int q = 0; q < w; ++q) e->ptr_h[q] = e->mask_h[q] ? reinterpret_cast<zd*>(e->lsrc[q]->d) : nullptr;
     ECHECK(hipMemcpyAsync(e->ptr_d, e->ptr_h, sizeof(zd*) * w, hipMemcpyHostToDevice, st));
-    lym::launch_pack(e->ptr_d, w, e->B, 24 * S, st);
+    lym::launch_lane_gather(e->ptr_d, e->B, 24 * S, w, st);
     // the even-odd driver's right-hand side (PreconditionedBiCGStab.cpp:56-70):
     // src_o = b_o - D_oe R_ee^-1 b_e, rhs = Qhat gamma5 src_o
-    const zd* b_e = e->B;
-    const zd* b_o = e->B + 12 * S * w;
-    lym::launch_clover_apply_lanes(c->g, e->Ainv, 36 * S, e->lset_d, e->mask_d, b_e, e->te, w, st);
+    lym::launch_clover_apply_lanes(c->g, e->Ainv, 36 * S, e->lset_d, e->mask_d, e->B, 24 * S, e->te, 12 * S, w, st);
     lym::DslashParams a = base(e, 0);
     a.hop_sign = -1.0;
     a.parity = 1;
     a.in[0] = e->te;
-    a.diag_in[1] = b_o;
+    a.diag_in[1] = e->B + 12 * S;
+    a.diag_lane = 24 * S;
     a.out[1] = e->src;
     a.lane_flags = e->mask_d;
     a.lane_skip_value = 0;
     lym::launch_dslash(a, e->lk64, 1, false, st);
-    lym::launch_scale_g5(e->src, 1, (int)(S * w), st);  // lanes outside the mask hold nothing in use
+    lym::launch_scale_g5(e->src, w, (int)S, st);  // lanes outside the mask hold nothing in use
     schur(e, 0, e->rhs, nullptr, e->src, nullptr, e->tmp, nullptr, nullptr, e->mask_d, 0);
     // FP64 start: x = rhs, r = rhs - Qhat^2 x, then the lanes' CG state
-    lym::launch_lane_copy(16, e->x, e->rhs, 12 * S, w, e->mask_d, st);
+    lym::launch_lane_copy(e->x, 12 * S, e->rhs, 12 * S, 12 * S, w, e->mask_d, st);
     schur2(e, 0, e->Ax, nullptr, e->x, nullptr, nullptr, e->mask_d, 0);
-    lym::launch_lane_sub(e->r, e->rhs, e->Ax, 12 * S, w, e->mask_d, st);
+    lym::launch_lane_sub(e->r, e->rhs, e->Ax, 12 * S, 12 * S, w, e->mask_d, st);
     lym::BcgArgs ba = bcg_args(e, e->mask_d);
     if (!lym::launch_bcg_step(0, e->prec, w, e->Sd, ba, st)) return fail(LYM_ERR_UNSUPPORTED, "width %d", w);
     ECHECK(hipGetLastError());
@@ -673,21 +674,20 @@ int engine_harvest(LaneEngine* e, std::vector<LaneResult>* done) {
     lym::BcgArgs ba = bcg_args(e, e->mask_d);
     lym::launch_bcg_step(6, e->prec, w, e->Sd, ba, st);
     // x_o, and x_e = R_ee^-1 (b_e - D_eo x_o) (PreconditionedBiCGStab.cpp:80-86)
-    zd* X_e = e->X;
-    zd* X_o = e->X + 12 * S * w;
-    lym::launch_lane_copy(16, X_o, e->x, 12 * S, w, e->mask_d, st);
+    lym::launch_lane_copy(e->X + 12 * S, 24 * S, e->x, 12 * S, 12 * S, w, e->mask_d, st);
     lym::DslashParams a = base(e, 0);
+    a.in_lane = a.diag_lane = a.out_lane = 24 * S;
     a.hop_sign = -1.0;
     a.parity = 0;
-    a.in[1] = X_o;
+    a.in[1] = e->X + 12 * S;
     a.diag_in[0] = e->B;
-    a.out[0] = X_e;
+    a.out[0] = e->X;
     a.lane_flags = e->mask_d;
     a.lane_skip_value = 0;
     lym::launch_dslash(a, e->lk64, 1, true, st);
     for (int q = 0; q < w; ++q) e->ptr_h[q] = e->mask_h[q] ? reinterpret_cast<zd*>(e->lsol[q]->d) : nullptr;
     ECHECK(hipMemcpyAsync(e->ptr_d, e->ptr_h, sizeof(zd*) * w, hipMemcpyHostToDevice, st));
-    lym::launch_unpack(e->X, w, e->ptr_d, 24 * S, st);
+    lym::launch_lane_scatter(e->X, e->ptr_d, 24 * S, w, st);
     ECHECK(hipGetLastError());
     int hi = 0;
     for (int q = 0; q < w; ++q) {

@@ -562,7 +562,7 @@ __device__ __forceinline__ void load_spinor(const cplx<double>* f, int stride, i
 // ---------------------------------------------------------------- clover blocks
 // o = A v for one packed hermitian 6x6 block; A points at the block's first
 // component of the parity, sc is the per-site scale (PR == 2) or 1.
-template <int PR>
+template <int PR, bool NT = true>
 __device__ __forceinline__ void herm6(const typename Prec<PR>::S* A, int stride, int idx,
                                       typename Prec<PR>::T sc, const cplx<typename Prec<PR>::T> v[6],
                                       cplx<typename Prec<PR>::T> o[6]) {
@@ -570,7 +570,7 @@ __device__ __forceinline__ void herm6(const typename Prec<PR>::S* A, int stride,
     T d[6];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        cplx<T> dd = to_c<PR>(fld<typename Prec<PR>::S, true>(A + (size_t)k * stride, (unsigned)idx));
+        cplx<T> dd = to_c<PR>(fld<typename Prec<PR>::S, NT>(A + (size_t)k * stride, (unsigned)idx));
         d[2 * k] = sc * dd.re;
         d[2 * k + 1] = sc * dd.im;
     }
@@ -581,7 +581,7 @@ __device__ __forceinline__ void herm6(const typename Prec<PR>::S* A, int stride,
     for (int i = 1; i < 6; ++i) {
 #pragma unroll
         for (int j = 0; j < i; ++j) {
-            cplx<T> a = sc * to_c<PR>(fld<typename Prec<PR>::S, true>(A + (size_t)k * stride, (unsigned)idx));
+            cplx<T> a = sc * to_c<PR>(fld<typename Prec<PR>::S, NT>(A + (size_t)k * stride, (unsigned)idx));
             cfma(o[i], a, v[j]);
             cfmac(o[j], a, v[i]);
             ++k;

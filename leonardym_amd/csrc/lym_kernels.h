@@ -16,7 +16,7 @@ enum { F64_STORE = 0, F64_NORM = 1, F64_CG = 2, F64_DOT = 3 };
 struct DslashParams {
     Geom g;
     int prec;              // storage precision of spinors, links and clover blocks
-    int nr;                // right-hand sides per field
+    int nr;                // FP32/FP16: right-hand sides per field, interleaved (rhs fastest)
     int spb;               // sites per workgroup (set by the launcher)
     const void* in[2];     // per parity: the field read at neighbours is in[1 - p]
     const float* in_sc[2];
@@ -39,7 +39,7 @@ struct DslashParams {
     int parity;            // 0 or 1: that parity only; -1: both
     int nblocks_per_parity;
     const int* skip;       // optional device flag: nonzero -> the launch does nothing (solver done)
-    const int* lane_flags; // optional per-RHS device flags: lane r does nothing when
+    const int* lane_flags; // optional per-RHS (FP64: per-lane) device flags: lane r does nothing when
     int lane_skip_value;   //   lane_flags[r] == lane_skip_value (an RHS that is done or needs no update)
     int threads;           // workgroup size (0: LYM_DSLASH_THREADS); a workgroup holds threads / nr sites
     int xslice_blocks;     // set by the launcher: site blocks per x-slice and parity when an x-slice
@@ -90,6 +90,12 @@ struct DslashParams {
     int fmode;
     const void* dotw[2];
     int part_stride;
+    // FP64: right-hand sides as fields of their own ("lanes"), lane l of a field at
+    // pointer + l * stride below (in complex elements); 0 or 1: one field.  The
+    // workgroups of the lanes of a site block follow one another on one XCD.
+    int lanes;
+    long in_lane, diag_lane, out_lane;
+    int grid1;             // set by the launcher: workgroups of one lane
 };
 // The arguments of such a step for vectors of one parity (an odd half) or two
 struct Fuse64 {
@@ -276,7 +282,7 @@ struct BcgArgs {
     float* p_sc;
     void* Ap;
     float* Ap_sc;
-    long nsites;
+    long nsites;  // x, r, b, Ax: FP64 lane fields of 12 * nsites elements per lane
     int stride;
     int max_steps;
     double* partials;  // BMAX * ceil(nsites / BATCH_CHUNK) doubles
@@ -298,26 +304,29 @@ struct BFuse {
 // 7 alpha and 8 the update's sums from the per-(site, RHS) values at bsite (a stencil's bmode 1 / 2)
 bool launch_bcg_step(int which, int prec, int nr, BState* s, const BcgArgs& a, hipStream_t st);
 bool batch_nr_supported(int nr);
+// FP64 lane fields: lane l of a field at l * its lane stride (elements), n
+// elements per lane; lanes with mask[l] == 0 (mask may be null) are left alone.
+// copy and difference; from and to single fields (a null pointer leaves its lane alone)
+void launch_lane_copy(zd* dst, long dst_lane, const zd* src, long src_lane, long n, int lanes, const int* mask,
+                      hipStream_t st);
+void launch_lane_sub(zd* out, const zd* a, const zd* b, long lane, long n, int lanes, const int* mask, hipStream_t st);
+void launch_lane_gather(const zd* const* srcs_dev, zd* dst, long n, int lanes, hipStream_t st);
+void launch_lane_scatter(const zd* src, zd* const* dsts_dev, long n, int lanes, hipStream_t st);
+// blocks (lane_set null: set 0 for every lane; else set lane_set[l] at stride
+// set_elems) applied to the even half of lane fields
+void launch_clover_apply_lanes(const Geom& g, const zd* blocks, long set_elems, const int* lane_set, const int* mask,
+                               const zd* in, long in_lane, zd* out, long out_lane, int lanes, hipStream_t st);
+// single full fields <-> an interleaved FP64 field (rhs fastest)
 void launch_pack(const zd* const* srcs_dev, int nr, zd* multi, long n, hipStream_t st);
 void launch_unpack(const zd* multi, int nr, zd* const* dsts_dev, long n, hipStream_t st);
-// lanes of nr-fields (rows x nr elements of esize bytes, lane fastest): copy or
-// subtract on the lanes with mask[q] != 0; relayout to another width (a lane
-// keeps its index; new lanes are zero)
-void launch_lane_copy(int esize, void* dst, const void* src, long rows, int nr, const int* mask, hipStream_t st);
-void launch_lane_sub(zd* out, const zd* a, const zd* b, long rows, int nr, const int* mask, hipStream_t st);
+// an interleaved field (rows x nr elements of esize bytes, lane fastest) to
+// another width (a lane keeps its index; new lanes are zero)
 void launch_relayout(int esize, const void* in, void* out, long rows, int w_old, int w_new, hipStream_t st);
 // zero the padding slots (sites vh..stride-1) of an nr-field of `groups` groups
 // of stride * nr elements of esize (16, 8 or 4) bytes.  No launch writes them,
 // and a buffer reused at another width would otherwise hold, there, values of
 // real sites of the old layout, which per-RHS sums and copies read.
 void launch_zero_padding(int esize, void* buf, long groups, int stride, int vh, int nr, hipStream_t st);
-void launch_clover_apply_nr(const Geom& g, const zd* blocks, const zd* in, zd* out, int nr, hipStream_t st);
-// the same with lane r's blocks at blocks + r * lane_elems, only for lanes with mask[r] != 0
-// lane r applies block set lane_set[r] (lane_set NULL: set r)
-void launch_clover_apply_lanes(const Geom& g, const zd* blocks, long lane_elems, const int* lane_set, const int* mask,
-                               const zd* in,
-                               zd* out, int nr, hipStream_t st);
-
 // x = uniform [0,1) complex on real sites, zero on padding (BiCGStab start for a zero source)
 void launch_fill_uniform(zd* x, int nparity, int stride, int Vh, uint64_t seed, hipStream_t st);
 }  // namespace lym

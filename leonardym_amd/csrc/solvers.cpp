@@ -69,8 +69,8 @@ int apply_schur_nr(lym_op* op, int prec, int nr, int threads, void* out_o, float
                    const int* lane_flags = nullptr, int lane_skip_value = 0, bool batch_links = false,
                    double* norm_partials = nullptr, int norm_max = 0, int mfma = 0,
                    const lym::UpdArgs* upd = nullptr, const lym::BFuse* bf = nullptr);
-void eo_source_nr(lym_op* op, int nr, const zd* b_e, const zd* b_o, zd* te, zd* src_o);
-void eo_reconstruct_nr(lym_op* op, int nr, const zd* b_e, const zd* x_o, zd* x_e);
+void eo_source_nr(lym_op* op, int nr, const zd* b, zd* te, zd* src_o);
+void eo_reconstruct_nr(lym_op* op, int nr, const zd* b, zd* X);
 }  // namespace lym_internal
 
 using lym_internal::fail;
@@ -121,7 +121,7 @@ struct lym_solver {
     void* bhost;
     zd** bptr_dev;
     zd** bptr_host;
-    zd* bzero;              // zero source / dummy destination for padded lanes
+    zd* bzero;              // zero source of padded lanes
     // plain BiCGStab on A + shift (the reference's shifted overload)
     double shift_re, shift_im;
     // captured iteration chunks (see queue_iterations), with the id of the
@@ -674,7 +674,7 @@ int ensure_batch(lym_solver* s, int nr, int dom, int prec) {
     }
     if (s->bnr >= nr && s->bdom >= dom && s->bprec == prec) return LYM_OK;
     const size_t S = c->g.stride;
-    // one component of a batched field is read through 32-bit buffer offsets
+    // one component of an interleaved field is read through 32-bit buffer offsets
     if (S * (size_t)nr * sizeof(zd) >= (size_t(1) << 31))
         return fail(LYM_ERR_INVALID, "%d right-hand sides per batch exceed the 2 GiB component stream on this lattice", nr);
     free_batch(s);
@@ -869,11 +869,10 @@ int run_batch(lym_solver* s, lym_op* op, bool eo, bool half, int nr, int thr, in
     const long nfull = 24 * S * nr, ndom = 12 * S * dom * nr;
     zd *B = s->bw[0], *X = s->bw[1], *x = s->bw[2], *r = s->bw[3], *Ax = s->bw[4], *mid = s->bw[5],
        *tmp = s->bw[6], *rhs = s->bw[7], *src = s->bw[8], *te = s->bw[9];
-    // padding slots of this width's layout to zero (the buffers may have held
-    // another width; lattices whose parity fills its stride have none)
+    // padding slots of this width's layout to zero (the interleaved buffers may have
+    // held another width; lattices whose parity fills its stride have none)
     {
         const int vh = c->g.Vh, G = prec == 1 ? 6 : 3;
-        for (int i = 0; i < 10; ++i) lym::launch_zero_padding(16, s->bw[i], i < 2 ? 24 : 12 * dom, (int)S, vh, nr, st);
         for (int i = 0; i < 4; ++i) {
             lym::launch_zero_padding(16, s->bsv[i], G * dom, (int)S, vh, nr, st);
             lym::launch_zero_padding(4, s->bsvsc[i], dom, (int)S, vh, nr, st);
@@ -885,17 +884,16 @@ int run_batch(lym_solver* s, lym_op* op, bool eo, bool half, int nr, int thr, in
     // pack sources
     for (int q = 0; q < nr; ++q) s->bptr_host[q] = q < nb ? reinterpret_cast<zd*>(sources[q]->d) : s->bzero;
     HIPCHECK(hipMemcpyAsync(s->bptr_dev, s->bptr_host, sizeof(zd*) * nr, hipMemcpyHostToDevice, st));
-    lym::launch_pack(s->bptr_dev, nr, B, full_n(c), st);
-    const zd* b;
+    lym::launch_lane_gather(s->bptr_dev, B, full_n(c), nr, st);
+    const zd* b = B;
     if (eo) {
-        const zd* b_e = B;
-        const zd* b_o = B + 12 * S * nr;
-        lym_internal::eo_source_nr(op, nr, b_e, b_o, te, src);
-        lym::launch_scale_g5(src, 1, (int)(S * nr), st);
+        lym_internal::eo_source_nr(op, nr, B, te, src);
+        lym::launch_scale_g5(src, nr, (int)S, st);
         lym_internal::apply_schur_nr(op, 0, nr, thr, rhs, nullptr, src, nullptr, tmp, nullptr, 1, nullptr);
         b = rhs;
-    } else {
-        b = half ? B + 12 * S * nr : B;
+    } else if (half) {
+        lym::launch_lane_copy(rhs, half_n(c), B + half_n(c), full_n(c), half_n(c), nr, nullptr, st);
+        b = rhs;
     }
     // the EO driver solves Qhat^2 with gamma5 = 1; otherwise the operator as configured
     const int g5 = eo ? 1 : op->gamma5;
@@ -982,21 +980,18 @@ int run_batch(lym_solver* s, lym_op* op, bool eo, bool half, int nr, int thr, in
     }
     lym::launch_bcg_step(6, prec, nr, Sdev, a, st);
     // solutions
-    if (eo) {
-        lym::launch_copy(X + 12 * S * nr, x, 12 * S * nr, st);
-        lym_internal::eo_reconstruct_nr(op, nr, B, X + 12 * S * nr, X);
-    } else if (half) {
-        lym::launch_copy(X, B, 12 * S * nr, st);
-        lym::launch_copy(X + 12 * S * nr, x, 12 * S * nr, st);
+    if (dom == 1) {
+        lym::launch_lane_copy(X + half_n(c), full_n(c), x, half_n(c), half_n(c), nr, nullptr, st);
+        if (eo) lym_internal::eo_reconstruct_nr(op, nr, B, X);
+        else lym::launch_lane_copy(X, full_n(c), B, full_n(c), half_n(c), nr, nullptr, st);
     } else {
         lym::launch_copy(X, x, nfull, st);
     }
-    for (int q = 0; q < nr; ++q) s->bptr_host[q] = q < nb ? reinterpret_cast<zd*>(solutions[q]->d) : s->bzero;
+    for (int q = 0; q < nr; ++q) s->bptr_host[q] = q < nb ? reinterpret_cast<zd*>(solutions[q]->d) : nullptr;
     HIPCHECK(hipMemcpyAsync(s->bptr_dev, s->bptr_host, sizeof(zd*) * nr, hipMemcpyHostToDevice, st));
-    lym::launch_unpack(X, nr, s->bptr_dev, full_n(c), st);
+    lym::launch_lane_scatter(X, s->bptr_dev, full_n(c), nr, st);
     HIPCHECK(hipMemcpyAsync(Sh, Sdev, sizeof(lym::BState), hipMemcpyDeviceToHost, st));
     HIPCHECK(hipStreamSynchronize(st));
-    HIPCHECK(hipMemsetAsync(s->bzero, 0, sizeof(zd) * full_n(c), st));
     for (int q = 0; q < nb; ++q) {
         lym_solve_info& f = infos[q];
         f.converged = Sh->conv[q];
