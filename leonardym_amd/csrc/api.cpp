@@ -101,30 +101,33 @@ int op_prepare(lym_op* op, bool force_blocks) {
     bool need_blocks = force_blocks || op_has_clover(op) || op->kind == LYM_OP_EO_CLOVER;
     if (!need_blocks || (!op->diag_dirty && op->A)) return LYM_OK;
     lym_gauge* g = const_cast<lym_gauge*>(op->gauge);
-    const size_t blk = sizeof(zd) * 36 * (size_t)c->g.stride;
+    // room for the forms of complex links, whichever the gauge field has
+    const size_t plane = (size_t)c->g.stride;
+    const size_t bytesA = 4 * plane * lym::block_bytes(0, lym::BLK_A);
+    const bool real = g->real_links;
     if (!g->B) {
-        int rc = dmalloc(c, (void**)&g->B, 2 * blk);
+        int rc = dmalloc(c, (void**)&g->B, bytesA);
         if (rc) return rc;
         lym::launch_clover_B(c->g, g->U, link_kind(g), reinterpret_cast<zd*>(g->B), c->stream);
         CHECK_LAUNCH();
     }
     if (!op->A) {
-        int rc = dmalloc(c, (void**)&op->A, 2 * blk);
+        int rc = dmalloc(c, (void**)&op->A, bytesA);
         if (rc) return rc;
     }
     if (!op->Ainv) {
-        int rc = dmalloc(c, (void**)&op->Ainv, blk);
+        int rc = dmalloc(c, (void**)&op->Ainv, 2 * plane * lym::block_bytes(0, lym::BLK_INV));
         if (rc) return rc;
     }
     lym::launch_clover_A(c->g, reinterpret_cast<const zd*>(g->B), op->kappa * op->csw, reinterpret_cast<zd*>(op->A),
-                         c->stream);
+                         real, c->stream);
     CHECK_LAUNCH();
     // unpivoted LDL^H inverse first; the pivoted Gauss-Jordan redoes the parity
     // if any block had a small pivot, and reports singular blocks
     int* flag = reinterpret_cast<int*>(c->red_result) + 32;
     HIPCHECK(hipMemsetAsync(flag, 0, 2 * sizeof(int), c->stream));
-    lym::launch_clover_inv_ldl(c->g, reinterpret_cast<const zd*>(op->A), reinterpret_cast<zd*>(op->Ainv), flag + 1,
-                               c->stream);
+    lym::launch_clover_inv_ldl(c->g, reinterpret_cast<const zd*>(op->A), reinterpret_cast<zd*>(op->Ainv), real,
+                               flag + 1, c->stream);
     CHECK_LAUNCH();
     int hflag[2] = {0, 0};
     HIPCHECK(hipMemcpyAsync(hflag, flag, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -132,7 +135,7 @@ int op_prepare(lym_op* op, bool force_blocks) {
     // LYM_CLOVER_INV_PIVOTED=1 always takes the pivoted path (lets tests cover it)
     const char* force = std::getenv("LYM_CLOVER_INV_PIVOTED");
     if (hflag[1] || (force && force[0] == '1')) {
-        lym::launch_clover_inv(c->g, reinterpret_cast<const zd*>(op->A), reinterpret_cast<zd*>(op->Ainv), flag,
+        lym::launch_clover_inv(c->g, reinterpret_cast<const zd*>(op->A), reinterpret_cast<zd*>(op->Ainv), real, flag,
                                c->stream);
         CHECK_LAUNCH();
         HIPCHECK(hipMemcpyAsync(hflag, flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -185,7 +188,6 @@ int op_sloppy_data(lym_op* op, int prec, bool full_rows) {
     const int ncomp = g->real_links ? g->compression : g->compression / 2;
     const long nl = 2L * 4 * ncomp * S;
     const size_t le = g->real_links ? (prec == 1 ? 4 : 2) : (prec == 1 ? 8 : 4);
-    const size_t se = prec == 1 ? 8 : 4;  // spinor/block element
     int rc = LYM_OK;
     if (!op->Us) rc = dmalloc(c, &op->Us, 2L * 4 * 9 * S * le);  // room for 18-real links
     if (rc) return rc;
@@ -209,14 +211,15 @@ int op_sloppy_data(lym_op* op, int prec, bool full_rows) {
         }
     }
     if (op->A) {
-        if (!op->As) rc = dmalloc(c, &op->As, 2L * 36 * S * se);
+        if (!op->As) rc = dmalloc(c, &op->As, 4L * S * lym::block_bytes(1, lym::BLK_A));
         if (!rc && !op->As_sc) rc = dmalloc(c, (void**)&op->As_sc, 2L * S * sizeof(float));
-        if (!rc && !op->Ainvs) rc = dmalloc(c, &op->Ainvs, 36L * S * se);
+        if (!rc && !op->Ainvs) rc = dmalloc(c, &op->Ainvs, 2L * S * lym::block_bytes(1, lym::BLK_INV));
         if (!rc && !op->Ainvs_sc) rc = dmalloc(c, (void**)&op->Ainvs_sc, S * sizeof(float));
         if (rc) return rc;
-        lym::launch_convert_blocks(prec, reinterpret_cast<const zd*>(op->A), op->As, op->As_sc, 2, (int)S, c->stream);
-        lym::launch_convert_blocks(prec, reinterpret_cast<const zd*>(op->Ainv), op->Ainvs, op->Ainvs_sc, 1, (int)S,
-                                   c->stream);
+        lym::launch_convert_blocks(prec, reinterpret_cast<const zd*>(op->A), op->As, op->As_sc,
+                                   g->real_links ? lym::BLK_A_REAL : lym::BLK_A, (int)S, c->stream);
+        lym::launch_convert_blocks(prec, reinterpret_cast<const zd*>(op->Ainv), op->Ainvs, op->Ainvs_sc,
+                                   g->real_links ? lym::BLK_INV_REAL : lym::BLK_INV, (int)S, c->stream);
     }
     CHECK_LAUNCH();
     op->sloppy_prec = prec;
@@ -532,8 +535,8 @@ int apply_schur_sloppy(lym_op* op, int prec, void* out_o, float* out_sc, const v
 // src_o = b_o - D_oe Ainv b_e  (te: even scratch)
 void eo_source_nr(lym_op* op, int nr, const zd* b, zd* te, zd* src_o) {
     lym_ctx* c = op->ctx;
-    lym::launch_clover_apply_lanes(c->g, reinterpret_cast<const zd*>(op->Ainv), 0, nullptr, nullptr, b, full_n(c), te,
-                                   half_n(c), nr, c->stream);
+    lym::launch_inv_apply(c->g, reinterpret_cast<const zd*>(op->Ainv), op->gauge->real_links, 0, nullptr, nullptr, b,
+                          full_n(c), te, half_n(c), nr, c->stream);
     lym::DslashParams a = base_params(op);
     set_lanes(a, nr, half_n(c), full_n(c), half_n(c));
     a.hop_sign = -1.0;

@@ -464,20 +464,6 @@ __global__ void k_relayout(const E* in, E* out, long rows, int w_old, int w_new)
     }
 }
 
-__global__ void k_clover_apply_lanes(Geom g, const zd* __restrict__ blocks, long set_elems, const int* lane_set,
-                                     const int* mask, const zd* __restrict__ in, long in_lane, zd* __restrict__ out,
-                                     long out_lane) {
-    const int l = blockIdx.y, idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (idx >= g.Vh || (mask && !mask[l])) return;
-    const zd* B = blocks + (lane_set ? lane_set[l] * set_elems : 0);
-    zd s[12], o[12];
-    load_spinor(in + l * in_lane, g.stride, idx, s);
-    herm6(B, g.stride, idx, s, o);
-    herm6(B + (size_t)18 * g.stride, g.stride, idx, s + 6, o + 6);
-#pragma unroll
-    for (int k = 0; k < 12; ++k) out[l * out_lane + (long)k * g.stride + idx] = o[k];
-}
-
 // ---------------------------------------------------------------- launchers
 static inline int bsite_blocks(long n) {
     long b = (n + 255) / 256;
@@ -618,11 +604,6 @@ void launch_zero_padding(int esize, void* buf, long groups, int stride, int vh, 
             break;
         default: hipLaunchKernelGGL(k_zero_padding<float>, g, b, 0, st, (float*)buf, groups, stride, vh, nr); break;
     }
-}
-void launch_clover_apply_lanes(const Geom& g, const zd* blocks, long set_elems, const int* lane_set, const int* mask,
-                               const zd* in, long in_lane, zd* out, long out_lane, int lanes, hipStream_t st) {
-    hipLaunchKernelGGL(k_clover_apply_lanes, dim3((g.Vh + 255) / 256, lanes), dim3(256), 0, st, g, blocks, set_elems,
-                       lane_set, mask, in, in_lane, out, out_lane);
 }
 
 }  // namespace lym

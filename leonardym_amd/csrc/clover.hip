@@ -101,30 +101,79 @@ __device__ M3 field_strength(const Geom& g, const void* links, const int c[4], i
 
 __device__ __forceinline__ zd ti(zd z) { return mulph<1>(z); }
 
-// store one hermitian 6x6 (full, row-major h[6][6]) packed
-__device__ __forceinline__ void store_herm6(zd* base, int stride, int idx, const zd h[36]) {
-    for (int k = 0; k < 3; ++k) base[(size_t)k * stride + idx] = mk(h[(2 * k) * 7].re, h[(2 * k + 1) * 7].re);
-    int k = 3;
-    for (int i = 1; i < 6; ++i)
-        for (int j = 0; j < i; ++j) {
-            base[(size_t)k * stride + idx] = h[6 * i + j];
-            ++k;
+// the inverse R of a block (row-major 6x6; real links: averaged over the entries
+// that are equal but for rounding)
+template <bool REAL>
+__device__ __forceinline__ void store_inverse(zd* base, int stride, int h, int idx, const zd R[36]) {
+    constexpr int BK = REAL ? BLK_INV_REAL : BLK_INV;
+    double e[block_reals(BK)];
+    if constexpr (REAL) {
+        int k = 3;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            e[i] = 0.5 * (R[7 * i].re + R[7 * (3 + i)].re);
+#pragma unroll
+            for (int j = 0; j < i; ++j) {
+                const zd a = R[6 * i + j], d = R[6 * (3 + i) + 3 + j];
+                e[k] = 0.5 * (a.re + d.re);
+                e[k + 3] = 0.5 * (a.im - d.im);
+                const zd x = 0.5 * (R[6 * (3 + i) + j] - R[6 * (3 + j) + i]);
+                e[2 * k + 3] = x.re;
+                e[2 * k + 4] = x.im;
+                ++k;
+            }
         }
+    } else {
+        int k = 6;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            e[i] = R[7 * i].re;
+#pragma unroll
+            for (int j = 0; j < i; ++j) {
+                e[k] = R[6 * i + j].re;
+                e[k + 1] = R[6 * i + j].im;
+                k += 2;
+            }
+        }
+    }
+    store_block<0, BK>(base, 2, stride, h, idx, e);
 }
 
-__device__ __forceinline__ void load_herm6(const zd* base, int stride, int idx, zd h[36]) {
-    for (int k = 0; k < 3; ++k) {
-        zd d = base[(size_t)k * stride + idx];
-        h[(2 * k) * 7] = mk(d.re, 0.0);
-        h[(2 * k + 1) * 7] = mk(d.im, 0.0);
-    }
-    int k = 3;
-    for (int i = 1; i < 6; ++i)
+// D's block (parity 0, chirality h) as a full row-major 6x6
+template <bool REAL>
+__device__ __forceinline__ void load_full(const zd* A, int stride, int h, int idx, zd M[36]) {
+    constexpr int BK = REAL ? BLK_A_REAL : BLK_A;
+    double e[block_reals(BK)];
+    load_block<0, BK, false>(A, 4, stride, h, idx, e);
+    int k = REAL ? 0 : 3, x = REAL ? 3 : 9;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        M[7 * i] = mk(REAL ? 1.0 : 1.0 + e[i], 0.0);
+        M[7 * (3 + i)] = mk(REAL ? 1.0 : 1.0 - e[i], 0.0);
+#pragma unroll
         for (int j = 0; j < i; ++j) {
-            zd a = base[(size_t)k * stride + idx];
-            h[6 * i + j] = a;
-            h[6 * j + i] = conj(a);
-            ++k;
+            const zd d = REAL ? mk(0.0, e[k]) : mk(e[k], e[k + 1]);
+            k += REAL ? 1 : 2;
+            M[6 * i + j] = d;
+            M[6 * j + i] = conj(d);
+            M[6 * (3 + i) + 3 + j] = -d;
+            M[6 * (3 + j) + 3 + i] = -conj(d);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            zd v = mk(0.0, 0.0);
+            if constexpr (REAL) {
+                const int hi = i > j ? i : j, lo = i > j ? j : i, o = 3 + 2 * (hi == 1 ? 0 : hi + lo - 1);
+                if (i != j) v = i > j ? mk(e[o], e[o + 1]) : mk(-e[o], -e[o + 1]);
+            } else {
+                v = mk(e[x], e[x + 1]);
+                x += 2;
+            }
+            M[6 * (3 + i) + j] = v;
+            M[6 * j + 3 + i] = conj(v);
         }
 }
 
@@ -162,18 +211,36 @@ __device__ __forceinline__ void acc_plane(const M3& F, zd du[6], zd dl[6], zd X[
     }
 }
 
-// the packed hermitian 6x6 of spin blocks (0,0) = d, (1,1) = -d, (1,0) = X:
-// diagonal pairs, then the lower entries row by row (the store_herm6 order)
-__device__ __forceinline__ void store_spin_blocks(zd* base, int stride, int idx, const zd d[6], const zd X[9]) {
-    base[idx] = mk(d[0].re, d[1].re);
-    base[(size_t)stride + idx] = mk(d[2].re, -d[0].re);
-    base[(size_t)2 * stride + idx] = mk(-d[1].re, -d[2].re);
-    const zd e[15] = {d[3],  d[4], d[5],                                     // rows 1, 2
-                      X[0],  X[1], X[2],                                     // row 3
-                      X[3],  X[4], X[5], -d[3],                              // row 4
-                      X[6],  X[7], X[8], -d[4], -d[5]};                      // row 5
+// the numbers of spin blocks (0,0) = d, (1,1) = -d, (1,0) = X (D and X of the stored
+// form; for real links d is imaginary and X antisymmetric, exactly)
+template <bool REAL>
+__device__ __forceinline__ void store_spin_blocks(zd* B, int stride, int plane, int idx, const zd d[6],
+                                                  const zd X[9]) {
+    constexpr int BK = REAL ? BLK_A_REAL : BLK_A;
+    double e[block_reals(BK)];
+    if constexpr (REAL) {
 #pragma unroll
-    for (int k = 0; k < 15; ++k) base[(size_t)(3 + k) * stride + idx] = e[k];
+        for (int k = 0; k < 3; ++k) e[k] = d[3 + k].im;
+        const zd x[3] = {X[3], X[6], X[7]};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            e[3 + 2 * k] = x[k].re;
+            e[4 + 2 * k] = x[k].im;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            e[k] = d[k].re;
+            e[3 + 2 * k] = d[3 + k].re;
+            e[4 + 2 * k] = d[3 + k].im;
+        }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            e[9 + 2 * k] = X[k].re;
+            e[10 + 2 * k] = X[k].im;
+        }
+    }
+    store_block<0, BK>(B, 4, stride, plane, idx, e);
 }
 
 // One thread per site.  Each XCD takes a contiguous range of site blocks with
@@ -205,27 +272,21 @@ __global__ __launch_bounds__(128) void k_clover_B(Geom g, const void* links, zd*
     acc_plane<3>(field_strength<LK>(g, links, c, 1, 2), du, dl, X, Y);
     acc_plane<4>(field_strength<LK>(g, links, c, 1, 3), du, dl, X, Y);
     acc_plane<5>(field_strength<LK>(g, links, c, 2, 3), du, dl, X, Y);
-    zd* base = B + (size_t)p * 36 * g.stride;
-    store_spin_blocks(base, g.stride, idx, du, X);
-    store_spin_blocks(base + (size_t)18 * g.stride, g.stride, idx, dl, Y);
+    store_spin_blocks<(LK >= 2)>(B, g.stride, 2 * p, idx, du, X);
+    store_spin_blocks<(LK >= 2)>(B, g.stride, 2 * p + 1, idx, dl, Y);
 }
 
-// A = 1 + kc gamma5 B: upper block 1 + kc B_u, lower block 1 - kc B_l
-__global__ void k_clover_A(Geom g, const zd* __restrict__ B, double kc, zd* __restrict__ A) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    long n = 2L * 36 * g.stride;
-    if (i >= n) return;
-    int comp = (int)((i / g.stride) % 36);
-    double s = comp < 18 ? kc : -kc;
-    int k = comp % 18;
-    zd b = B[i];
-    zd a = mk(s * b.re, s * b.im);
-    if (k < 3) {
-        // diagonal pairs
-        a.re += 1.0;
-        a.im += 1.0;
-    }
-    A[i] = a;
+// A = 1 + kc gamma5 B: upper block 1 + kc B_u, lower block 1 - kc B_l (the 1 is not
+// stored); n numbers per (plane, site), all but the last in pairs
+__global__ void k_clover_A(Geom g, const double* __restrict__ B, double kc, double* __restrict__ A, int n) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x, na = 4L * g.stride;
+    if (i >= na) return;
+    const double s = (i / g.stride) & 1 ? -kc : kc;
+    const zd* b = reinterpret_cast<const zd*>(B);
+    zd* a = reinterpret_cast<zd*>(A);
+    for (int k = 0; k < n / 2; ++k) a[na * k + i] = s * b[na * k + i];
+    const long t = 2 * na * (n / 2) + i;
+    if (n & 1) A[t] = s * B[t];
 }
 
 // Inverse of a hermitian 6x6 block through A = L D L^H (L unit lower
@@ -279,6 +340,7 @@ __device__ __forceinline__ bool herm6_inverse_ldl(const zd M[36], zd R[36]) {
     return ok;
 }
 
+template <bool REAL>
 __global__ __launch_bounds__(128) void k_clover_inv_ldl(Geom g, const zd* __restrict__ A, zd* __restrict__ Ainv,
                                                        int* fallback) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -286,20 +348,21 @@ __global__ __launch_bounds__(128) void k_clover_inv_ldl(Geom g, const zd* __rest
 #pragma unroll 1
     for (int blk = 0; blk < 2; ++blk) {
         zd M[36], R[36];
-        load_herm6(A + (size_t)18 * blk * g.stride, g.stride, idx, M);
+        load_full<REAL>(A, g.stride, blk, idx, M);
         if (!herm6_inverse_ldl(M, R)) atomicAdd(fallback, 1);
-        store_herm6(Ainv + (size_t)18 * blk * g.stride, g.stride, idx, R);
+        store_inverse<REAL>(Ainv, g.stride, blk, idx, R);
     }
 }
 
 // blockwise inverse on parity-0 sites: Gauss-Jordan with partial pivoting
+template <bool REAL>
 __global__ __launch_bounds__(64) void k_clover_inv(Geom g, const zd* __restrict__ A, zd* __restrict__ Ainv,
                                                    int* flag) {
     int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= g.Vh) return;
     for (int blk = 0; blk < 2; ++blk) {
         zd M[36], R[36];
-        load_herm6(A + (size_t)18 * blk * g.stride, g.stride, idx, M);
+        load_full<REAL>(A, g.stride, blk, idx, M);
         for (int k = 0; k < 36; ++k) R[k] = mk(k % 7 == 0 ? 1.0 : 0.0, 0.0);
         bool ok = true;
         for (int col = 0; col < 6; ++col) {
@@ -329,23 +392,25 @@ __global__ __launch_bounds__(64) void k_clover_inv(Geom g, const zd* __restrict_
             }
         }
         if (!ok) atomicAdd(flag, 1);
-        store_herm6(Ainv + (size_t)18 * blk * g.stride, g.stride, idx, R);
+        store_inverse<REAL>(Ainv, g.stride, blk, idx, R);
     }
 }
 
-// out = blocks * in on one parity (half fields), optional gamma5
-__global__ void k_clover_apply(Geom g, const zd* __restrict__ blocks, const zd* __restrict__ in, zd* __restrict__ out,
-                               int gamma5) {
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= g.Vh) return;
-    zd s[12], t[12];
-    load_spinor(in, g.stride, idx, s);
-    herm6(blocks, g.stride, idx, s, t);
-    herm6(blocks + (size_t)18 * g.stride, g.stride, idx, s + 6, t + 6);
-    for (int k = 0; k < 12; ++k) {
-        zd v = (gamma5 && k >= 6) ? -t[k] : t[k];
-        out[(size_t)k * g.stride + idx] = v;
-    }
+// out = blocks * in on the even half of lane fields
+template <bool REAL>
+__global__ void k_inv_apply(Geom g, const zd* __restrict__ blocks, long set_elems, const int* lane_set,
+                            const int* mask, const zd* __restrict__ in, long in_lane, zd* __restrict__ out,
+                            long out_lane) {
+    constexpr int BK = REAL ? BLK_INV_REAL : BLK_INV;
+    const int l = blockIdx.y, idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (idx >= g.Vh || (mask && !mask[l])) return;
+    const zd* B = blocks + (lane_set ? lane_set[l] * set_elems : 0);
+    zd s[12], o[12];
+    load_spinor(in + l * in_lane, g.stride, idx, s);
+    block_apply_at<0, BK>(B, 2, g.stride, 0, idx, 1.0, s, o);
+    block_apply_at<0, BK>(B, 2, g.stride, 1, idx, 1.0, s + 6, o + 6);
+#pragma unroll
+    for (int k = 0; k < 12; ++k) out[l * out_lane + (long)k * g.stride + idx] = o[k];
 }
 
 void launch_clover_B(const Geom& g, const void* links, int link_kind, zd* B, hipStream_t st) {
@@ -358,21 +423,33 @@ void launch_clover_B(const Geom& g, const void* links, int link_kind, zd* B, hip
     }
 }
 
-void launch_clover_A(const Geom& g, const zd* B, double kc, zd* A, hipStream_t st) {
-    long n = 2L * 36 * g.stride;
-    hipLaunchKernelGGL(k_clover_A, dim3((n + 255) / 256), dim3(256), 0, st, g, B, kc, A);
+void launch_clover_A(const Geom& g, const zd* B, double kc, zd* A, bool real_links, hipStream_t st) {
+    hipLaunchKernelGGL(k_clover_A, dim3((4L * g.stride + 255) / 256), dim3(256), 0, st, g,
+                       reinterpret_cast<const double*>(B), kc, reinterpret_cast<double*>(A),
+                       block_reals(real_links ? BLK_A_REAL : BLK_A));
 }
 
-void launch_clover_inv(const Geom& g, const zd* A, zd* Ainv, int* flag, hipStream_t st) {
-    hipLaunchKernelGGL(k_clover_inv, dim3((g.Vh + 63) / 64), dim3(64), 0, st, g, A, Ainv, flag);
+void launch_clover_inv(const Geom& g, const zd* A, zd* Ainv, bool real_links, int* flag, hipStream_t st) {
+    const dim3 nb((g.Vh + 63) / 64), th(64);
+    if (real_links) hipLaunchKernelGGL(k_clover_inv<true>, nb, th, 0, st, g, A, Ainv, flag);
+    else hipLaunchKernelGGL(k_clover_inv<false>, nb, th, 0, st, g, A, Ainv, flag);
 }
 
-void launch_clover_inv_ldl(const Geom& g, const zd* A, zd* Ainv, int* fallback, hipStream_t st) {
-    hipLaunchKernelGGL(k_clover_inv_ldl, dim3((g.Vh + 127) / 128), dim3(128), 0, st, g, A, Ainv, fallback);
+void launch_clover_inv_ldl(const Geom& g, const zd* A, zd* Ainv, bool real_links, int* fallback, hipStream_t st) {
+    const dim3 nb((g.Vh + 127) / 128), th(128);
+    if (real_links) hipLaunchKernelGGL(k_clover_inv_ldl<true>, nb, th, 0, st, g, A, Ainv, fallback);
+    else hipLaunchKernelGGL(k_clover_inv_ldl<false>, nb, th, 0, st, g, A, Ainv, fallback);
 }
 
-void launch_clover_apply(const Geom& g, const zd* blocks, const zd* in, zd* out, int gamma5, hipStream_t st) {
-    hipLaunchKernelGGL(k_clover_apply, dim3((g.Vh + 255) / 256), dim3(256), 0, st, g, blocks, in, out, gamma5);
+void launch_inv_apply(const Geom& g, const zd* blocks, bool real_links, long set_elems, const int* lane_set,
+                      const int* mask, const zd* in, long in_lane, zd* out, long out_lane, int lanes, hipStream_t st) {
+    const dim3 nb((g.Vh + 255) / 256, lanes), th(256);
+    if (real_links)
+        hipLaunchKernelGGL(k_inv_apply<true>, nb, th, 0, st, g, blocks, set_elems, lane_set, mask, in, in_lane, out,
+                           out_lane);
+    else
+        hipLaunchKernelGGL(k_inv_apply<false>, nb, th, 0, st, g, blocks, set_elems, lane_set, mask, in, in_lane, out,
+                           out_lane);
 }
 
 }  // namespace lym

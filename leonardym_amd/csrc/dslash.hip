@@ -155,7 +155,7 @@ __device__ __forceinline__ void hop_pair(const DslashParams& a, int p, int site,
     if constexpr (pin_end) pin(acc);
 }
 
-template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD = false, int BM = 0, int FM = 0,
+template <int PR, int LK, int DIAG, bool INV, bool NORM, bool LO, bool UPD = false, int BM = 0, int FM = 0,
           bool NT = true>
 __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, int site, int r,
                                                   const cplx<typename Prec<PR>::T> acc[12], float ual = 0.f,
@@ -191,13 +191,13 @@ __device__ __forceinline__ double dslash_site(const DslashParams& a, int p, int 
         hop_pair<2, PR, LK>(a, p, site, r, c, acc, lds, lbase);
         hop_pair<3, PR, LK>(a, p, site, r, c, acc, lds, lbase);
     }
-    return dslash_epilogue<PR, DIAG, INV, NORM, LO, UPD, BM, FM, NT>(a, p, site, r, acc, ual, al, sums);
+    return dslash_epilogue<PR, LK, DIAG, INV, NORM, LO, UPD, BM, FM, NT>(a, p, site, r, acc, ual, al, sums);
 }
 
 // The site's output from its hopping sum acc: v = diag(psi_x) + hop_sign
 // (-kappa acc), then R^-1, gamma5, the axpy and the store (the value
 // returned is as for dslash_site)
-template <int PR, int DIAG, bool INV, bool NORM, bool LO, bool UPD, int BM, int FM, bool NT>
+template <int PR, int LK, int DIAG, bool INV, bool NORM, bool LO, bool UPD, int BM, int FM, bool NT>
 __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, int site, int r,
                                                   const cplx<typename Prec<PR>::T> acc[12], float ual, double al64,
                                                   double* sums) {
@@ -206,6 +206,7 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
     const int ST = a.g.stride;
     const double kap = LO ? a.kappa_dev[r] : (a.kappa_dev ? *a.kappa_dev : a.kappa);
     const T hk = (T)(-kap * a.hop_sign);
+    constexpr int BK_A = LK >= 2 ? BLK_A_REAL : BLK_A, BK_I = LK >= 2 ? BLK_INV_REAL : BLK_INV;
     // this lane's clover blocks
     const void* Ab_ = a.A;
     const void* Ai_ = a.Ainv;
@@ -226,14 +227,18 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
 #pragma unroll
         for (int k = 0; k < 12; ++k) v[k] = hk * acc[k];
     } else if constexpr (DIAG == 2 && PR >= 1) {
-        // A (sc_psi psi) = (sc_A sc_psi) (A psi): both FP16 scales on the 12 outputs
+        // the field's FP16 scale on the 12 outputs
         cplx<T> s[12], t[12];
         T scp;
         load_spinor_unscaled<PR>(SpinorRef<PR>{reinterpret_cast<const S*>(a.diag_in[p]), a.diag_sc[p]}, ST, a.nr,
                                  site, r, s, scp);
-        const T sc = PR == 2 ? (T)Asc_[(size_t)p * ST + site] * scp : (T)1;
-        herm6_packed<PR>(Ab_, 4 * (size_t)ST, (size_t)(2 * p) * ST, site, sc, s, t);
-        herm6_packed<PR>(Ab_, 4 * (size_t)ST, (size_t)(2 * p + 1) * ST, site, sc, s + 6, t + 6);
+        const T sc = PR == 2 ? (T)Asc_[(size_t)p * ST + site] : (T)1;
+        block_apply_at<PR, BK_A>(Ab_, 4, ST, 2 * p, site, sc, s, t);
+        block_apply_at<PR, BK_A>(Ab_, 4, ST, 2 * p + 1, site, sc, s + 6, t + 6);
+        if constexpr (PR == 2) {
+#pragma unroll
+            for (int k = 0; k < 12; ++k) t[k] = scp * t[k];
+        }
 #pragma unroll
         for (int k = 0; k < 12; ++k) v[k] = axpy1(hk, acc[k], t[k]);
     } else {
@@ -242,9 +247,8 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
                         site, field_rhs<PR>(r), s);
         if constexpr (DIAG == 2) {
             cplx<T> t[12];
-            const S* Ab = reinterpret_cast<const S*>(Ab_) + (size_t)p * 36 * ST;
-            herm6<PR, NT>(Ab, ST, site, (T)1, s, t);
-            herm6<PR, NT>(Ab + (size_t)18 * ST, ST, site, (T)1, s + 6, t + 6);
+            block_apply_at<PR, BK_A, NT>(Ab_, 4, ST, 2 * p, site, (T)1, s, t);
+            block_apply_at<PR, BK_A, NT>(Ab_, 4, ST, 2 * p + 1, site, (T)1, s + 6, t + 6);
 #pragma unroll
             for (int k = 0; k < 12; ++k) v[k] = axpy1(hk, acc[k], t[k]);
         } else {
@@ -254,15 +258,9 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
     }
     if constexpr (INV) {
         cplx<T> t[12];
-        if constexpr (PR == 0) {
-            const S* Ai = reinterpret_cast<const S*>(Ai_);
-            herm6<PR, NT>(Ai, ST, site, (T)1, v, t);
-            herm6<PR, NT>(Ai + (size_t)18 * ST, ST, site, (T)1, v + 6, t + 6);
-        } else {
-            const T sc = PR == 2 ? (T)Aisc_[site] : (T)1;
-            herm6_packed<PR>(Ai_, 2 * (size_t)ST, 0, site, sc, v, t);
-            herm6_packed<PR>(Ai_, 2 * (size_t)ST, (size_t)ST, site, sc, v + 6, t + 6);
-        }
+        const T sc = PR == 2 ? (T)Aisc_[site] : (T)1;
+        block_apply_at<PR, BK_I, NT || PR != 0>(Ai_, 2, ST, 0, site, sc, v, t);
+        block_apply_at<PR, BK_I, NT || PR != 0>(Ai_, 2, ST, 1, site, sc, v + 6, t + 6);
 #pragma unroll
         for (int k = 0; k < 12; ++k) v[k] = t[k];
     }
@@ -509,11 +507,11 @@ __device__ __forceinline__ void epilogue_half_lp(const DslashParams& a, int p, i
 #pragma unroll
         for (int k = 0; k < 6; ++k) s6[k] = to_c<PR>(e[k]);
         if constexpr (DIAG == 2) {
-            const T sc = PR == 2 ? (T)a.A_sc[(size_t)p * ST + site] * scp : (T)1;
+            const T sc = PR == 2 ? (T)a.A_sc[(size_t)p * ST + site] : (T)1;
             cplx<T> t[6];
-            herm6_packed<PR>(a.A, 4 * (size_t)ST, (size_t)(2 * p + h) * ST, site, sc, s6, t);
+            block_apply_at<PR, LK >= 2 ? BLK_A_REAL : BLK_A>(a.A, 4, ST, 2 * p + h, site, sc, s6, t);
 #pragma unroll
-            for (int k = 0; k < 6; ++k) v[k] = t[k] + hk * u[k];
+            for (int k = 0; k < 6; ++k) v[k] = axpy1(hk, u[k], PR == 2 ? scp * t[k] : t[k]);
         } else {
 #pragma unroll
             for (int k = 0; k < 6; ++k) v[k] = scp * s6[k] + hk * u[k];
@@ -522,7 +520,7 @@ __device__ __forceinline__ void epilogue_half_lp(const DslashParams& a, int p, i
     if constexpr (INV) {
         const T sc = PR == 2 ? (T)a.Ainv_sc[site] : (T)1;
         cplx<T> t[6];
-        herm6_packed<PR>(a.Ainv, 2 * (size_t)ST, (size_t)h * ST, site, sc, v, t);
+        block_apply_at<PR, LK >= 2 ? BLK_INV_REAL : BLK_INV>(a.Ainv, 2, ST, h, site, sc, v, t);
 #pragma unroll
         for (int k = 0; k < 6; ++k) v[k] = t[k];
     }
@@ -889,7 +887,7 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) void k_dslash_mfma(DslashParams
                 const float* slot = accs + t * MFMA_LDS_STRIDE;
 #pragma unroll
                 for (int k = 0; k < 12; ++k) acc[k] = mk(slot[2 * k], slot[2 * k + 1]);
-                (void)dslash_epilogue<2, DIAG, INV, false, LO>(a, p, site, r, acc);
+                (void)dslash_epilogue<2, 0, DIAG, INV, false, LO>(a, p, site, r, acc);
             }
         }
         __syncthreads();

@@ -96,19 +96,6 @@ __device__ __forceinline__ void add_hop(cplx<typename Prec<PR>::T> u[6], const c
     if constexpr (PR == 0 || !FWD) asm volatile("" ::: "memory");
 }
 
-// the 18 entries of the clover block (chirality h) of a site, unscaled
-template <int PR>
-__device__ __forceinline__ void load_block(const void* base, int nparity, int stride, int p, int h, int idx,
-                                           cplx<typename Prec<PR>::T> e[18]) {
-    if constexpr (PR == 0) {
-        const zd* A = reinterpret_cast<const zd*>(base) + (size_t)(36 * p + 18 * h) * stride;
-#pragma unroll
-        for (int k = 0; k < 18; ++k) e[k] = fld<zd, true>(A + (size_t)k * stride, (unsigned)idx);
-    } else {
-        load_block_packed<PR>(base, 2 * (size_t)nparity * stride, (size_t)(2 * p + h) * stride, idx, e);
-    }
-}
-
 // spins 2h, 2h + 1 of a spinor, unscaled
 template <int PR, bool NT = false>
 __device__ __forceinline__ void load_half(const void* base, size_t ks, unsigned o, int h,
@@ -322,7 +309,9 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
 
     // ------------------------------------------------ chirality h
     const int h = w - HOP_WAVES;
-    cplx<T> s[6], binv[18], w2[6];  // s: the diagonal term, formed while the hops are under way
+    constexpr int BK_A = LK >= 2 ? BLK_A_REAL : BLK_A, BK_I = LK >= 2 ? BLK_INV_REAL : BLK_INV;
+    cplx<T> s[6], w2[6];  // s: the diagonal term, formed while the hops are under way
+    T binv[block_reals(BK_I)];
     T isc = (T)1, hk = (T)0, wsc = (T)1;
     if (ok) {
         const void *Ab = a.A, *Ai = a.Ainv;
@@ -337,7 +326,7 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
             }
         }
         if constexpr (INV) {
-            load_block<PR>(Ai, 1, ST, 0, h, site, binv);
+            load_block<PR, BK_I>(Ai, 2, ST, h, site, binv);
             if constexpr (PR == 2) isc = Aisc[site];
         }
         if (!INV && a.v2[p]) {
@@ -345,12 +334,13 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
             if constexpr (PR == 2) wsc = fld<float>(a.v2_sc[p], o);
         }
         if constexpr (DIAG == 2) {
-            cplx<T> blk[18], t[6];
+            cplx<T> t[6];
+            T blk[block_reals(BK_A)];
             T sc = (T)1;
             load_half<PR>(lane_base<PR>(a.diag_in[p], a.diag_lane, r), ks, o, h, t);
-            load_block<PR>(Ab, 2, ST, p, h, site, blk);
-            if constexpr (PR == 2) sc = Asc[(size_t)p * ST + site] * fld<float>(a.diag_sc[p], o);
-            herm6_mul<T>(blk, t, s);
+            load_block<PR, BK_A>(Ab, 4, ST, 2 * p + h, site, blk);
+            if constexpr (PR == 2) sc = fld<float>(a.diag_sc[p], o);
+            block_apply<PR, BK_A>(blk, PR == 2 ? (T)Asc[(size_t)p * ST + site] : (T)1, t, s);
             if constexpr (PR == 2) {
 #pragma unroll
                 for (int k = 0; k < 6; ++k) s[k] = sc * s[k];
@@ -431,12 +421,9 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
         }
         if constexpr (INV) {
             cplx<T> t[6];
-            herm6_mul<T>(binv, v, t);
+            block_apply<PR, BK_I>(binv, isc, v, t);
 #pragma unroll
-            for (int k = 0; k < 6; ++k) {
-                if constexpr (PR == 2) v[k] = isc * t[k];
-                else v[k] = t[k];
-            }
+            for (int k = 0; k < 6; ++k) v[k] = t[k];
         }
         if (a.gamma5 && h) {
 #pragma unroll

@@ -127,6 +127,14 @@ bool full_rows(const lym_gauge* g) {
     return !(g->rows_rebuild && ncomp == 6);
 }
 
+// bytes of one block set: D's blocks and the inverses
+long set_bytes_A(const lym_gauge* g, int prec) {
+    return 4L * g->ctx->g.stride * lym::block_bytes(prec, g->real_links ? lym::BLK_A_REAL : lym::BLK_A);
+}
+long set_bytes_inv(const lym_gauge* g, int prec) {
+    return 2L * g->ctx->g.stride * lym::block_bytes(prec, g->real_links ? lym::BLK_INV_REAL : lym::BLK_INV);
+}
+
 // the per-lane operator data of one launch at storage precision prec
 void lane_ops(LaneEngine* e, lym::DslashParams& a, int prec) {
     a.prec = prec;
@@ -138,16 +146,16 @@ void lane_ops(LaneEngine* e, lym::DslashParams& a, int prec) {
         a.links = e->g->U;
         a.A = e->A;
         a.Ainv = e->Ainv;
-        a.A_lane_bytes = 72 * S * (long)sizeof(zd);
-        a.Ainv_lane_bytes = 36 * S * (long)sizeof(zd);
+        a.A_lane_bytes = set_bytes_A(e->g, 0);
+        a.Ainv_lane_bytes = set_bytes_inv(e->g, 0);
     } else {
         a.links = e->Us;
         a.A = e->As;
         a.A_sc = e->As_sc;
         a.Ainv = e->Ainvs;
         a.Ainv_sc = e->Ainvs_sc;
-        a.A_lane_bytes = 72 * S * (long)e->es;
-        a.Ainv_lane_bytes = 36 * S * (long)e->es;
+        a.A_lane_bytes = set_bytes_A(e->g, e->prec);
+        a.Ainv_lane_bytes = set_bytes_inv(e->g, e->prec);
         a.Asc_lane = 2 * S;
         a.Ainvsc_lane = S;
     }
@@ -342,7 +350,10 @@ size_t engine_bytes(const int dims[4], int rep, int storage, int prec, int wmax)
     b += 2 * 24 * S * W * 16 + 8 * 12 * S * W * 16;  // FP64 nr-fields
     b += 2 * 12 * S * W * 8 + S * W * 8;             // x_s, r_s, the fused steps' terms
     b += 4 * (12 * S * W * es + S * W * 4);          // sloppy nr-fields
-    b += W * (72 * S * 16 + 36 * S * 16 + 72 * S * es + 36 * S * es + 3 * S * 4);  // operator data per lane
+    const int ka = rep == LYM_REP_SU2_ADJ ? lym::BLK_A_REAL : lym::BLK_A;
+    const int ki = rep == LYM_REP_SU2_ADJ ? lym::BLK_INV_REAL : lym::BLK_INV, pr = prec == LYM_PREC_SINGLE ? 1 : 2;
+    b += W * S * (4 * (lym::block_bytes(0, ka) + lym::block_bytes(pr, ka)) +
+                  2 * (lym::block_bytes(0, ki) + lym::block_bytes(pr, ki)) + 12);  // operator data per lane
     b += 72 * S * le;                                // low-precision links
     b += 2 * W * 24 * S * 16 + 12 * V * 16;          // transfer spinors, context staging
     return (size_t)(b * 1.03) + (32u << 20);
@@ -386,11 +397,11 @@ int engine_create(lym_ctx* ctx, const lym_gauge* g, double csw, int prec, unsign
         if (!rc) rc = ealloc(e, p, bytes);
     };
     A((void**)&e->kappa, sizeof(double) * lym::BMAX);
-    A((void**)&e->A, sizeof(zd) * 72 * S * W);
-    A((void**)&e->Ainv, sizeof(zd) * 36 * S * W);
-    A(&e->As, 72 * S * W * e->es);
+    A((void**)&e->A, set_bytes_A(g, 0) * W);
+    A((void**)&e->Ainv, set_bytes_inv(g, 0) * W);
+    A(&e->As, set_bytes_A(g, e->prec) * W);
     A((void**)&e->As_sc, sizeof(float) * 2 * S * W);
-    A(&e->Ainvs, 36 * S * W * e->es);
+    A(&e->Ainvs, set_bytes_inv(g, e->prec) * W);
     A((void**)&e->Ainvs_sc, sizeof(float) * S * W);
     // low-precision links: all three rows when the FP64 field has them
     // (every lane would otherwise rebuild row 2 of the same link)
@@ -498,22 +509,25 @@ static int build_set(LaneEngine* e, int q, double kappa) {
     lym_ctx* c = e->ctx;
     hipStream_t st = c->stream;
     const long S = e->S;
-    zd* Aq = e->A + 72 * S * q;
-    zd* Iq = e->Ainv + 36 * S * q;
-    lym::launch_clover_A(c->g, reinterpret_cast<const zd*>(e->g->B), kappa * e->csw, Aq, st);
+    const bool real = e->g->real_links;
+    zd* Aq = e->A + set_bytes_A(e->g, 0) / (long)sizeof(zd) * q;
+    zd* Iq = e->Ainv + set_bytes_inv(e->g, 0) / (long)sizeof(zd) * q;
+    lym::launch_clover_A(c->g, reinterpret_cast<const zd*>(e->g->B), kappa * e->csw, Aq, real, st);
     // a unit block for every lane stays exact at csw = 0 (B is then ignored)
     ECHECK(hipMemsetAsync(e->flag_d, 0, 2 * sizeof(int), st));
-    lym::launch_clover_inv_ldl(c->g, Aq, Iq, e->flag_d + 1, st);
+    lym::launch_clover_inv_ldl(c->g, Aq, Iq, real, e->flag_d + 1, st);
     ECHECK(hipMemcpyAsync(e->flag_h, e->flag_d, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
     ECHECK(hipStreamSynchronize(st));
     if (e->flag_h[1]) {
-        lym::launch_clover_inv(c->g, Aq, Iq, e->flag_d, st);
+        lym::launch_clover_inv(c->g, Aq, Iq, real, e->flag_d, st);
         ECHECK(hipMemcpyAsync(e->flag_h, e->flag_d, sizeof(int), hipMemcpyDeviceToHost, st));
         ECHECK(hipStreamSynchronize(st));
     }
     if (e->flag_h[0]) return fail(LYM_ERR_SINGULAR, "%d clover blocks are singular at kappa %g", e->flag_h[0], kappa);
-    lym::launch_convert_blocks(e->prec, Aq, (char*)e->As + 72 * S * e->es * q, e->As_sc + 2 * S * q, 2, (int)S, st);
-    lym::launch_convert_blocks(e->prec, Iq, (char*)e->Ainvs + 36 * S * e->es * q, e->Ainvs_sc + S * q, 1, (int)S, st);
+    lym::launch_convert_blocks(e->prec, Aq, (char*)e->As + set_bytes_A(e->g, e->prec) * q, e->As_sc + 2 * S * q,
+                               real ? lym::BLK_A_REAL : lym::BLK_A, (int)S, st);
+    lym::launch_convert_blocks(e->prec, Iq, (char*)e->Ainvs + set_bytes_inv(e->g, e->prec) * q, e->Ainvs_sc + S * q,
+                               real ? lym::BLK_INV_REAL : lym::BLK_INV, (int)S, st);
     ECHECK(hipGetLastError());
     return LYM_OK;
 }
@@ -597,7 +611,8 @@ int engine_admit(LaneEngine* e, int n, const LaneRequest* reqs, std::vector<Lane
     lym::launch_lane_gather(e->ptr_d, e->B, 24 * S, w, st);
     // the even-odd driver's right-hand side (PreconditionedBiCGStab.cpp:56-70):
     // src_o = b_o - D_oe R_ee^-1 b_e, rhs = Qhat gamma5 src_o
-    lym::launch_clover_apply_lanes(c->g, e->Ainv, 36 * S, e->lset_d, e->mask_d, e->B, 24 * S, e->te, 12 * S, w, st);
+    lym::launch_inv_apply(c->g, e->Ainv, e->g->real_links, set_bytes_inv(e->g, 0) / (long)sizeof(zd), e->lset_d,
+                          e->mask_d, e->B, 24 * S, e->te, 12 * S, w, st);
     lym::DslashParams a = base(e, 0);
     a.hop_sign = -1.0;
     a.parity = 1;

@@ -13,9 +13,9 @@
 //     links 18-real : double2 [2][4 mu][9 = 3*row + col][stride]
 //     links 12-real : double2 [2][4][6 = rows 0,1][stride], row 2 = conj(row0 x row1)
 //     adjoint links : double  [2][4][9 or 6][stride] (real SO(3), row 2 = row0 x row1)
-//     clover blocks : double2 [2][36][stride]: two hermitian 6x6 blocks (spins 0,1
-//                     and 2,3), each packed as 3 double2 of diagonal pairs then 15
-//                     complex lower-triangle entries, k = i(i-1)/2 + j for i > j.
+//     clover blocks : per parity and chirality the numbers a hermitian 6x6 block is
+//                     made of (BlockKind), in 16-byte vectors [planes][stride] and a
+//                     shorter rest (lym_device.h)
 //   Links are stored without the fermion boundary sign; the kernels apply the
 //   sign bc_t to the time hops that cross t = Lt-1 <-> 0, which keeps the
 //   12-real reconstruction exact for the sign-flipped links.
@@ -27,6 +27,17 @@
 #include <cstdint>
 
 namespace lym {
+
+// stored forms of a site's 6x6 diagonal blocks (lym_device.h): D's blocks and their
+// inverses, for complex and for real links; the numbers of one, and its bytes at a
+// storage precision (0 FP64, 1 FP32, 2 FP16)
+enum BlockKind { BLK_INV = 0, BLK_A = 1, BLK_INV_REAL = 2, BLK_A_REAL = 3 };
+__host__ __device__ constexpr int block_reals(int kind) {
+    return kind == BLK_INV ? 36 : kind == BLK_A ? 27 : kind == BLK_INV_REAL ? 15 : 9;
+}
+__host__ __device__ constexpr int block_bytes(int prec, int kind) {
+    return prec == 0 ? 8 * block_reals(kind) : prec == 1 ? 4 * block_reals(kind) : (2 * block_reals(kind) + 3) / 4 * 4;
+}
 
 // Device site order.  0: t fastest (the reference's lexicographic order; the
 // even-odd split needs Lt even).  1: t slowest, x fastest (needs Lx even): the
@@ -212,7 +223,7 @@ struct lym_gauge {
     int compression;   // 18 or 12 (9 or 6 for real adjoint links)
     int real_links;    // 1 for SU(2) adjoint
     void* U;           // links, see layout above
-    double2* B;        // kappa-independent clover blocks (hermitian, packed), built lazily
+    double2* B;        // kappa-independent clover blocks (BLK_A, BLK_A_REAL), built lazily
     int rows_rebuild;  // 1: row 2 of every link is the one rebuilt from rows 0 and 1 (SU(3) /
                        // SO(3) links), so the low-precision copies keep rows 0 and 1 only
 };

@@ -560,117 +560,220 @@ __device__ __forceinline__ void load_spinor(const cplx<double>* f, int stride, i
 }
 
 // ---------------------------------------------------------------- clover blocks
-// o = A v for one packed hermitian 6x6 block; A points at the block's first
-// component of the parity, sc is the per-site scale (PR == 2) or 1.
-template <int PR, bool NT = true>
-__device__ __forceinline__ void herm6(const typename Prec<PR>::S* A, int stride, int idx,
-                                      typename Prec<PR>::T sc, const cplx<typename Prec<PR>::T> v[6],
-                                      cplx<typename Prec<PR>::T> o[6]) {
+// A site's diagonal term is one hermitian 6x6 block per chirality (spins 2h, 2h + 1;
+// rows 3 spin + colour), and it is stored as the numbers it is made of.
+//  BLK_A       D's block: 1 + [[D, X^H], [X, -D]], D hermitian 3x3, X any 3x3:
+//              27 reals (D's diagonal, D_10 D_20 D_21, X by rows)
+//  BLK_INV     its inverse: 36 reals (six diagonal entries, the lower ones by rows)
+//  BLK_A_REAL, BLK_INV_REAL  the same for real links, whose field strengths are real
+//              and antisymmetric: D = i T and X antisymmetric (T real, X complex):
+//              9 reals (T_10 T_20 T_21, X_10 X_20 X_21); the inverse
+//              [[S + i T, X^H], [X, S - i T]], S real symmetric: 15 reals (S's
+//              diagonal, S_10 S_20 S_21, then as above)
+// The stencil is bound by memory, and stored as general hermitian blocks (36 reals)
+// they were 576 of the 1536 bytes of an FP64 clover apply's site (432 of 1392 now:
+// 32^3x64 761 -> 717 us) and 576 of the 1536 and 1728 of a Schur complement's even and
+// odd sites on real links (240 and 144 now: 24^3x48 Qhat^2 471 -> 389 us; its FP16
+// two-threads-per-site clover launch 59 -> 43 us).
+// D and X are stored without the 1, so the FP16 form's per-site scale is theirs.
+//
+// Layout, for every precision: a plane's block as 16-byte vectors and an 8- and
+// a 4-byte rest, piece k of every (plane, site) in one array [nplanes][stride],
+// the arrays one after the other (plane = 2 parity + h; h for the inverse).
+template <int BK>
+inline constexpr bool block_is_A = BK == BLK_A || BK == BLK_A_REAL;
+
+template <int PR, int BK>
+struct BlockStore {
     typedef typename Prec<PR>::T T;
-    T d[6];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        cplx<T> dd = to_c<PR>(fld<typename Prec<PR>::S, NT>(A + (size_t)k * stride, (unsigned)idx));
-        d[2 * k] = sc * dd.re;
-        d[2 * k + 1] = sc * dd.im;
-    }
-#pragma unroll
-    for (int i = 0; i < 6; ++i) o[i] = d[i] * v[i];
-    int k = 3;
-#pragma unroll
-    for (int i = 1; i < 6; ++i) {
-#pragma unroll
-        for (int j = 0; j < i; ++j) {
-            cplx<T> a = sc * to_c<PR>(fld<typename Prec<PR>::S, NT>(A + (size_t)k * stride, (unsigned)idx));
-            cfma(o[i], a, v[j]);
-            cfmac(o[j], a, v[i]);
-            ++k;
-        }
-    }
-}
-
-// The same product from the block's 18 entries already in registers (scaled).
-template <class T>
-__device__ __forceinline__ void herm6_mul(const cplx<T> a[18], const cplx<T> v[6], cplx<T> o[6]) {
-    T d[6];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        d[2 * k] = a[k].re;
-        d[2 * k + 1] = a[k].im;
-    }
-#pragma unroll
-    for (int i = 0; i < 6; ++i) o[i] = d[i] * v[i];
-    int k = 3;
-#pragma unroll
-    for (int i = 1; i < 6; ++i) {
-#pragma unroll
-        for (int j = 0; j < i; ++j) {
-            cfma(o[i], a[k], v[j]);
-            cfmac(o[j], a[k], v[i]);
-            ++k;
-        }
-    }
-}
-
-// Low-precision clover blocks: the 18 entries of each hermitian 6x6 block
-// (3 diagonal pairs, 15 off-diagonal) packed into 16- and 8-byte vectors.
-// Group g is an array [nplanes][stride] of vectors (plane = 2 parity + block
-// for the blocks of D, block for R^-1), the groups one after the other.
-// FP32: 144 B = 9 x 16; FP16: 72 B = 4 x 16 + 8.
-template <int PR>
-struct PackedBlock {
-    static_assert(PR >= 1, "packed blocks are low-precision only");
-    typedef typename Prec<PR>::S E;
-    static constexpr int BYTES = 18 * (int)sizeof(E);
+    static constexpr int N = block_reals(BK);
+    static constexpr int BYTES = block_bytes(PR, BK);
     static constexpr int N16 = BYTES / 16;
-    static constexpr bool H8 = BYTES - 16 * N16 >= 8;
+    static constexpr bool H8 = (BYTES & 8) != 0, H4 = (BYTES & 4) != 0;
+    static constexpr int SLOTS = BYTES / (PR == 0 ? 8 : PR == 1 ? 4 : 2);  // N and the FP16 form's padding
+};
+template <int PR>
+struct BlockReal {
+    typedef double E;
+};
+template <>
+struct BlockReal<1> {
+    typedef float E;
+};
+template <>
+struct BlockReal<2> {
+    typedef _Float16 E;
 };
 
-// the 18 entries (unscaled) of the block at plane_off = plane * stride of a
-// packed field whose group arrays hold ngroup vectors each
-template <int PR>
-__device__ __forceinline__ void load_block_packed(const void* base, size_t ngroup, size_t plane_off, int idx,
-                                                  cplx<typename Prec<PR>::T> a[18]) {
-    typedef PackedBlock<PR> P;
+// the block's numbers as stored (FP16: without the site's scale)
+template <int PR, int BK, bool NT = true>
+__device__ __forceinline__ void load_block(const void* base, int nplanes, int stride, int plane, int idx,
+                                           typename Prec<PR>::T e[block_reals(BK)]) {
+    typedef BlockStore<PR, BK> P;
     const char* gb = reinterpret_cast<const char*>(base);
+    const size_t na = (size_t)nplanes * stride, po = (size_t)plane * stride;
     unsigned char buf[P::BYTES];
-    int off = 0;
 #pragma unroll
-    for (int g = 0; g < P::N16; ++g) {
-        V16 w = fld<V16, true>(reinterpret_cast<const V16*>(gb) + plane_off, (unsigned)idx);
-        __builtin_memcpy(buf + off, &w, 16);
-        off += 16;
-        gb += ngroup * 16;
+    for (int k = 0; k < P::N16; ++k) {
+        const V16 w = fld<V16, NT>(reinterpret_cast<const V16*>(gb + 16 * na * k) + po, (unsigned)idx);
+        __builtin_memcpy(buf + 16 * k, &w, 16);
     }
+    gb += 16 * na * P::N16;
     if constexpr (P::H8) {
-        V8 w = fld<V8, true>(reinterpret_cast<const V8*>(gb) + plane_off, (unsigned)idx);
-        __builtin_memcpy(buf + off, &w, 8);
+        const V8 w = fld<V8, NT>(reinterpret_cast<const V8*>(gb) + po, (unsigned)idx);
+        __builtin_memcpy(buf + 16 * P::N16, &w, 8);
+        gb += 8 * na;
     }
-    typename P::E e[18];
-    __builtin_memcpy(e, buf, P::BYTES);
+    if constexpr (P::H4) {
+        const float w = fld<float, NT>(reinterpret_cast<const float*>(gb) + po, (unsigned)idx);
+        __builtin_memcpy(buf + P::BYTES - 4, &w, 4);
+    }
+    typename BlockReal<PR>::E s[P::SLOTS];
+    __builtin_memcpy(s, buf, P::BYTES);
 #pragma unroll
-    for (int k = 0; k < 18; ++k) a[k] = to_c<PR>(e[k]);
+    for (int k = 0; k < P::N; ++k) e[k] = (typename Prec<PR>::T)s[k];
+}
+template <int PR, int BK>
+__device__ __forceinline__ void store_block(void* base, int nplanes, int stride, int plane, int idx,
+                                            const typename Prec<PR>::T e[block_reals(BK)]) {
+    typedef BlockStore<PR, BK> P;
+    typename BlockReal<PR>::E s[P::SLOTS];
+#pragma unroll
+    for (int k = 0; k < P::SLOTS; ++k) s[k] = (typename BlockReal<PR>::E)(k < P::N ? e[k < P::N ? k : 0] : 0);
+    char* gb = reinterpret_cast<char*>(base);
+    const size_t na = (size_t)nplanes * stride, o = (size_t)plane * stride + idx;
+    const char* buf = reinterpret_cast<const char*>(s);
+#pragma unroll
+    for (int k = 0; k < P::N16; ++k) __builtin_memcpy(gb + 16 * (na * k + o), buf + 16 * k, 16);
+    gb += 16 * na * P::N16;
+    if constexpr (P::H8) {
+        __builtin_memcpy(gb + 8 * o, buf + 16 * P::N16, 8);
+        gb += 8 * na;
+    }
+    if constexpr (P::H4) __builtin_memcpy(gb + 4 * o, buf + P::BYTES - 4, 4);
 }
 
-// o = sc * A v for that block
-template <int PR>
-__device__ __forceinline__ void herm6_packed(const void* base, size_t ngroup, size_t plane_off, int idx,
-                                             typename Prec<PR>::T sc, const cplx<typename Prec<PR>::T> v[6],
-                                             cplx<typename Prec<PR>::T> o[6]) {
-    cplx<typename Prec<PR>::T> a[18];
-    load_block_packed<PR>(base, ngroup, plane_off, idx, a);
-    herm6_mul<typename Prec<PR>::T>(a, v, o);
-    if constexpr (PR == 2) {
-        // the block's scale on the 6 outputs instead of its 18 entries
-#pragma unroll
-        for (int i = 0; i < 6; ++i) o[i] = sc * o[i];
-    }
+// s += i t b (t real)
+template <class T>
+__device__ __forceinline__ void ifma(cplx<T>& s, T t, cplx<T> b) {
+    s.re = fmadd(-t, b.im, s.re);
+    s.im = fmadd(t, b.re, s.im);
 }
 
-// FP64 form used by the clover builder and the EO driver
-__device__ __forceinline__ void herm6(const cplx<double>* A, int stride, int idx, const cplx<double> v[6],
-                                      cplx<double> o[6]) {
-    herm6<0>(A, stride, idx, 1.0, v, o);
+// o = E v for the numbers e of a block (BLK_A: without the 1)
+template <int BK, class T>
+__device__ __forceinline__ void block_mul(const T e[block_reals(BK)], const cplx<T> v[6], cplx<T> o[6]) {
+    if constexpr (BK == BLK_INV) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) o[i] = e[i] * v[i];
+        int k = 6;
+#pragma unroll
+        for (int i = 1; i < 6; ++i) {
+#pragma unroll
+            for (int j = 0; j < i; ++j) {
+                const cplx<T> a = mk(e[k], e[k + 1]);
+                cfma(o[i], a, v[j]);
+                cfmac(o[j], a, v[i]);
+                k += 2;
+            }
+        }
+    } else if constexpr (BK == BLK_A) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            o[i] = e[i] * v[i];
+            o[3 + i] = -e[i] * v[3 + i];
+        }
+        int k = 3;
+#pragma unroll
+        for (int i = 1; i < 3; ++i) {
+#pragma unroll
+            for (int j = 0; j < i; ++j) {
+                const cplx<T> d = mk(e[k], e[k + 1]), m = mk(-e[k], -e[k + 1]);
+                cfma(o[i], d, v[j]);
+                cfmac(o[j], d, v[i]);
+                cfma(o[3 + i], m, v[3 + j]);
+                cfmac(o[3 + j], m, v[3 + i]);
+                k += 2;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const cplx<T> x = mk(e[k], e[k + 1]);
+                cfma(o[3 + i], x, v[j]);
+                cfmac(o[j], x, v[3 + i]);
+                k += 2;
+            }
+        }
+    } else {
+        int k = 0;
+        if constexpr (BK == BLK_INV_REAL) {
+#pragma unroll
+            for (int i = 0; i < 6; ++i) o[i] = e[i % 3] * v[i];
+            k = 3;
+#pragma unroll
+            for (int i = 1; i < 3; ++i) {
+#pragma unroll
+                for (int j = 0; j < i; ++j) {
+#pragma unroll
+                    for (int s = 0; s < 6; s += 3) {
+                        o[s + i] = axpy1(e[k], v[s + j], o[s + i]);
+                        o[s + j] = axpy1(e[k], v[s + i], o[s + j]);
+                    }
+                    ++k;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 6; ++i) o[i] = mk((T)0, (T)0);
+        }
+#pragma unroll
+        for (int i = 1; i < 3; ++i) {
+#pragma unroll
+            for (int j = 0; j < i; ++j) {
+                ifma(o[i], e[k], v[j]);
+                ifma(o[j], -e[k], v[i]);
+                ifma(o[3 + i], -e[k], v[3 + j]);
+                ifma(o[3 + j], e[k], v[3 + i]);
+                ++k;
+            }
+        }
+#pragma unroll
+        for (int i = 1; i < 3; ++i) {
+#pragma unroll
+            for (int j = 0; j < i; ++j) {
+                const cplx<T> x = mk(e[k], e[k + 1]), m = mk(-e[k], -e[k + 1]);
+                cfma(o[3 + i], x, v[j]);
+                cfma(o[3 + j], m, v[i]);
+                cfmac(o[j], x, v[3 + i]);
+                cfmac(o[i], m, v[3 + j]);
+                k += 2;
+            }
+        }
+    }
+}
+// o = the block times v; FP16: sc is the site's scale, put on the outputs.  The 1 is
+// added last: the sum's roundings are then those of E v (the FP64 clover apply's
+// error 1.9e-16, as with the 1 in the block's diagonal; 2.0e-16 with it first).
+template <int PR, int BK>
+__device__ __forceinline__ void block_apply(const typename Prec<PR>::T e[block_reals(BK)], typename Prec<PR>::T sc,
+                                            const cplx<typename Prec<PR>::T> v[6], cplx<typename Prec<PR>::T> o[6]) {
+    constexpr bool A = block_is_A<BK>;
+    block_mul<BK>(e, v, o);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+        if constexpr (PR == 2) o[i] = A ? axpy1(sc, o[i], v[i]) : sc * o[i];
+        else if constexpr (A) o[i] = v[i] + o[i];
+    }
+}
+template <int PR, int BK, bool NT = true>
+__device__ __forceinline__ void block_apply_at(const void* base, int nplanes, int stride, int plane, int idx,
+                                               typename Prec<PR>::T sc, const cplx<typename Prec<PR>::T> v[6],
+                                               cplx<typename Prec<PR>::T> o[6]) {
+    typename Prec<PR>::T e[block_reals(BK)];
+    load_block<PR, BK, NT>(base, nplanes, stride, plane, idx, e);
+    block_apply<PR, BK>(e, sc, v, o);
 }
 
 }  // namespace lym

@@ -27,9 +27,9 @@ struct DslashParams {
     const void* v2[2];     // optional axpy operand
     const float* v2_sc[2];
     const void* links;
-    const void* A;         // [2][36][stride] clover blocks of D
+    const void* A;         // clover blocks of D, 4 planes
     const float* A_sc;     // [2][stride] (FP16)
-    const void* Ainv;      // [36][stride] inverse blocks (even sites)
+    const void* Ainv;      // inverse blocks (even sites), 2 planes
     const float* Ainv_sc;  // [stride] (FP16)
     double kappa;
     const double* kappa_dev;  // when set, kappa is read from device memory instead
@@ -142,11 +142,17 @@ void launch_links_to_eo(const Geom& g, const void* links_aos, int real_links, in
 
 // ---------------------------------------------------------------- clover (clover.hip)
 void launch_clover_B(const Geom& g, const void* links, int link_kind, zd* B, hipStream_t st);
-void launch_clover_A(const Geom& g, const zd* B, double kc, zd* A, hipStream_t st);
+// real_links: the block kinds of real links
+void launch_clover_A(const Geom& g, const zd* B, double kc, zd* A, bool real_links, hipStream_t st);
 // Ainv on parity 0 from A; returns via *flag (device int) nonzero when a block is singular
-void launch_clover_inv(const Geom& g, const zd* A, zd* Ainv, int* flag, hipStream_t st);  // pivoted; flag: singular count
-void launch_clover_inv_ldl(const Geom& g, const zd* A, zd* Ainv, int* fallback, hipStream_t st);  // unpivoted
-void launch_clover_apply(const Geom& g, const zd* blocks, const zd* in, zd* out, int gamma5, hipStream_t st);
+void launch_clover_inv(const Geom& g, const zd* A, zd* Ainv, bool real_links, int* flag,
+                       hipStream_t st);  // pivoted; flag: singular count
+void launch_clover_inv_ldl(const Geom& g, const zd* A, zd* Ainv, bool real_links, int* fallback,
+                           hipStream_t st);  // unpivoted
+// inverse blocks (lane_set null: set 0 for every lane; else set lane_set[l] at stride
+// set_elems) applied to the even half of lane fields (mask: as for launch_lane_copy)
+void launch_inv_apply(const Geom& g, const zd* blocks, bool real_links, long set_elems, const int* lane_set,
+                      const int* mask, const zd* in, long in_lane, zd* out, long out_lane, int lanes, hipStream_t st);
 
 // ---------------------------------------------------------------- BLAS-1 (blas.hip)
 constexpr int RED_BLOCKS = 512;
@@ -226,7 +232,7 @@ struct MCGState {
 
 // low-precision copies of operator data (mixed.hip); prec 1 FP32, 2 FP16
 void launch_convert_links(int prec, const void* src, void* dst, long n, int real_links, hipStream_t st);
-void launch_convert_blocks(int prec, const zd* src, void* dst, float* sc, int nparity, int stride, hipStream_t st);
+void launch_convert_blocks(int prec, const zd* src, void* dst, float* sc, int kind, int stride, hipStream_t st);
 // rows 0 and 1 of FP64 links [2][4][nc][stride] into the packed low-precision
 // layout of link kinds 1 / 3 (row 2 rebuilt in the stencil)
 void launch_pack_links(int prec, const void* src, int nc, int real_links, void* dst, int stride, hipStream_t st);
@@ -312,10 +318,6 @@ void launch_lane_copy(zd* dst, long dst_lane, const zd* src, long src_lane, long
 void launch_lane_sub(zd* out, const zd* a, const zd* b, long lane, long n, int lanes, const int* mask, hipStream_t st);
 void launch_lane_gather(const zd* const* srcs_dev, zd* dst, long n, int lanes, hipStream_t st);
 void launch_lane_scatter(const zd* src, zd* const* dsts_dev, long n, int lanes, hipStream_t st);
-// blocks (lane_set null: set 0 for every lane; else set lane_set[l] at stride
-// set_elems) applied to the even half of lane fields
-void launch_clover_apply_lanes(const Geom& g, const zd* blocks, long set_elems, const int* lane_set, const int* mask,
-                               const zd* in, long in_lane, zd* out, long out_lane, int lanes, hipStream_t st);
 // single full fields <-> an interleaved FP64 field (rhs fastest)
 void launch_pack(const zd* const* srcs_dev, int nr, zd* multi, long n, hipStream_t st);
 void launch_unpack(const zd* multi, int nr, zd* const* dsts_dev, long n, hipStream_t st);

@@ -278,43 +278,26 @@ __global__ __launch_bounds__(MR_THREADS) void k_link_row2_err(const void* src, i
     }
 }
 
-// blocks [nparity][36][stride] -> PR storage with one scale per site
-// blocks [nparity][36][stride] (FP64) -> the packed low-precision layout of
-// lym_device.h (planes 2 p + block), FP16 with one scale per site
-template <int PR>
+// FP64 blocks of nparity parities -> storage precision PR, FP16 with one scale per site
+template <int PR, int BK>
 __global__ void k_convert_blocks(const zd* src, void* dst, float* sc, int nparity, int stride) {
-    typedef PackedBlock<PR> P;
-    const long ngroup = 2L * nparity * stride;
+    constexpr int N = block_reals(BK);
     SITE_LOOP(j, (long)nparity * stride) {
-        const long p = j / stride, i = j % stride;
-        const zd* s = src + p * 36 * stride + i;
+        const int p = (int)(j / stride), i = (int)(j % stride);
+        double e[2][N];
+        for (int h = 0; h < 2; ++h) load_block<0, BK, false>(src, 2 * nparity, stride, 2 * p + h, i, e[h]);
         float m = 1.f;
         if constexpr (PR == 2) {
             m = 0.f;
-            for (int k = 0; k < 36; ++k) {
-                zd z = s[(long)k * stride];
-                m = fmaxf(m, fmaxf(fabsf((float)z.re), fabsf((float)z.im)));
-            }
+            for (int h = 0; h < 2; ++h)
+                for (int k = 0; k < N; ++k) m = fmaxf(m, fabsf((float)e[h][k]));
         }
         const float inv = fp16_site_inv(m);
         if constexpr (PR == 2) sc[j] = m;
-        for (int blk = 0; blk < 2; ++blk) {
-            typename P::E e[18];
-            for (int k = 0; k < 18; ++k) {
-                zd z = s[(long)(18 * blk + k) * stride];
-                e[k] = from_c<PR>(mk((typename Prec<PR>::T)(inv * z.re), (typename Prec<PR>::T)(inv * z.im)));
-            }
-            unsigned char buf[P::BYTES];
-            __builtin_memcpy(buf, e, P::BYTES);
-            const long el = (2 * p + blk) * stride + i;
-            char* gb = reinterpret_cast<char*>(dst);
-            int off = 0;
-            for (int g = 0; g < P::N16; ++g) {
-                __builtin_memcpy(gb + el * 16, buf + off, 16);
-                off += 16;
-                gb += ngroup * 16;
-            }
-            if constexpr (P::H8) __builtin_memcpy(gb + el * 8, buf + off, 8);
+        for (int h = 0; h < 2; ++h) {
+            float f[N];
+            for (int k = 0; k < N; ++k) f[k] = (float)(inv * e[h][k]);
+            store_block<PR, BK>(dst, 2 * nparity, stride, 2 * p + h, i, f);
         }
     }
 }
@@ -344,12 +327,20 @@ void launch_link_row2_err(const void* src, int real_links, int stride, double* p
     hipLaunchKernelGGL(k_link_row2_err, dim3(RED_BLOCKS), dim3(MR_THREADS), 0, st, src, real_links, stride, partials);
 }
 
-void launch_convert_blocks(int prec, const zd* src, void* dst, float* sc, int nparity, int stride, hipStream_t st) {
-    long n = (long)nparity * stride;
-    if (prec == 1)
-        hipLaunchKernelGGL(k_convert_blocks<1>, dim3(site_blocks(n)), dim3(256), 0, st, src, dst, sc, nparity, stride);
-    else
-        hipLaunchKernelGGL(k_convert_blocks<2>, dim3(site_blocks(n)), dim3(256), 0, st, src, dst, sc, nparity, stride);
+template <int BK>
+static void convert_blocks(int prec, const zd* src, void* dst, float* sc, int stride, hipStream_t st) {
+    const int nparity = block_is_A<BK> ? 2 : 1;
+    const dim3 nb(site_blocks((long)nparity * stride)), th(256);
+    if (prec == 1) hipLaunchKernelGGL((k_convert_blocks<1, BK>), nb, th, 0, st, src, dst, sc, nparity, stride);
+    else hipLaunchKernelGGL((k_convert_blocks<2, BK>), nb, th, 0, st, src, dst, sc, nparity, stride);
+}
+void launch_convert_blocks(int prec, const zd* src, void* dst, float* sc, int kind, int stride, hipStream_t st) {
+    switch (kind) {
+        case BLK_A: convert_blocks<BLK_A>(prec, src, dst, sc, stride, st); break;
+        case BLK_A_REAL: convert_blocks<BLK_A_REAL>(prec, src, dst, sc, stride, st); break;
+        case BLK_INV_REAL: convert_blocks<BLK_INV_REAL>(prec, src, dst, sc, stride, st); break;
+        default: convert_blocks<BLK_INV>(prec, src, dst, sc, stride, st); break;
+    }
 }
 
 // ---------------------------------------------------------------- spinor precision conversion

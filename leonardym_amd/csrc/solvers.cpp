@@ -1336,7 +1336,8 @@ int lym_solver_solve(lym_solver* s, lym_op* op, const lym_spinor* source, lym_sp
         zd* rhs = s->w[7] + half_n(c);
         zd* src = s->w[1];
         zd* xo = par(x, c, 1);
-        lym::launch_clover_apply(c->g, reinterpret_cast<const zd*>(op->Ainv), par(b, c, 0), te, 0, st);
+        lym::launch_inv_apply(c->g, reinterpret_cast<const zd*>(op->Ainv), op->gauge->real_links, 0, nullptr, nullptr,
+                              par(b, c, 0), 0, te, 0, 1, st);
         std::memset(&a, 0, sizeof(a));
         a.g = c->g;
         a.links = op->gauge->U;
