@@ -158,18 +158,17 @@ void free_sloppy(lym_op* op) {
 }
 
 // all three rows of 18-real (9-real) links in low precision, for multi-RHS
-// applies: there the NR lanes of a site would each rebuild row 2 of the same
-// link, and the batched stencil is bound by arithmetic, not bandwidth
+// applies (rounded once; a rebuilt row carries the roundings of rows 0 and 1, and
+// the NR lanes of a site would each rebuild it)
 int op_sloppy_full_rows(lym_op* op, int prec) {
     lym_ctx* c = op->ctx;
     const lym_gauge* g = op->gauge;
     const int ncomp = g->real_links ? g->compression : g->compression / 2;
     if (!g->rows_rebuild || ncomp != 9 || op->Usf) return LYM_OK;  // Us already has every row, or Usf is current
     const long S = c->g.stride;
-    const size_t le = g->real_links ? (prec == 1 ? 4 : 2) : (prec == 1 ? 8 : 4);
-    int rc = dmalloc(c, &op->Usf, 2L * 4 * 9 * S * le);
+    int rc = dmalloc(c, &op->Usf, 8L * S * lym::link_bytes(prec, g->real_links, 3));
     if (rc) return rc;
-    lym::launch_convert_links(prec, g->U, op->Usf, 2L * 4 * 9 * S, g->real_links, c->stream);
+    lym::launch_pack_links(prec, g->U, 9, 3, g->real_links, op->Usf, (int)S, c->stream);
     CHECK_LAUNCH();
     return LYM_OK;
 }
@@ -186,23 +185,22 @@ int op_sloppy_data(lym_op* op, int prec, bool full_rows) {
     const lym_gauge* g = op->gauge;
     const long S = c->g.stride;
     const int ncomp = g->real_links ? g->compression : g->compression / 2;
-    const long nl = 2L * 4 * ncomp * S;
-    const size_t le = g->real_links ? (prec == 1 ? 4 : 2) : (prec == 1 ? 8 : 4);
     int rc = LYM_OK;
-    if (!op->Us) rc = dmalloc(c, &op->Us, 2L * 4 * 9 * S * le);  // room for 18-real links
+    // room for three rows
+    if (!op->Us) rc = dmalloc(c, &op->Us, 8L * S * lym::link_bytes(prec, g->real_links, 3));
     if (rc) return rc;
     op->sloppy_alloc = prec;
     if (g->rows_rebuild) {
-        // rows 0 and 1 in 16/8/4-byte vectors, row 2 rebuilt in the stencil
-        lym::launch_pack_links(prec, g->U, ncomp, g->real_links, op->Us, (int)S, c->stream);
+        // rows 0 and 1, row 2 rebuilt in the stencil
+        lym::launch_pack_links(prec, g->U, ncomp, 2, g->real_links, op->Us, (int)S, c->stream);
         op->sloppy_lk = g->real_links ? 3 : 1;
     } else {
-        lym::launch_convert_links(prec, g->U, op->Us, nl, g->real_links, c->stream);
+        lym::launch_pack_links(prec, g->U, 9, 3, g->real_links, op->Us, (int)S, c->stream);
         op->sloppy_lk = link_kind(g);
     }
     if (op->Usf) {
         if (g->rows_rebuild && ncomp == 9) {
-            lym::launch_convert_links(prec, g->U, op->Usf, nl, g->real_links, c->stream);
+            lym::launch_pack_links(prec, g->U, 9, 3, g->real_links, op->Usf, (int)S, c->stream);
         } else {
             // the new gauge field's Us already serves batches (compressed
             // storage, or rows not rebuilt): a stale full-row copy must not be used

@@ -700,9 +700,16 @@ struct MfmaLane {
     bool aval;          // A row < 12 and k-group < 3: this lane loads A
     int arow, aore;     // A row: 0 direct, 1 partner; 0 real row, 1 imaginary row
     bool partP[2];      // A/B k slot s: colour block of the partner spin (else of spin h)
-    unsigned lofs_f[2], lofs_b[2];  // link entry of slot s (in units of the link component stride)
+    // link entry of slot s of link li: entry (li << lsh) + lofs of the packed field
+    unsigned lofs_f[2], lofs_b[2], lsh_f[2], lsh_b[2];
     int kgrp;           // k-group l / 16
 };
+
+// entry k of a packed FP16 link: vectors of entries 0-3 and 4-7, then entry 8
+__device__ __forceinline__ void mfma_entry(int stride, int k, unsigned& ofs, unsigned& sh) {
+    ofs = k < 8 ? (unsigned)(k >> 2) * 32u * (unsigned)stride + (k & 3) : 64u * (unsigned)stride;
+    sh = k < 8 ? 2 : 0;
+}
 
 template <int MU>
 __device__ __forceinline__ int mfma_phase(const MfmaLane& L, int s, bool fwd) {
@@ -722,13 +729,15 @@ template <int MU, bool FWD>
 __device__ __forceinline__ void mfma_load(const DslashParams& a, const MfmaLane& L, int lp, int lsite, int q, int nb,
                                           const unsigned sofs[2], bool use_b, hv4& Av, hv4& Bv, float& sc) {
     const int ST = a.g.stride;
-    const h2_t* lb = reinterpret_cast<const h2_t*>(a.links) + (size_t)((lp * 4 + MU) * 9) * ST + lsite;
+    const unsigned li = (unsigned)((lp * 4 + MU) * ST + lsite);  // the packed link: entries 0-3, 4-7, 8
+    const h2_t* lb = reinterpret_cast<const h2_t*>(a.links);
     const h2_t* sb = reinterpret_cast<const h2_t*>(a.in[q]) + (size_t)nb * a.nr * 4;
     constexpr bool SIGN1 = Dir<MU>::C1 != Dir<MU>::C0;  // c_1 = -c_0
     const _Float16 hz = (_Float16)0;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-        h2_t z = fld<h2_t>(lb, L.aval ? (FWD ? L.lofs_f[s] : L.lofs_b[s]) : 0u);
+        const unsigned lo = FWD ? L.lofs_f[s] : L.lofs_b[s], sh = FWD ? L.lsh_f[s] : L.lsh_b[s];
+        h2_t z = fld<h2_t>(lb, L.aval ? (li << sh) + lo : 0u);
         if (!FWD) z.y = -z.y;
         z = mul_ip(z, mfma_phase<MU>(L, s, FWD));
         Av[2 * s] = L.aval ? (L.aore ? z.y : z.x) : hz;
@@ -786,8 +795,8 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) void k_dslash_mfma(DslashParams
             const int idx = 2 * L.kgrp + s;  // 0..5: (spin h, colour 0..2), then (partner, colour 0..2)
             const int j = idx % 3;
             L.partP[s] = idx >= 3;
-            L.lofs_f[s] = (unsigned)((3 * ai + j) * a.g.stride);
-            L.lofs_b[s] = (unsigned)((3 * j + ai) * a.g.stride);
+            mfma_entry(a.g.stride, 3 * ai + j, L.lofs_f[s], L.lsh_f[s]);
+            mfma_entry(a.g.stride, 3 * j + ai, L.lofs_b[s], L.lsh_b[s]);
         }
     }
     // B offsets (h2 elements from the neighbour's base) per direction and slot
@@ -929,8 +938,10 @@ static void launch_one(const DslashParams& a, int nblocks, hipStream_t st) {
 template <int PR, int LK, int DIAG, bool INV>
 static void launch_lp(const DslashParams& a, int nblocks, hipStream_t st) {
     if constexpr (PR == 2 && LK == 0) {
-        // matrix-core form: FP16 SU(3) batches of 2, 4 or 8 RHS in whole waves
-        if (a.mfma && !a.bmode && (a.nr == 2 || a.nr == 4 || a.nr == 8) && (a.spb * a.nr) % 64 == 0) {
+        // matrix-core form: FP16 SU(3) batches of 2, 4 or 8 RHS in whole waves (its
+        // lanes address the links by 32-bit byte offsets)
+        if (a.mfma && !a.bmode && 8L * a.g.stride * link_bytes(2, false, 3) < (1L << 32) &&
+            (a.nr == 2 || a.nr == 4 || a.nr == 8) && (a.spb * a.nr) % 64 == 0) {
             if (a.lane_ops)
                 hipLaunchKernelGGL((k_dslash_mfma<DIAG, INV, true>), dim3(nblocks), dim3(a.spb * a.nr), 0, st, a);
             else

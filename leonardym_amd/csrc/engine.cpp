@@ -343,7 +343,6 @@ size_t engine_bytes(const int dims[4], int rep, int storage, int prec, int wmax)
     const double V = (double)dims[0] * dims[1] * dims[2] * dims[3];
     const double S = std::ceil(V / 2 / 64) * 64;
     const double es = prec == LYM_PREC_SINGLE ? 8 : 4;
-    const double le = rep == LYM_REP_SU2_ADJ ? es / 2 : es;
     (void)storage;
     const double W = next_width(wmax);
     double b = 0;
@@ -354,7 +353,7 @@ size_t engine_bytes(const int dims[4], int rep, int storage, int prec, int wmax)
     const int ki = rep == LYM_REP_SU2_ADJ ? lym::BLK_INV_REAL : lym::BLK_INV, pr = prec == LYM_PREC_SINGLE ? 1 : 2;
     b += W * S * (4 * (lym::block_bytes(0, ka) + lym::block_bytes(pr, ka)) +
                   2 * (lym::block_bytes(0, ki) + lym::block_bytes(pr, ki)) + 12);  // operator data per lane
-    b += 72 * S * le;                                // low-precision links
+    b += 8 * S * lym::link_bytes(pr, rep == LYM_REP_SU2_ADJ, 3);                                // low-precision links
     b += 2 * W * 24 * S * 16 + 12 * V * 16;          // transfer spinors, context staging
     return (size_t)(b * 1.03) + (32u << 20);
 }
@@ -405,8 +404,7 @@ int engine_create(lym_ctx* ctx, const lym_gauge* g, double csw, int prec, unsign
     A((void**)&e->Ainvs_sc, sizeof(float) * S * W);
     // low-precision links: all three rows when the FP64 field has them
     // (every lane would otherwise rebuild row 2 of the same link)
-    const size_t le = g->real_links ? e->es / 2 : e->es;
-    A(&e->Us, 72 * S * le);
+    A(&e->Us, 8 * S * lym::link_bytes(e->prec, g->real_links, 3));
     for (zd** f : {&e->B, &e->X}) A((void**)f, sizeof(zd) * 24 * S * W);
     for (zd** f : {&e->x, &e->r, &e->Ax, &e->mid, &e->tmp, &e->rhs, &e->src, &e->te})
         A((void**)f, sizeof(zd) * 12 * S * W);
@@ -449,11 +447,11 @@ int engine_create(lym_ctx* ctx, const lym_gauge* g, double csw, int prec, unsign
     if (!rc) {
         const int ncomp = g->real_links ? g->compression : g->compression / 2;
         if (full_rows(g)) {
-            lym::launch_convert_links(prec, g->U, e->Us, 2L * 4 * ncomp * S, g->real_links, ctx->stream);
+            lym::launch_pack_links(prec, g->U, 9, 3, g->real_links, e->Us, (int)S, ctx->stream);
             e->lks = e->lk64;
         } else {
             // 12/6-real storage: rows 0 and 1 packed, row 2 rebuilt in the stencil
-            lym::launch_pack_links(prec, g->U, ncomp, g->real_links, e->Us, (int)S, ctx->stream);
+            lym::launch_pack_links(prec, g->U, ncomp, 2, g->real_links, e->Us, (int)S, ctx->stream);
             e->lks = g->real_links ? 3 : 1;
         }
         if (hipGetLastError() != hipSuccess) rc = fail(LYM_ERR_DEVICE, "link conversion");

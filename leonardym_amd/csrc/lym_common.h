@@ -38,6 +38,10 @@ __host__ __device__ constexpr int block_reals(int kind) {
 __host__ __device__ constexpr int block_bytes(int prec, int kind) {
     return prec == 0 ? 8 * block_reals(kind) : prec == 1 ? 4 * block_reals(kind) : (2 * block_reals(kind) + 3) / 4 * 4;
 }
+// bytes of a low-precision link (precision 1 or 2) of 2 or 3 rows
+__host__ __device__ constexpr int link_bytes(int prec, bool real, int rows) {
+    return (3 * rows * (real ? 1 : 2) * (prec == 1 ? 4 : 2) + 3) / 4 * 4;
+}
 
 // Device site order.  0: t fastest (the reference's lexicographic order; the
 // even-odd split needs Lt even).  1: t slowest, x fastest (needs Lx even): the

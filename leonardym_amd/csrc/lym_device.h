@@ -418,26 +418,34 @@ __device__ __forceinline__ void store_half_lp(typename Prec<PR>::S* pbase, size_
 }
 
 // ---------------------------------------------------------------- packed low-precision links
-// FP32/FP16 links of kinds 1 and 3 hold rows 0 and 1 only (6 entries; row 2 is
-// rebuilt: conj(row0 x row1) for SU(3), row0 x row1 for the real adjoint
-// links), packed into 16-, 8- and 4-byte vectors.  Group g of the field is an
+// FP32/FP16 links, rows 0 and 1 (kinds 1 and 3; row 2 is rebuilt: conj(row0 x row1)
+// for SU(3), row0 x row1 for the real adjoint links) or all three (kinds 0 and 2),
+// packed into 16-, 8- and 4-byte vectors.  Group g of the field is an
 // array [2 parity][4 mu][stride] of vectors of its size; the groups follow
-// one another.  Bytes per link: FP32 complex 48 (16+16+16), FP16 complex 24
-// (16+8), FP32 real 24 (16+8), FP16 real 12 (8+4).
-template <int PR, bool REAL>
+// one another.  Bytes per link of two rows: FP32 complex 48 (16+16+16), FP16 complex
+// 24 (16+8), FP32 real 24 (16+8), FP16 real 12 (8+4); of three: 72 (4 x 16 + 8), 36
+// (16+16+4), 36 (16+16+4), 20 (16+4, the last 2 unused).
+// Three rows as 9 single entries took 9 loads a link (72 a site), which the batched
+// launches, whose lanes share the links, spent much of their time issuing: the clover
+// Schur launches of 8 right-hand sides on 32^3x64 went from 488 to 450 us at FP16 and
+// from 1090 to 970 at FP32, on 24^3x48 adjoint links from 150 to 124 at FP16.  (Two
+// rows and the rebuild: 456 and 856; the batches keep all rows, which are the FP64
+// links rounded once.)
+template <int PR, bool REAL, int ROWS>
 struct PackedLink {
     static_assert(PR >= 1, "packed links are low-precision only");
     typedef typename std::conditional<REAL, typename Prec<PR>::R, typename Prec<PR>::S>::type E;
-    static constexpr int BYTES = 6 * (int)sizeof(E);
+    static constexpr int BYTES = link_bytes(PR, REAL, ROWS);
+    static constexpr int NE = BYTES / (int)sizeof(E);  // 3 ROWS and the padding
     static constexpr int N16 = BYTES / 16;
     static constexpr bool H8 = (BYTES - 16 * N16) >= 8;
     static constexpr bool H4 = (BYTES - 16 * N16) % 8 == 4;
 };
 
-template <int PR, bool REAL>
+template <int PR, bool REAL, int ROWS>
 __device__ __forceinline__ void load_link_rows(const void* base, int stride, int p, int mu, int idx,
-                                               typename PackedLink<PR, REAL>::E e[6]) {
-    typedef PackedLink<PR, REAL> P;
+                                               typename PackedLink<PR, REAL, ROWS>::E e[3 * ROWS]) {
+    typedef PackedLink<PR, REAL, ROWS> P;
     const char* gb = reinterpret_cast<const char*>(base);
     const size_t plane = (size_t)(p * 4 + mu) * stride;
     unsigned char buf[P::BYTES];
@@ -459,7 +467,7 @@ __device__ __forceinline__ void load_link_rows(const void* base, int stride, int
         unsigned v = fld<unsigned, LYM_NT_LINKS != 0>(reinterpret_cast<const unsigned*>(gb) + plane, (unsigned)idx);
         __builtin_memcpy(buf + off, &v, 4);
     }
-    __builtin_memcpy(e, buf, P::BYTES);
+    __builtin_memcpy(e, buf, 3 * ROWS * sizeof(typename P::E));
 }
 
 // row 2 from rows 0 and 1: conj(row0 x row1), for real links row0 x row1
@@ -486,20 +494,17 @@ template <int PR, int LK>
 __device__ __forceinline__ void load_link(const void* base, int stride, int p, int mu, int idx,
                                           LinkMat<LK, typename Prec<PR>::T>& L) {
     typedef typename Prec<PR>::T T;
-    if constexpr (PR >= 1 && (LK == 1 || LK == 3)) {
-        constexpr bool REAL = LK == 3;
-        typename PackedLink<PR, REAL>::E e[6];
-        load_link_rows<PR, REAL>(base, stride, p, mu, idx, e);
+    if constexpr (PR >= 1) {
+        constexpr bool REAL = LK >= 2;
+        constexpr int ROWS = LK & 1 ? 2 : 3;
+        typename PackedLink<PR, REAL, ROWS>::E e[3 * ROWS];
+        load_link_rows<PR, REAL, ROWS>(base, stride, p, mu, idx, e);
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
+        for (int k = 0; k < 3 * ROWS; ++k) {
             if constexpr (REAL) L.m[k] = (T)e[k];
             else L.m[k] = to_c<PR>(e[k]);
         }
-        if constexpr (REAL) {
-            rebuild_row2(L.m);
-        } else {
-            rebuild_row2(L.m);
-        }
+        if constexpr (ROWS == 2) rebuild_row2(L.m);
     } else if constexpr (LK == 0 || LK == 1) {
         constexpr int NC = (LK == 0) ? 9 : 6;
         const typename Prec<PR>::S* b =

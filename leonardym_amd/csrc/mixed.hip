@@ -191,32 +191,18 @@ __device__ __forceinline__ void d_store(zd* v, int stride, long j, const zd s[12
 }
 
 // ---------------------------------------------------------------- operator data conversion
-template <int PR>
-__global__ void k_convert_links(const void* src, void* dst, long n, int real_links) {
-    SITE_LOOP(i, n) {
-        if (real_links) {
-            reinterpret_cast<typename Prec<PR>::R*>(dst)[i] =
-                (typename Prec<PR>::R)reinterpret_cast<const double*>(src)[i];
-        } else {
-            zd z = reinterpret_cast<const zd*>(src)[i];
-            reinterpret_cast<typename Prec<PR>::S*>(dst)[i] =
-                from_c<PR>(mk((typename Prec<PR>::T)z.re, (typename Prec<PR>::T)z.im));
-        }
-    }
-}
-
 // FP64 links [2][4][nc][stride] (nc = 9 or 6; entries 0..5 are rows 0 and 1)
-// -> rows 0, 1 in the packed low-precision layout (lym_device.h)
-template <int PR, bool REAL>
+// -> ROWS rows in the packed low-precision layout (lym_device.h)
+template <int PR, bool REAL, int ROWS>
 __global__ void k_pack_links(const void* src, int nc, void* dst, int stride) {
-    typedef PackedLink<PR, REAL> P;
+    typedef PackedLink<PR, REAL, ROWS> P;
     typedef typename P::E E;
     const long n = 8L * stride;
     SITE_LOOP(j, n) {
         const long plane = j / stride, i = j % stride;
-        E e[6];
+        E e[P::NE] = {};
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
+        for (int k = 0; k < 3 * ROWS; ++k) {
             const long o = (plane * nc + k) * stride + i;
             if constexpr (REAL) e[k] = (E)reinterpret_cast<const double*>(src)[o];
             else {
@@ -307,19 +293,20 @@ static inline int site_blocks(long n) {
     return (int)(b < 4096 ? b : 4096);
 }
 
-void launch_convert_links(int prec, const void* src, void* dst, long n, int real_links, hipStream_t st) {
-    if (prec == 1) hipLaunchKernelGGL(k_convert_links<1>, dim3(site_blocks(n)), dim3(256), 0, st, src, dst, n, real_links);
-    else hipLaunchKernelGGL(k_convert_links<2>, dim3(site_blocks(n)), dim3(256), 0, st, src, dst, n, real_links);
+template <int PR, bool REAL>
+static void pack_links(const void* src, int nc, int rows, void* dst, int stride, hipStream_t st) {
+    const dim3 nb(site_blocks(8L * stride)), th(256);
+    if (rows == 3) hipLaunchKernelGGL((k_pack_links<PR, REAL, 3>), nb, th, 0, st, src, nc, dst, stride);
+    else hipLaunchKernelGGL((k_pack_links<PR, REAL, 2>), nb, th, 0, st, src, nc, dst, stride);
 }
-
-void launch_pack_links(int prec, const void* src, int nc, int real_links, void* dst, int stride, hipStream_t st) {
-    const long n = 8L * stride;
+void launch_pack_links(int prec, const void* src, int nc, int rows, int real_links, void* dst, int stride,
+                       hipStream_t st) {
     if (prec == 1) {
-        if (real_links) hipLaunchKernelGGL((k_pack_links<1, true>), dim3(site_blocks(n)), dim3(256), 0, st, src, nc, dst, stride);
-        else hipLaunchKernelGGL((k_pack_links<1, false>), dim3(site_blocks(n)), dim3(256), 0, st, src, nc, dst, stride);
+        if (real_links) pack_links<1, true>(src, nc, rows, dst, stride, st);
+        else pack_links<1, false>(src, nc, rows, dst, stride, st);
     } else {
-        if (real_links) hipLaunchKernelGGL((k_pack_links<2, true>), dim3(site_blocks(n)), dim3(256), 0, st, src, nc, dst, stride);
-        else hipLaunchKernelGGL((k_pack_links<2, false>), dim3(site_blocks(n)), dim3(256), 0, st, src, nc, dst, stride);
+        if (real_links) pack_links<2, true>(src, nc, rows, dst, stride, st);
+        else pack_links<2, false>(src, nc, rows, dst, stride, st);
     }
 }
 
