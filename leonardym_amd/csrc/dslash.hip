@@ -26,9 +26,14 @@
 #endif
 // both parities of a block range run on the same XCD (links and spinors of a
 // region are then fetched into one L2 for the even and the odd sites)
-// -1: automatic -- one sweeping workgroup per CU for launches of at most
-// LYM_SWEEP_MAX_BLOCKS workgroups (small lattices, where it was ~4 % faster),
-// all workgroups at once above that (large lattices, where sweeping was slower)
+// -1: automatic -- one sweeping workgroup per CU for FP64 launches and FP32 ones of
+// two threads per site of at most LYM_SWEEP_MAX_BLOCKS workgroups (small lattices:
+// 16^3x32 FP64 clover 38.1 us, 42.1 with all workgroups at once; FP32 21.5, 22.7),
+// all workgroups at once above that (large lattices, where sweeping was slower) and
+// for the others, whose waves are smaller and wait longer for what they load: one
+// workgroup per CU leaves them one wave per SIMD (16^3x32 FP16 two threads per
+// site 17.1 us swept, 14.8 at once; Schur complement of 3 and 4 right-hand sides
+// 69.5 and 73.4, 44.7 and 45.3 at once; FP32 78.9, 72.3 at once)
 #ifndef LYM_GRID_PER_CU
 #define LYM_GRID_PER_CU -1
 #endif
@@ -1052,23 +1057,26 @@ static int plan_dslash(DslashParams& a) {
     }
     int nblocks = a.nblocks_per_parity * (a.parity >= 0 ? 1 : 2);
     // workgroups in flight: LYM_GRID_PER_CU per CU of the 256 CUs, sweeping
-    const int gpc = LYM_GRID_PER_CU >= 0 ? LYM_GRID_PER_CU : (nblocks <= LYM_SWEEP_MAX_BLOCKS ? 1 : 0);
+    const bool sweep = (a.prec == 0 || (a.prec == 1 && a.split)) && nblocks <= LYM_SWEEP_MAX_BLOCKS;
+    const int gpc = LYM_GRID_PER_CU >= 0 ? LYM_GRID_PER_CU : (sweep ? 1 : 0);
     if (gpc > 0 && nblocks > 256 * gpc) nblocks = 256 * gpc;
     return nblocks;
 }
 
 // Launches of at most this many (site, RHS) lanes take the one-wave-per-direction
-// form (dslash_hop.hip).  Measured, that form against the other: half-lattice
-// launches, time of an FP64 even-odd CG / FP16 mixed CG iteration: 83 against
-// 91 us / 48 against 57 us at 32768 lanes, 147 against 141 us / 78 against 67 us
-// at 65536; batched FP16 solves of 4 RHS 5.9 against 7.0 ms at 41472 lanes, 10.9
-// against 9.9 ms at 131072.  Full-lattice FP64 applies: 10.2 against 13.6 us at
-// 20736 lanes (clover), 14.3 against 12.5 us at 41472 (Wilson).
-#ifndef LYM_HOP_MAX_HALF
-#define LYM_HOP_MAX_HALF 49152
+// form (dslash_hop.hip); low-precision launches of one parity, whose other form
+// waits longest, more of them.  Measured, that form against the other: FP64 even-odd
+// CG iteration 83 against 91 us at 32768 lanes, Schur complement 39.0 against 38.4 at
+// 40960 and 43.0 against 41.9 at 49152; full applies 10.2 against 13.6 us at 20736
+// lanes (clover), 14.3 against 12.5 us at 41472 (Wilson).  Low-precision Schur
+// complement at 41472 lanes of two RHS 14.2 against 21.9 us (FP16), 18.8 against 22.5
+// (FP32), at 49152 lanes of one 17.7 against 19.6 and 23.3 against 25.7; FP16 mixed CG
+// iteration 78 against 67 us at 65536.
+#ifndef LYM_HOP_MAX
+#define LYM_HOP_MAX 32768
 #endif
-#ifndef LYM_HOP_MAX_FULL
-#define LYM_HOP_MAX_FULL 32768
+#ifndef LYM_HOP_MAX_LOWP_HALF
+#define LYM_HOP_MAX_LOWP_HALF 49152
 #endif
 
 // The launch geometry of that form: sites per workgroup and site blocks per
@@ -1076,7 +1084,7 @@ static int plan_dslash(DslashParams& a) {
 static int plan_hop(DslashParams& a) {
     const int par = a.parity >= 0 ? 1 : 2;
     const long lanes = (long)a.g.Vh * a.nr * par;
-    if (LYM_T_SLOW || a.mfma || a.nr > 64 || lanes > (par == 1 ? LYM_HOP_MAX_HALF : LYM_HOP_MAX_FULL)) return 0;
+    if (LYM_T_SLOW || a.mfma || a.nr > 64 || lanes > (par == 1 && a.prec ? LYM_HOP_MAX_LOWP_HALF : LYM_HOP_MAX)) return 0;
     a.spb = 64 / a.nr;
     // tiny launches: fewer sites per workgroup, so that more CUs share the loads
     while (a.spb > 1 && a.spb * a.nr > 16 && (a.g.Vh + a.spb - 1) / a.spb * par < 256) a.spb = (a.spb + 1) / 2;
