@@ -35,23 +35,47 @@ __device__ __forceinline__ void chunk_store(double v, double* partials, long nch
     if (sl == 0) partials[(long)q * nchunks + blockIdx.x] = red[q * BC];
 }
 
-// final per-RHS sums (valid in thread 0), one FT-thread block
+// final per-RHS sums into tot (shared, valid after the call), one FT-thread block.
+// Thread t sums the chunks t, t + FT, ...; the tree over the FT sums pairs t with
+// t + 512, then 256, ... 1.  All lanes (in groups of FG) load at once, and wave q of
+// the block runs lane q's tree, the steps down to 64 in registers and the rest by
+// shuffles (one lane after the other, with a barrier a step, 8 lanes of 16384 chunks
+// took 45 us and 4 lanes of small lattices 8 to 11, now below 10 and 3.5 to 4).
+constexpr int FG = 8;
 template <int NR>
-__device__ __forceinline__ void final_sums(const double* partials, long nchunks, double out[NR]) {
-    __shared__ double sh[FT];
-    for (int q = 0; q < NR; ++q) {
-        double v = 0;
-        for (long c = threadIdx.x; c < nchunks; c += FT) v += partials[(long)q * nchunks + c];
-        sh[threadIdx.x] = v;
-        __syncthreads();
+__device__ __forceinline__ void final_sums(const double* partials, long nchunks, double* tot) {
+    constexpr int G = NR < FG ? NR : FG;
+    __shared__ double sh[G * FT];
+    const int t = threadIdx.x, w = t >> 6, l = t & 63;
 #pragma unroll
-        for (int off = FT / 2; off > 0; off >>= 1) {
-            if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-            __syncthreads();
+    for (int q0 = 0; q0 < NR; q0 += G) {
+        double v[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) v[g] = 0;
+        for (long c = t; c < nchunks; c += FT) {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                if (q0 + g < NR) v[g] += partials[(long)(q0 + g) * nchunks + c];
         }
-        if (threadIdx.x == 0) out[q] = sh[0];
+        if (q0) __syncthreads();  // the trees of the group before have read sh
+#pragma unroll
+        for (int g = 0; g < G; ++g) sh[g * FT + t] = v[g];
         __syncthreads();
+        if (w < G && q0 + w < NR) {
+            double u[FT / 64];
+#pragma unroll
+            for (int m = 0; m < FT / 64; ++m) u[m] = sh[w * FT + l + 64 * m];
+#pragma unroll
+            for (int off = FT / 128; off > 0; off >>= 1) {
+#pragma unroll
+                for (int m = 0; m < off; ++m) u[m] += u[m + off];
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) u[0] += __shfl_down(u[0], off);
+            if (l == 0) tot[q0 + w] = u[0];
+        }
     }
+    __syncthreads();
 }
 
 #define BSITE_LOOP(j, n) for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < (n); j += (long)gridDim.x * blockDim.x)
@@ -178,30 +202,26 @@ __global__ __launch_bounds__(BC * NR) void k_bcg_init(const zd* r, cplx<float>* 
 template <int NR>
 __global__ __launch_bounds__(FT) void k_bcg_init_final(BState* s, const double* partials, long nchunks,
                                                        int max_steps, const int* mask) {
-    double out[NR];
-    final_sums<NR>(partials, nchunks, out);
-    if (threadIdx.x == 0) {
-        int all = 1;
-        for (int q = 0; q < NR; ++q) {
-            if (mask && !mask[q]) {  // a lane that keeps its state
-                all = all && s->done[q];
-                continue;
-            }
-            s->rr_s[q] = s->rr_true[q] = s->maxrr[q] = out[q];
-            s->step[q] = 0;
-            s->nrel[q] = 0;
-            s->rel[q] = 0;
-            s->alpha[q] = s->beta[q] = 0;
-            // a zero source has the solution x = x0 = 0: nothing to iterate
-            s->conv[q] = out[q] == 0.0 ? 1 : 0;
-            s->done[q] = (max_steps <= 0 || out[q] == 0.0) ? 1 : 0;
-            all = all && s->done[q];
-        }
+    __shared__ double tot[NR];
+    final_sums<NR>(partials, nchunks, tot);
+    const int q = threadIdx.x;
+    if (q >= 64) return;
+    const bool on = q < NR;
+    if (on && !(mask && !mask[q])) {  // else a lane that keeps its state
+        s->rr_s[q] = s->rr_true[q] = s->maxrr[q] = tot[q];
+        s->step[q] = 0;
+        s->nrel[q] = 0;
+        s->rel[q] = 0;
+        s->alpha[q] = s->beta[q] = 0;
+        // a zero source has the solution x = x0 = 0: nothing to iterate
+        s->conv[q] = tot[q] == 0.0 ? 1 : 0;
+        s->done[q] = (max_steps <= 0 || tot[q] == 0.0) ? 1 : 0;
+    }
+    // a lane that keeps its state may hold an update due at the next slot
+    const int any = __any(on && s->rel[q] && !s->done[q]), all = __all(!on || s->done[q]);
+    if (q == 0) {
         s->max_steps = max_steps;
         s->all_done = all;
-        // a lane that keeps its state may hold an update due at the next slot
-        int any = 0;
-        for (int q = 0; q < NR; ++q) any = any || (s->rel[q] && !s->done[q]);
         s->any_rel = any;
         s->skip_rel = any ? 0 : 1;
     }
@@ -230,25 +250,56 @@ __global__ __launch_bounds__(BC * NR) void k_bcg_dot(const BState* s, const type
 // (bsite[j * NR + q]); lanes that are done contribute zero, as in k_bcg_dot.
 // Only the vh real sites of each parity count: the stencil never writes the
 // padding slots up to the stride, which may hold values a wider batch left.
+// Widths of a power of two: a wave per chunk, its BC sites x NR lanes in NR registers
+// a thread (value 64 m + l of the chunk in register m of lane l), the tree's steps
+// (pairs of sites 32, 16, ... 1 apart) first between registers, then by shuffles, in
+// the same order as chunk_store.  A block of BC x NR threads with a barrier a step
+// read 1.5 TB/s (45 us for 8 lanes of 32^3x64, now 14).
+constexpr int CHUNK_WAVES = 4;
 template <int NR>
-__global__ __launch_bounds__(BC * NR) void k_bcg_chunksum(const BState* s, const double* bsite, long nsites,
-                                                          int stride, int vh, double* partials, long nchunks) {
+constexpr bool chunk_wave = (NR & (NR - 1)) == 0;
+template <int NR>
+__global__ __launch_bounds__(chunk_wave<NR> ? 64 * CHUNK_WAVES : BC * NR) void k_bcg_chunksum(
+    const BState* s, const double* bsite, long nsites, int stride, int vh, double* partials, long nchunks) {
     if (s->all_done) return;
-    long j;
-    int q;
-    double v = 0;
-    if (chunk_pair<NR>(nsites, j, q) && !s->done[q] && j % stride < vh) v = bsite[j * NR + q];
-    chunk_store<NR>(v, partials, nchunks);
+    if constexpr (chunk_wave<NR>) {
+        const int l = threadIdx.x & 63;
+        const long c = (long)blockIdx.x * CHUNK_WAVES + (threadIdx.x >> 6), j0 = c * BC;
+        if (c >= nchunks) return;
+        const bool on = !s->done[l % NR];
+        const int i0 = (int)(j0 % stride);  // a chunk lies within one parity (the stride is a multiple of BC)
+        double v[NR];
+#pragma unroll
+        for (int m = 0; m < NR; ++m) {
+            const int sl = (64 * m + l) / NR;
+            v[m] = on && j0 + sl < nsites && i0 + sl < vh ? bsite[j0 * NR + 64 * m + l] : 0.0;
+        }
+#pragma unroll
+        for (int off = NR / 2; off > 0; off >>= 1) {
+#pragma unroll
+            for (int m = 0; m < off; ++m) v[m] += v[m + off];
+        }
+#pragma unroll
+        for (int off = 32; off >= NR; off >>= 1) v[0] += __shfl_down(v[0], off);
+        if (l < NR) partials[(long)l * nchunks + c] = v[0];
+    } else {
+        long j;
+        int q;
+        double v = 0;
+        if (chunk_pair<NR>(nsites, j, q) && !s->done[q] && j % stride < vh) v = bsite[j * NR + q];
+        chunk_store<NR>(v, partials, nchunks);
+    }
 }
 
 template <int NR>
 __global__ __launch_bounds__(FT) void k_bcg_alpha_final(BState* s, const double* partials, long nchunks) {
     if (s->all_done) return;
-    double out[NR];
-    final_sums<NR>(partials, nchunks, out);
-    if (threadIdx.x == 0)
-        for (int q = 0; q < NR; ++q)
-            if (!s->done[q]) s->alpha[q] = s->rr_s[q] / out[q];
+    __shared__ double tot[NR];
+    const int q = threadIdx.x < NR ? threadIdx.x : 0;
+    const double rr = s->rr_s[q];
+    const int done = s->done[q];
+    final_sums<NR>(partials, nchunks, tot);
+    if (threadIdx.x < NR && !done) s->alpha[q] = rr / tot[q];
 }
 
 template <int PR, int NR>
@@ -282,26 +333,29 @@ __global__ __launch_bounds__(BC * NR) void k_bcg_update(const BState* s, cplx<fl
 template <int NR>
 __global__ __launch_bounds__(FT) void k_bcg_update_final(BState* s, const double* partials, long nchunks) {
     if (s->all_done) return;
-    double out[NR];
-    final_sums<NR>(partials, nchunks, out);
+    __shared__ double tot[NR];
+    const bool on = threadIdx.x < NR;
+    const int q = on ? threadIdx.x : 0;
+    double mx = s->maxrr[q];
+    const double rr = s->rr_s[q], eps = s->eps[q], delta2 = s->delta2;
+    int done = s->done[q], rel = s->rel[q];
+    const int step = s->step[q] + 1, max_steps = s->max_steps;
+    final_sums<NR>(partials, nchunks, tot);
+    if (threadIdx.x >= 64) return;
+    if (on && !done) {
+        const double rn = tot[q];
+        if (rn > mx) s->maxrr[q] = mx = rn;
+        // due reliable updates run at the next reliable-update slot
+        if (rn < delta2 * mx || rn < eps) s->rel[q] = rel = 1;
+        s->beta[q] = rn / rr;
+        s->rr_s[q] = rn;
+        s->step[q] = step;
+        if (step >= max_steps) s->done[q] = done = 1;
+    }
+    const int any = __any(on && rel && !done), all = __all(!on || done);
     if (threadIdx.x == 0) {
-        int any = 0;
-        for (int q = 0; q < NR; ++q) {
-            if (s->done[q]) continue;
-            const double rn = out[q];
-            if (rn > s->maxrr[q]) s->maxrr[q] = rn;
-            // due reliable updates run at the next reliable-update slot
-            if (rn < s->delta2 * s->maxrr[q] || rn < s->eps[q]) s->rel[q] = 1;
-            s->beta[q] = rn / s->rr_s[q];
-            s->rr_s[q] = rn;
-            s->step[q] += 1;
-            if (s->step[q] >= s->max_steps) s->done[q] = 1;
-        }
-        for (int q = 0; q < NR; ++q) any = any || (s->rel[q] && !s->done[q]);
         s->any_rel = any;
         s->skip_rel = any ? 0 : 1;
-        int all = 1;
-        for (int q = 0; q < NR; ++q) all = all && s->done[q];
         s->all_done = all;
     }
 }
@@ -355,32 +409,35 @@ __global__ __launch_bounds__(BC * NR) void k_brel_resid(const BState* s, zd* r, 
 template <int NR>
 __global__ __launch_bounds__(FT) void k_brel_final(BState* s, const double* partials, long nchunks) {
     if (s->skip_rel) return;
-    double out[NR];
-    final_sums<NR>(partials, nchunks, out);
-    if (threadIdx.x == 0) {
-        for (int q = 0; q < NR; ++q) {
-            if (!s->rel[q]) continue;
-            const double rt = out[q];
-            s->rr_true[q] = rt;
-            s->nrel[q] += 1;
-            s->rel[q] = 0;
-            if (rt < s->eps[q]) {
-                s->done[q] = 1;
-                s->conv[q] = 1;
-                continue;
-            }
+    __shared__ double tot[NR];
+    const bool on = threadIdx.x < NR;
+    const int q = on ? threadIdx.x : 0;
+    int done = s->done[q];
+    const int rel = s->rel[q], nrel = s->nrel[q] + 1;
+    const double eps = s->eps[q];
+    final_sums<NR>(partials, nchunks, tot);
+    if (threadIdx.x >= 64) return;
+    if (on && rel) {
+        const double rt = tot[q];
+        s->rr_true[q] = rt;
+        s->nrel[q] = nrel;
+        s->rel[q] = 0;
+        if (rt < eps) {
+            s->done[q] = done = 1;
+            s->conv[q] = 1;
+        } else {
             s->rr_s[q] = rt;
             s->maxrr[q] = rt;
         }
+    }
+    const int all = __all(!on || done);
+    if (threadIdx.x == 0) {
         s->any_rel = 0;
         s->skip_rel = 1;
-        int all = 1;
-        for (int q = 0; q < NR; ++q) all = all && s->done[q];
         s->all_done = all;
     }
 }
 
-// p = r_s + beta p for the RHS still running
 template <int PR, int NR>
 __global__ void k_bcg_p(const BState* s, typename Prec<PR>::S* p, float* p_sc, const cplx<float>* rs, long nsites,
                         int stride) {
@@ -483,6 +540,8 @@ static void bcg_step_impl(int which, BState* s, const BcgArgs& a, hipStream_t st
     const long nch = (a.nsites + BC - 1) / BC;
     const dim3 cg((unsigned)nch), cb(BC * NR), fb(FT);
     const int eb = pair_blocks(a.nsites * NR);
+    const dim3 sg(chunk_wave<NR> ? (unsigned)((nch + CHUNK_WAVES - 1) / CHUNK_WAVES) : (unsigned)nch);
+    const dim3 sb(chunk_wave<NR> ? 64 * CHUNK_WAVES : BC * NR);
     switch (which) {
         case 0:
             hipLaunchKernelGGL((k_bcg_init<PR, NR>), cg, cb, 0, st, a.r, a.rs, a.xs, p, a.p_sc, a.nsites, a.stride,
@@ -511,12 +570,12 @@ static void bcg_step_impl(int which, BState* s, const BcgArgs& a, hipStream_t st
             hipLaunchKernelGGL((k_bcg_p<PR, NR>), dim3(eb), dim3(256), 0, st, s, p, a.p_sc, a.rs, a.nsites, a.stride);
             break;
         case 7:
-            hipLaunchKernelGGL((k_bcg_chunksum<NR>), cg, cb, 0, st, s, a.bsite, a.nsites, a.stride, a.vh, a.partials,
+            hipLaunchKernelGGL((k_bcg_chunksum<NR>), sg, sb, 0, st, s, a.bsite, a.nsites, a.stride, a.vh, a.partials,
                                nch);
             hipLaunchKernelGGL((k_bcg_alpha_final<NR>), dim3(1), fb, 0, st, s, a.partials, nch);
             break;
         case 8:
-            hipLaunchKernelGGL((k_bcg_chunksum<NR>), cg, cb, 0, st, s, a.bsite, a.nsites, a.stride, a.vh, a.partials,
+            hipLaunchKernelGGL((k_bcg_chunksum<NR>), sg, sb, 0, st, s, a.bsite, a.nsites, a.stride, a.vh, a.partials,
                                nch);
             hipLaunchKernelGGL((k_bcg_update_final<NR>), dim3(1), fb, 0, st, s, a.partials, nch);
             break;
