@@ -93,18 +93,18 @@ __device__ __forceinline__ void pin(cplx<T> acc[12]) {
 }
 
 // the neighbour spinor at idx: from the LDS copy of the other parity's site
-// block [lbase, lbase + LYM_DSLASH_THREADS) when lds is set and idx is inside,
+// block [lbase, lbase + TH) when lds is set and idx is inside,
 // else from the field
-template <int MU, int PR>
+template <int MU, int PR, int TH>
 __device__ __forceinline__ void load_nb(const SpinorRef<PR>& src, int stride, int nr, int idx, int r,
                                         cplx<typename Prec<PR>::T> psi[12], typename Prec<PR>::T& sc,
                                         const cplx<double>* lds, int lbase) {
     if constexpr (PR == 0 && MU >= 2) {
         if (lds) {
             const unsigned j = (unsigned)(idx - lbase);
-            if (j < (unsigned)LYM_DSLASH_THREADS) {
+            if (j < (unsigned)TH) {
 #pragma unroll
-                for (int k = 0; k < 12; ++k) psi[k] = lds[k * LYM_DSLASH_THREADS + j];
+                for (int k = 0; k < 12; ++k) psi[k] = lds[k * TH + j];
                 sc = 1.0;
                 return;
             }
@@ -115,7 +115,7 @@ __device__ __forceinline__ void load_nb(const SpinorRef<PR>& src, int stride, in
 
 // one hop pair (forward and backward, or backward first when BWD_FIRST) in
 // direction MU for site (p, site), rhs r; lds, lbase: as for load_nb
-template <int MU, int PR, int LK, bool BWD_FIRST = false>
+template <int MU, int PR, int LK, bool BWD_FIRST = false, int TH = LYM_DSLASH_THREADS>
 __device__ __forceinline__ void hop_pair(const DslashParams& a, int p, int site, int r, const int c[4],
                                          cplx<typename Prec<PR>::T> acc[12], const cplx<double>* lds = nullptr,
                                          int lbase = 0) {
@@ -138,7 +138,7 @@ __device__ __forceinline__ void hop_pair(const DslashParams& a, int p, int site,
     constexpr bool pin_mid = PH == 1;
     constexpr bool pin_end = PH <= 2 || (PH == 4 && (MU & 1));
     if constexpr (!BWD_FIRST) {
-        load_nb<MU, PR>(src, g.stride, a.nr, iu, rr, psi, sc, lds, lbase);
+        load_nb<MU, PR, TH>(src, g.stride, a.nr, iu, rr, psi, sc, lds, lbase);
         load_link<PR, LK>(a.links, g.stride, p, MU, site, L);
         hop_dir<MU, true, LK, T, SC>(acc, psi, L, anti && c[3] == g.L[3] - 1, sc);
         if constexpr (pin_mid) pin(acc);
@@ -147,13 +147,13 @@ __device__ __forceinline__ void hop_pair(const DslashParams& a, int p, int site,
         cplx<T> psi2[12];
         T sc2;
         LinkMat<LK, T> L2;
-        load_nb<MU, PR>(src, g.stride, a.nr, id, rr, psi2, sc2, lds, lbase);
+        load_nb<MU, PR, TH>(src, g.stride, a.nr, id, rr, psi2, sc2, lds, lbase);
         load_link<PR, LK>(a.links, g.stride, q, MU, id, L2);
         hop_dir<MU, false, LK, T, SC>(acc, psi2, L2, anti && c[3] == 0, sc2);
     }
     if constexpr (BWD_FIRST) {
         if constexpr (pin_mid) pin(acc);
-        load_nb<MU, PR>(src, g.stride, a.nr, iu, rr, psi, sc, lds, lbase);
+        load_nb<MU, PR, TH>(src, g.stride, a.nr, iu, rr, psi, sc, lds, lbase);
         load_link<PR, LK>(a.links, g.stride, p, MU, site, L);
         hop_dir<MU, true, LK, T, SC>(acc, psi, L, anti && c[3] == g.L[3] - 1, sc);
     }
@@ -175,7 +175,7 @@ __device__ __forceinline__ double dslash_epilogue(const DslashParams& a, int p, 
 // FM: a fused step of the FP64 solvers (F64_*), with step al, its terms added to
 // sums.  NT: FP64 blocks stream past the caches (no other lane reads them).
 template <int PR, int LK, int DIAG, bool INV, bool NORM = false, bool LO = false, bool UPD = false, int BM = 0,
-          int FM = 0, bool NT = true>
+          int FM = 0, bool NT = true, int TH = LYM_DSLASH_THREADS>
 __device__ __forceinline__ double dslash_site(const DslashParams& a, int p, int site, int r, float ual = 0.f,
                                               const cplx<double>* lds = nullptr, int lbase = 0, double al = 0.0,
                                               double* sums = nullptr) {
@@ -193,8 +193,8 @@ __device__ __forceinline__ double dslash_site(const DslashParams& a, int p, int 
     } else {
         hop_pair<0, PR, LK>(a, p, site, r, c, acc);
         hop_pair<1, PR, LK>(a, p, site, r, c, acc);
-        hop_pair<2, PR, LK>(a, p, site, r, c, acc, lds, lbase);
-        hop_pair<3, PR, LK>(a, p, site, r, c, acc, lds, lbase);
+        hop_pair<2, PR, LK, false, TH>(a, p, site, r, c, acc, lds, lbase);
+        hop_pair<3, PR, LK, false, TH>(a, p, site, r, c, acc, lds, lbase);
     }
     return dslash_epilogue<PR, LK, DIAG, INV, NORM, LO, UPD, BM, FM, NT>(a, p, site, r, acc, ual, al, sums);
 }
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash(DslashPar
     }
 }
 
-// FP64, one thread per site (spb == LYM_DSLASH_THREADS): each site
+// FP64, one thread per site (spb == TH): each site
 // block first copies the other parity's spinors of the same block index --
 // with t fastest, the z and t neighbours of most of the block's sites -- into
 // LDS, coalesced, once; those hops then read LDS instead of issuing four
@@ -448,9 +448,9 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash(DslashPar
 // the first the same, the second 15 % slower on 16^3x32.
 // FM: a fused step of the FP64 solvers; its terms' per-workgroup sums go to
 // a.upd_rpart.  LN: over lanes; LO: per-lane operators.
-template <int LK, int DIAG, bool INV, int FM = 0, bool LN = false, bool LO = false>
-__global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash_stg(DslashParams a) {
-    __shared__ cplx<double> stg[12 * LYM_DSLASH_THREADS];
+template <int LK, int DIAG, bool INV, int FM = 0, bool LN = false, bool LO = false, int TH = LYM_DSLASH_THREADS>
+__global__ __launch_bounds__(TH) LYM_OCC void k_dslash_stg(DslashParams a) {
+    __shared__ cplx<double> stg[12 * TH];
     if (a.skip && *a.skip) return;
     int bx = (int)blockIdx.x, gd = (int)gridDim.x, lane = 0;
     if constexpr (LN) {
@@ -463,18 +463,18 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash_stg(Dslas
     for (int lb = b.lo + b.k; lb < b.hi; lb += b.nphys) {
         int p, bi;
         (void)block_of_at(a, b, lb, bx, p, bi);
-        const int base = bi * LYM_DSLASH_THREADS;
+        const int base = bi * TH;
         __syncthreads();  // the previous block's reads of stg are done
         if (base + t < a.g.Vh) {
             const zd* src = lane_base<0>(a.in[p ^ a.g.tsh], a.in_lane, LN ? lane : 0);
 #pragma unroll
             for (int k = 0; k < 12; ++k)
-                stg[k * LYM_DSLASH_THREADS + t] = fld<zd>(src + (size_t)k * a.g.stride, (unsigned)(base + t));
+                stg[k * TH + t] = fld<zd>(src + (size_t)k * a.g.stride, (unsigned)(base + t));
         }
         __syncthreads();
         const int site = base + t;
         if (site < a.g.Vh)
-            dslash_site<0, LK, DIAG, INV, false, LO, false, 0, FM, !LN>(a, p, site, LN ? lane : 0, 0.f, stg, base, al,
+            dslash_site<0, LK, DIAG, INV, false, LO, false, 0, FM, !LN, TH>(a, p, site, LN ? lane : 0, 0.f, stg, base, al,
                                                                       sums);
     }
     if constexpr (FM == F64_DOT) block_sums_store<3>(sums, a.upd_rpart, a.part_stride);
@@ -908,6 +908,26 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) void k_dslash_mfma(DslashParams
     }
 }
 
+// one field, in workgroups of TH sites
+template <int LK, int DIAG, bool INV, int TH>
+static void launch_stg(const DslashParams& a, int nblocks, hipStream_t st) {
+    const dim3 g(nblocks), th(TH);
+    if constexpr (DIAG >= 1 && !INV) {
+        switch (a.fmode) {
+            case F64_NORM:
+                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_NORM, false, false, TH>), g, th, 0, st, a);
+                return;
+            case F64_CG:
+                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_CG, false, false, TH>), g, th, 0, st, a);
+                return;
+            case F64_DOT:
+                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_DOT, false, false, TH>), g, th, 0, st, a);
+                return;
+            default: break;
+        }
+    }
+    hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_STORE, false, false, TH>), g, th, 0, st, a);
+}
 template <int LK, int DIAG, bool INV>
 static void launch_f64(const DslashParams& a, int nblocks, hipStream_t st) {
     const dim3 g(lane_grid(a, nblocks)), th(LYM_DSLASH_THREADS);
@@ -919,15 +939,8 @@ static void launch_f64(const DslashParams& a, int nblocks, hipStream_t st) {
         hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_STORE, true>), g, th, 0, st, a);
         return;
     }
-    if constexpr (DIAG >= 1 && !INV) {
-        switch (a.fmode) {
-            case F64_NORM: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_NORM>), g, th, 0, st, a); return;
-            case F64_CG: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_CG>), g, th, 0, st, a); return;
-            case F64_DOT: hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_DOT>), g, th, 0, st, a); return;
-            default: break;
-        }
-    }
-    hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV>), g, th, 0, st, a);
+    if (a.spb == 64) launch_stg<LK, DIAG, INV, 64>(a, nblocks, st);
+    else launch_stg<LK, DIAG, INV, LYM_DSLASH_THREADS>(a, nblocks, st);
 }
 
 template <int PR, int LK, int DIAG, bool INV>
@@ -1095,12 +1108,36 @@ static int plan_hop(DslashParams& a) {
     return a.nblocks_per_parity * par;
 }
 
+// FP64 launches of one field that a sweep would spread badly run one wave to a
+// workgroup instead of four.  A CU's time is that of the waves it gets: with n
+// workgroups of four waves, 4 ceil(n / 256), some CUs a workgroup more than others;
+// with single waves ceil(4 n / 256).  Where that is at most 0.8 of the other (more
+// than it costs that fewer z neighbours are in the block's own copy): SU(3) clover
+// 16^3x20 31.4 -> 24.6 us, 16^3x24 33.6 -> 30.1, 14^4 16.3 -> 15.1, 17x15x13x21
+// 31.7 -> 24.4, Schur complement 16x20^2x24 81.0 -> 68.6.  Above it the four waves are as
+// fast or faster: at 7 against 8 (16^3x28) 35.4 and 36.4, at 4 against 4 (15^4) 18.1 and
+// 18.7.  Returns the workgroups, or 0 when the launch keeps workgroups of four.
+static int plan_waves(DslashParams& a) {
+    if (a.prec != 0 || a.lanes > 1 || a.lane_flags || a.lane_ops || LYM_DSLASH_THREADS != 256) return 0;
+    const int par = a.parity >= 0 ? 1 : 2;
+    const int n4 = a.nblocks_per_parity * par, nb = (a.g.Vh + 63) / 64, n1 = nb * par;
+    if (n4 > LYM_SWEEP_MAX_BLOCKS || 5 * ((n1 + 255) / 256) > 16 * ((n4 + 255) / 256)) return 0;
+    if (a.fmode && n1 > FOLD_MAX) return 0;  // a fold more would take what it gains
+    a.spb = 64;
+    a.nblocks_per_parity = nb;
+    const int xs = a.g.Vh / a.g.L[0];
+    a.xslice_blocks = xs % 64 == 0 ? xs / 64 : 0;
+    return n1;
+}
+
 int launch_dslash(DslashParams a, int link_kind, int diag, bool inv, hipStream_t st) {
     const int threads = (a.threads > 0 && a.threads <= LYM_DSLASH_THREADS) ? a.threads : LYM_DSLASH_THREADS;
     if (a.nr < 1) a.nr = 1;
     if (a.prec == 0) a.threads = 0;
     const int hop_blocks = plan_hop(a);
-    const int nblocks = hop_blocks ? hop_blocks : plan_dslash(a);
+    int nblocks = hop_blocks ? hop_blocks : plan_dslash(a);
+    if (!hop_blocks)
+        if (const int n = plan_waves(a)) nblocks = n;
     a.grid1 = nblocks;
     // output norm partials: low precision only, one per workgroup, and only
     // when the caller's buffer holds one per workgroup of this launch
