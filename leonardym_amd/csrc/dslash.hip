@@ -448,25 +448,21 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) LYM_OCC void k_dslash(DslashPar
 // the first the same, the second 15 % slower on 16^3x32.
 // FM: a fused step of the FP64 solvers; its terms' per-workgroup sums go to
 // a.upd_rpart.  LN: over lanes; LO: per-lane operators.
-template <int LK, int DIAG, bool INV, int FM = 0, bool LN = false, bool LO = false, int TH = LYM_DSLASH_THREADS>
+template <int LK, int DIAG, bool INV, int FM = 0, int TH = LYM_DSLASH_THREADS>
 __global__ __launch_bounds__(TH) LYM_OCC void k_dslash_stg(DslashParams a) {
     __shared__ cplx<double> stg[12 * TH];
     if (a.skip && *a.skip) return;
-    int bx = (int)blockIdx.x, gd = (int)gridDim.x, lane = 0;
-    if constexpr (LN) {
-        if (!lane_of_block(a, bx, gd, lane)) return;
-    }
-    const BlockSweep b = block_sweep_at(a, bx, gd);
+    const BlockSweep b = block_sweep(a);
     const int t = (int)threadIdx.x;
     double al = 0, sums[3] = {0, 0, 0};
     if constexpr (FM == F64_CG) al = upd_alpha<CGState>(a);
     for (int lb = b.lo + b.k; lb < b.hi; lb += b.nphys) {
         int p, bi;
-        (void)block_of_at(a, b, lb, bx, p, bi);
+        block_of(a, b, lb, p, bi);
         const int base = bi * TH;
         __syncthreads();  // the previous block's reads of stg are done
         if (base + t < a.g.Vh) {
-            const zd* src = lane_base<0>(a.in[p ^ a.g.tsh], a.in_lane, LN ? lane : 0);
+            const zd* src = reinterpret_cast<const zd*>(a.in[p ^ a.g.tsh]);
 #pragma unroll
             for (int k = 0; k < 12; ++k)
                 stg[k * TH + t] = fld<zd>(src + (size_t)k * a.g.stride, (unsigned)(base + t));
@@ -474,11 +470,42 @@ __global__ __launch_bounds__(TH) LYM_OCC void k_dslash_stg(DslashParams a) {
         __syncthreads();
         const int site = base + t;
         if (site < a.g.Vh)
-            dslash_site<0, LK, DIAG, INV, false, LO, false, 0, FM, !LN, TH>(a, p, site, LN ? lane : 0, 0.f, stg, base, al,
-                                                                      sums);
+            dslash_site<0, LK, DIAG, INV, false, false, false, 0, FM, true, TH>(a, p, site, 0, 0.f, stg, base, al, sums);
     }
     if constexpr (FM == F64_DOT) block_sums_store<3>(sums, a.upd_rpart, a.part_stride);
     else if constexpr (FM != F64_STORE) block_sums_store<1>(sums, a.upd_rpart, 0);
+}
+
+// The same over lanes: a workgroup holds 64 sites of LANE_WAVES (or fewer) lanes, a
+// wave each, so that the waves that read a site's links and blocks do so from one
+// CU's cache; a wave stages its own lane's spinors and waits for no other.  Against
+// workgroups of 256 sites of one lane, whose lanes shared links in the L2 only: 32^3x64
+// propagator 625 -> 597 ms (4 RHS at a time 654 -> 612), served burst 38.4 -> 37.6 ms.
+// Eight waves to a workgroup: 610 and 38.9.
+constexpr int LANE_WAVES = 4;
+template <int LK, int DIAG, bool INV, bool LO>
+__global__ __launch_bounds__(64 * LANE_WAVES) LYM_OCC void k_dslash_lanes(DslashParams a) {
+    __shared__ cplx<double> stg_all[LANE_WAVES * 12 * 64];
+    if (a.skip && *a.skip) return;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
+    int bx, gd, lane;
+    if (!lane_of_block(a, nw, w, bx, gd, lane)) return;
+    cplx<double>* stg = stg_all + w * (12 * 64);
+    const BlockSweep b = block_sweep_at(a, bx, gd);
+    const int t = (int)threadIdx.x & 63;
+    int p, bi;
+    if (b.lo + b.k >= b.hi) return;
+    (void)block_of_at(a, b, b.lo + b.k, bx, p, bi);
+    const int base = bi * 64, site = base + t;
+    if (site < a.g.Vh) {
+        const zd* src = lane_base<0>(a.in[p ^ a.g.tsh], a.in_lane, lane);
+#pragma unroll
+        for (int k = 0; k < 12; ++k) stg[k * 64 + t] = fld<zd>(src + (size_t)k * a.g.stride, (unsigned)site);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (site < a.g.Vh)
+        dslash_site<0, LK, DIAG, INV, false, LO, false, 0, F64_STORE, false, 64>(a, p, site, lane, 0.f, stg, base);
 }
 
 // ---------------------------------------------------------------- two threads per site (FP32/FP16)
@@ -908,6 +935,15 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) void k_dslash_mfma(DslashParams
     }
 }
 
+// FP64 launches over lanes: their waves to a workgroup, a divisor of the lanes (the
+// batch widths are 1, 2, 3, 4, 6, 8, 12 and 16)
+static bool over_lanes(const DslashParams& a) { return a.prec == 0 && (a.lanes > 1 || a.lane_flags || a.lane_ops); }
+static int lane_waves(const DslashParams& a) {
+    for (int w = LANE_WAVES; w > 1; --w)
+        if (a.lanes % w == 0) return a.lanes > 1 ? w : 1;
+    return 1;
+}
+
 // one field, in workgroups of TH sites
 template <int LK, int DIAG, bool INV, int TH>
 static void launch_stg(const DslashParams& a, int nblocks, hipStream_t st) {
@@ -915,31 +951,29 @@ static void launch_stg(const DslashParams& a, int nblocks, hipStream_t st) {
     if constexpr (DIAG >= 1 && !INV) {
         switch (a.fmode) {
             case F64_NORM:
-                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_NORM, false, false, TH>), g, th, 0, st, a);
+                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_NORM, TH>), g, th, 0, st, a);
                 return;
             case F64_CG:
-                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_CG, false, false, TH>), g, th, 0, st, a);
+                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_CG, TH>), g, th, 0, st, a);
                 return;
             case F64_DOT:
-                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_DOT, false, false, TH>), g, th, 0, st, a);
+                hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_DOT, TH>), g, th, 0, st, a);
                 return;
             default: break;
         }
     }
-    hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_STORE, false, false, TH>), g, th, 0, st, a);
+    hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_STORE, TH>), g, th, 0, st, a);
 }
 template <int LK, int DIAG, bool INV>
 static void launch_f64(const DslashParams& a, int nblocks, hipStream_t st) {
-    const dim3 g(lane_grid(a, nblocks)), th(LYM_DSLASH_THREADS);
-    if (a.lane_ops) {
-        hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_STORE, true, true>), g, th, 0, st, a);
+    if (over_lanes(a)) {
+        const int nw = lane_waves(a);
+        const dim3 g(lane_grid(a, nblocks, nw)), th(64 * nw);
+        if (a.lane_ops) hipLaunchKernelGGL((k_dslash_lanes<LK, DIAG, INV, true>), g, th, 0, st, a);
+        else hipLaunchKernelGGL((k_dslash_lanes<LK, DIAG, INV, false>), g, th, 0, st, a);
         return;
     }
-    if (a.lanes > 1 || a.lane_flags) {
-        hipLaunchKernelGGL((k_dslash_stg<LK, DIAG, INV, F64_STORE, true>), g, th, 0, st, a);
-        return;
-    }
-    if (a.spb == 64) launch_stg<LK, DIAG, INV, 64>(a, nblocks, st);
+    if (a.spb == 64) launch_stg<LK, DIAG, INV, 64>(a, nblocks, st);  // plan_waves
     else launch_stg<LK, DIAG, INV, LYM_DSLASH_THREADS>(a, nblocks, st);
 }
 
@@ -1118,11 +1152,13 @@ static int plan_hop(DslashParams& a) {
 // fast or faster: at 7 against 8 (16^3x28) 35.4 and 36.4, at 4 against 4 (15^4) 18.1 and
 // 18.7.  Returns the workgroups, or 0 when the launch keeps workgroups of four.
 static int plan_waves(DslashParams& a) {
-    if (a.prec != 0 || a.lanes > 1 || a.lane_flags || a.lane_ops || LYM_DSLASH_THREADS != 256) return 0;
+    if (a.prec != 0 || LYM_DSLASH_THREADS != 256) return 0;
     const int par = a.parity >= 0 ? 1 : 2;
     const int n4 = a.nblocks_per_parity * par, nb = (a.g.Vh + 63) / 64, n1 = nb * par;
-    if (n4 > LYM_SWEEP_MAX_BLOCKS || 5 * ((n1 + 255) / 256) > 16 * ((n4 + 255) / 256)) return 0;
-    if (a.fmode && n1 > FOLD_MAX) return 0;  // a fold more would take what it gains
+    if (!over_lanes(a)) {
+        if (n4 > LYM_SWEEP_MAX_BLOCKS || 5 * ((n1 + 255) / 256) > 16 * ((n4 + 255) / 256)) return 0;
+        if (a.fmode && n1 > FOLD_MAX) return 0;  // a fold more would take what it gains
+    }
     a.spb = 64;
     a.nblocks_per_parity = nb;
     const int xs = a.g.Vh / a.g.L[0];

@@ -220,7 +220,7 @@ __global__ __launch_bounds__(HOP_THREADS, PR == 0 ? 3 : (PR == 1 ? 5 : 6)) void 
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int bx = (int)blockIdx.x, gd = (int)gridDim.x, ls, r;
     if constexpr (PR == 0) {
-        if (!lane_of_block(a, bx, gd, r)) return;
+        if (!lane_of_block(a, 1, 0, bx, gd, r)) return;
         ls = lane;
     } else {
         ls = lane / a.nr;
@@ -540,12 +540,12 @@ static void hop_go(const DslashParams& a, int nblocks, hipStream_t st) {
     if constexpr (MODE != HOP_NORM && MODE != HOP_UPD) {
         if (a.lane_ops) {
             hipLaunchKernelGGL((k_dslash_hop<PR, LK, DIAG, INV, MODE, true>),
-                               dim3(PR == 0 ? lane_grid(a, nblocks) : nblocks), dim3(HOP_THREADS), 0, st, a);
+                               dim3(PR == 0 ? lane_grid(a, nblocks, 1) : nblocks), dim3(HOP_THREADS), 0, st, a);
             return;
         }
     }
-    hipLaunchKernelGGL((k_dslash_hop<PR, LK, DIAG, INV, MODE, false>), dim3(PR == 0 ? lane_grid(a, nblocks) : nblocks),
-                       dim3(HOP_THREADS), 0, st, a);
+    hipLaunchKernelGGL((k_dslash_hop<PR, LK, DIAG, INV, MODE, false>),
+                       dim3(PR == 0 ? lane_grid(a, nblocks, 1) : nblocks), dim3(HOP_THREADS), 0, st, a);
 }
 
 // the FP64 solvers' fused steps

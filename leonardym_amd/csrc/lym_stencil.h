@@ -276,20 +276,21 @@ __host__ __device__ __forceinline__ int block_of_at(const DslashParams& a, const
     return MAP_PLAIN;
 }
 
-// Workgroups of an FP64 launch over lanes: the lanes of one logical workgroup
-// follow one another on its XCD (links and blocks that one lane reads are then in
-// the L2 for the next).  Launcher: the grid; device: the logical workgroup bx of
-// gd and its lane, false when there is nothing to do.
-static inline int lane_grid(const DslashParams& a, int nblocks) {
-    return a.lanes > 1 ? (nblocks + 7) / 8 * 8 * a.lanes : nblocks;
+// Workgroups of an FP64 launch over lanes, nw of them to a workgroup (a wave each): the
+// lanes of one site block follow one another on its XCD (links and blocks that one
+// lane reads are then in the L2 for the next).  Launcher: the grid; device: the
+// site block's workgroup bx of gd and the lane of wave w, false when there is nothing
+// to do.
+static inline int lane_grid(const DslashParams& a, int nblocks, int nw) {
+    return a.lanes > nw ? (nblocks + 7) / 8 * 8 * (a.lanes / nw) : nblocks;
 }
-__device__ __forceinline__ bool lane_of_block(const DslashParams& a, int& bx, int& gd, int& lane) {
+__device__ __forceinline__ bool lane_of_block(const DslashParams& a, int nw, int w, int& bx, int& gd, int& lane) {
     bx = (int)blockIdx.x;
     gd = (int)gridDim.x;
-    lane = 0;
-    if (a.lanes > 1) {
-        const int t = bx >> 3, u = t / a.lanes;
-        lane = t - u * a.lanes;
+    lane = w;
+    if (a.lanes > nw) {
+        const int t = bx >> 3, ng = a.lanes / nw, u = t / ng;
+        lane += (t - u * ng) * nw;
         bx = u * 8 + (bx & 7);
         gd = a.grid1;
         if (bx >= gd) return false;

@@ -41,7 +41,7 @@ def test_widths(dims, kind, solver, power):
     ctx, g, op, srcs = _case(dims, 0.11, power, kind)
     eps = [(REL * np.linalg.norm(b)) ** 2 for b in srcs]
     got = {}
-    for block in (1, 2, 4):
+    for block in (1, 2, 3, 4, 6):
         print("dims", dims, "block", block, flush=True)
         s = lym.Solver(ctx, solver, max_steps=2000, sloppy=lym.PREC_HALF)
         s.set_rhs_block(block)
@@ -50,7 +50,7 @@ def test_widths(dims, kind, solver, power):
         assert all(i.converged for i in infos)
         got[block] = [x.download() for x in X]
     for q, b in enumerate(srcs):
-        assert np.array_equal(got[1][q], got[2][q]) and np.array_equal(got[1][q], got[4][q])
+        assert all(np.array_equal(got[1][q], got[k][q]) for k in (2, 3, 4, 6))
         if solver == lym.SOLVER_MIXED_CG:
             assert _residual(ctx, op, got[4][q], b) <= BOUND
         else:
