@@ -385,7 +385,8 @@ int lym_stout_smear(const int dims[4], int ncolors, double rho, int levels, cons
  * branches (3 ints, or NULL) counts the blocks mapped by each renumbering:
  * plain order, x-slice fastest, XCD pairs.  The mapping is that of the one- and
  * two-threads-per-site forms; a launch of so few lanes that it takes the
- * one-wave-per-direction form visits its blocks once each in plain order. */
+ * one-wave-per-direction form visits its blocks once each in plain order, and an
+ * FP64 launch in workgroups of one wave visits blocks of 64 sites in this order. */
 int lym_launch_plan(const int dims[4], int parity, int nr, int threads, int lowp, int* grid, int* spb, int* nbpp,
                     int* xslice_blocks, int* visits, long visits_len, int* branches);
 
