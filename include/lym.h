@@ -383,12 +383,43 @@ int lym_stout_smear(const int dims[4], int ncolors, double rho, int levels, cons
  * per x-slice (0 when an x-slice is not a whole number of blocks).  visits
  * (2 * nbpp ints, or NULL) counts how often each (parity, block) is visited;
  * branches (3 ints, or NULL) counts the blocks mapped by each renumbering:
- * plain order, x-slice fastest, XCD pairs.  The mapping is that of the one- and
- * two-threads-per-site forms; a launch of so few lanes that it takes the
- * one-wave-per-direction form visits its blocks once each in plain order, and an
- * FP64 launch in workgroups of one wave visits blocks of 64 sites in this order. */
+ * plain order, x-slice fastest, XCD pairs.  The mapping is that of the forms of
+ * one and two threads per site in workgroups of `threads`, whether or not a launch
+ * takes them; lym_launch_form tells which form one takes. */
 int lym_launch_plan(const int dims[4], int parity, int nr, int threads, int lowp, int* grid, int* spb, int* nbpp,
                     int* xslice_blocks, int* visits, long visits_len, int* branches);
+
+/* What one stencil launch runs (no counterpart in the reference): the selection
+ * of form, workgroups and block order that the library's launches make,
+ * evaluated on the host.  prec 0 (FP64), LYM_PREC_SINGLE or LYM_PREC_HALF; nrhs
+ * right-hand sides (FP64: fields of their own); parity and threads as above;
+ * options: LYM_LAUNCH_SINGLE for the low-precision applies of one right-hand side
+ * (not of a batch), LYM_LAUNCH_MATRIX_CORES, LYM_LAUNCH_LANE_OPS for a kappa per
+ * right-hand side; step 1: a launch that also leaves partial sums, part_max of
+ * them at most.  SU(3) links of three rows.
+ * visits (2 * nbpp ints, or NULL) counts how often each (parity, block) is
+ * visited: once per right-hand side of an FP64 launch, else once. */
+enum {
+    LYM_FORM_SITE = 0,   /* a thread per (site, right-hand side) */
+    LYM_FORM_SPLIT = 1,  /* two threads per site (low precision, one right-hand side) */
+    LYM_FORM_HOP = 2,    /* a wave per direction (launches of few lanes) */
+    LYM_FORM_STAGED = 3, /* FP64: a thread per site, workgroups of four waves */
+    LYM_FORM_WAVE = 4,   /* the same in workgroups of one wave */
+    LYM_FORM_LANES = 5,  /* FP64, several right-hand sides: a wave per 64 sites of one */
+    LYM_FORM_MFMA = 6    /* the matrix cores (FP16) */
+};
+enum { LYM_LAUNCH_SINGLE = 1, LYM_LAUNCH_MATRIX_CORES = 2, LYM_LAUNCH_LANE_OPS = 4 };
+typedef struct {
+    int form;        /* LYM_FORM_* */
+    int grid;        /* workgroups */
+    int threads;     /* threads per workgroup */
+    int spb;         /* sites per workgroup (LYM_FORM_LANES: per wave) */
+    int nbpp;        /* site blocks per parity */
+    int partials;    /* partial sums left (0: step 0, or more than part_max) */
+    int branches[3]; /* blocks in plain order, x-slice fastest, XCD pairs */
+} lym_launch_info;
+int lym_launch_form(const int dims[4], int parity, int prec, int nrhs, int threads, int options, int step,
+                    int part_max, lym_launch_info* info, int* visits, long visits_len);
 
 /* ------------------------------------------------------------------ host-side input preparation
  * Seeded synthetic inputs (the reference seeds from time(NULL),

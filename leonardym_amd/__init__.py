@@ -119,6 +119,7 @@ SIGNATURES = {
     "lym_gen_gaussian_spinor": (_I, [_L, _U64, _P]),
     "lym_point_source": (_I, [_P, _P, _I, _I, _P]),
     "lym_launch_plan": (_I, [_P, _I, _I, _I, _I, _PI, _PI, _PI, _PI, _PI, _L, _PI]),
+    "lym_launch_form": (_I, [_P, _I, _I, _I, _I, _I, _I, _I, _P, _PI, _L]),
     "lym_meson_correlators": (_I, [_P, _P, _P, _PD, ctypes.POINTER(SolveInfo)]),
     "lym_config_write": (_I, [_I, ctypes.c_char_p, ctypes.c_char_p, _I, _PI, _I, _P, ctypes.POINTER(ConfigInfo)]),
     "lym_config_read": (_I, [_I, ctypes.c_char_p, ctypes.c_char_p, _I, _PI, _I, _P, ctypes.POINTER(ConfigInfo)]),
@@ -180,6 +181,30 @@ def launch_plan(dims, parity=-1, nr=1, threads=0, lowp=False):
                                  visits.ctypes.data_as(_PI), visits.size, branches.ctypes.data_as(_PI)))
     return {"grid": grid.value, "spb": spb.value, "nbpp": nbpp.value, "xslice_blocks": W.value,
             "visits": visits.reshape(2, nbpp.value), "branches": branches}
+
+
+FORM_SITE, FORM_SPLIT, FORM_HOP, FORM_STAGED, FORM_WAVE, FORM_LANES, FORM_MFMA = range(7)
+
+
+class LaunchInfo(ctypes.Structure):
+    _fields_ = [("form", _I), ("grid", _I), ("threads", _I), ("spb", _I), ("nbpp", _I), ("partials", _I),
+                ("branches", _I * 3)]
+
+
+def launch_form(dims, parity=-1, prec=0, nrhs=1, threads=0, single=False, matrix_cores=False, lane_ops=False,
+                step=False, part_max=0):
+    """The form, workgroups and block order one stencil launch takes, chosen on
+    the host by the library's own selection (no device needed): dict with form
+    (FORM_*), grid, threads, spb, nbpp, partials, branches (plain, x-slice, XCD
+    pairs) and visits [2, nbpp]."""
+    info = LaunchInfo()
+    args = (_arr(np.array(dims, np.int32)), parity, prec, nrhs, threads,
+            int(single) + 2 * int(matrix_cores) + 4 * int(lane_ops), int(step), part_max, ctypes.byref(info))
+    _check(lib().lym_launch_form(*args, None, 0))
+    visits = np.zeros(2 * info.nbpp, np.int32)
+    _check(lib().lym_launch_form(*args, visits.ctypes.data_as(_PI), visits.size))
+    return {"form": info.form, "grid": info.grid, "threads": info.threads, "spb": info.spb, "nbpp": info.nbpp,
+            "partials": info.partials, "branches": np.array(info.branches[:]), "visits": visits.reshape(2, -1)}
 
 
 # ---------------------------------------------------------------- host-side inputs

@@ -18,37 +18,8 @@
 //   EO driver source b_o - D_oe R^-1 b_e and even reconstruction
 //   R_ee^-1 (b_e - D_eo x_o)                  diag = 1, hop_sign = -1 [, INV]
 // (PreconditionedBiCGStab.cpp:56-86).
-#include "lym_stencil.h"
+#include "lym_plan.h"
 
-// Launch shape of the stencil (swept on the device; defaults are the measured best)
-#ifndef LYM_DSLASH_THREADS
-#define LYM_DSLASH_THREADS 256
-#endif
-// both parities of a block range run on the same XCD (links and spinors of a
-// region are then fetched into one L2 for the even and the odd sites)
-// -1: automatic -- one sweeping workgroup per CU for FP64 launches and FP32 ones of
-// two threads per site of at most LYM_SWEEP_MAX_BLOCKS workgroups (small lattices:
-// 16^3x32 FP64 clover 38.1 us, 42.1 with all workgroups at once; FP32 21.5, 22.7),
-// all workgroups at once above that (large lattices, where sweeping was slower) and
-// for the others, whose waves are smaller and wait longer for what they load: one
-// workgroup per CU leaves them one wave per SIMD (16^3x32 FP16 two threads per
-// site 17.1 us swept, 14.8 at once; Schur complement of 3 and 4 right-hand sides
-// 69.5 and 73.4, 44.7 and 45.3 at once; FP32 78.9, 72.3 at once)
-#ifndef LYM_GRID_PER_CU
-#define LYM_GRID_PER_CU -1
-#endif
-#ifndef LYM_SWEEP_MAX_BLOCKS
-#define LYM_SWEEP_MAX_BLOCKS 1024
-#endif
-// 1: single-RHS FP32/FP16 applies of at most LYM_SPLIT_MAX_SITES sites per
-// parity run two threads per site (k_dslash_split).  Measured: mixed CG on
-// 16^3x32 (65536 sites) 5 % faster, on 24^3x48 (331776) 4 % slower
-#ifndef LYM_SPLIT_LOWP
-#define LYM_SPLIT_LOWP 1
-#endif
-#ifndef LYM_SPLIT_MAX_SITES
-#define LYM_SPLIT_MAX_SITES 131072
-#endif
 // Full-lattice applies: odd-parity sites take each direction's backward hop
 // before its forward hop, so the two reads of a link U_mu(y) -- by y (forward)
 // and by y + mu (backward), sites of opposite parity -- happen at the same
@@ -482,7 +453,6 @@ __global__ __launch_bounds__(TH) LYM_OCC void k_dslash_stg(DslashParams a) {
 // workgroups of 256 sites of one lane, whose lanes shared links in the L2 only: 32^3x64
 // propagator 625 -> 597 ms (4 RHS at a time 654 -> 612), served burst 38.4 -> 37.6 ms.
 // Eight waves to a workgroup: 610 and 38.9.
-constexpr int LANE_WAVES = 4;
 template <int LK, int DIAG, bool INV, bool LO>
 __global__ __launch_bounds__(64 * LANE_WAVES) LYM_OCC void k_dslash_lanes(DslashParams a) {
     __shared__ cplx<double> stg_all[LANE_WAVES * 12 * 64];
@@ -935,15 +905,6 @@ __global__ __launch_bounds__(LYM_DSLASH_THREADS) void k_dslash_mfma(DslashParams
     }
 }
 
-// FP64 launches over lanes: their waves to a workgroup, a divisor of the lanes (the
-// batch widths are 1, 2, 3, 4, 6, 8, 12 and 16)
-static bool over_lanes(const DslashParams& a) { return a.prec == 0 && (a.lanes > 1 || a.lane_flags || a.lane_ops); }
-static int lane_waves(const DslashParams& a) {
-    for (int w = LANE_WAVES; w > 1; --w)
-        if (a.lanes % w == 0) return a.lanes > 1 ? w : 1;
-    return 1;
-}
-
 // one field, in workgroups of TH sites
 template <int LK, int DIAG, bool INV, int TH>
 static void launch_stg(const DslashParams& a, int nblocks, hipStream_t st) {
@@ -990,10 +951,7 @@ static void launch_one(const DslashParams& a, int nblocks, hipStream_t st) {
 template <int PR, int LK, int DIAG, bool INV>
 static void launch_lp(const DslashParams& a, int nblocks, hipStream_t st) {
     if constexpr (PR == 2 && LK == 0) {
-        // matrix-core form: FP16 SU(3) batches of 2, 4 or 8 RHS in whole waves (its
-        // lanes address the links by 32-bit byte offsets)
-        if (a.mfma && !a.bmode && 8L * a.g.stride * link_bytes(2, false, 3) < (1L << 32) &&
-            (a.nr == 2 || a.nr == 4 || a.nr == 8) && (a.spb * a.nr) % 64 == 0) {
+        if (takes_mfma(a)) {
             if (a.lane_ops)
                 hipLaunchKernelGGL((k_dslash_mfma<DIAG, INV, true>), dim3(nblocks), dim3(a.spb * a.nr), 0, st, a);
             else
@@ -1085,182 +1043,18 @@ static void launch_pr(const DslashParams& a, int link_kind, int diag, bool inv, 
     }
 }
 
-// Launch geometry: sites per workgroup, the split form, site blocks per parity
-// and per x-slice; returns the number of workgroups.
-static int plan_dslash(DslashParams& a) {
-    if (a.nr < 1) a.nr = 1;
-    const int threads = (a.threads > 0 && a.threads <= LYM_DSLASH_THREADS) ? a.threads : LYM_DSLASH_THREADS;
-    a.spb = threads / a.nr;
-    if (a.spb < 1) a.spb = 1;
-    // two threads per site: low-precision single-RHS applies that allow it
-    a.split = (LYM_SPLIT_LOWP && a.allow_split && !a.lane_ops && !a.bmode && a.prec >= 1 && threads % 64 == 0 &&
-               (long)a.g.Vh * a.nr <= LYM_SPLIT_MAX_SITES)
-                  ? threads
-                  : 0;
-    a.nblocks_per_parity = (a.g.Vh + a.spb - 1) / a.spb;
-    {
-        const int xs = a.g.Vh / a.g.L[0];  // sites of one parity per x-slice
-        a.xslice_blocks = (xs % a.spb == 0) ? xs / a.spb : 0;
-    }
-    int nblocks = a.nblocks_per_parity * (a.parity >= 0 ? 1 : 2);
-    // workgroups in flight: LYM_GRID_PER_CU per CU of the 256 CUs, sweeping
-    const bool sweep = (a.prec == 0 || (a.prec == 1 && a.split)) && nblocks <= LYM_SWEEP_MAX_BLOCKS;
-    const int gpc = LYM_GRID_PER_CU >= 0 ? LYM_GRID_PER_CU : (sweep ? 1 : 0);
-    if (gpc > 0 && nblocks > 256 * gpc) nblocks = 256 * gpc;
-    return nblocks;
-}
-
-// Launches of at most this many (site, RHS) lanes take the one-wave-per-direction
-// form (dslash_hop.hip); low-precision launches of one parity, whose other form
-// waits longest, more of them.  Measured, that form against the other: FP64 even-odd
-// CG iteration 83 against 91 us at 32768 lanes, Schur complement 39.0 against 38.4 at
-// 40960 and 43.0 against 41.9 at 49152; full applies 10.2 against 13.6 us at 20736
-// lanes (clover), 14.3 against 12.5 us at 41472 (Wilson).  Low-precision Schur
-// complement at 41472 lanes of two RHS 14.2 against 21.9 us (FP16), 18.8 against 22.5
-// (FP32), at 49152 lanes of one 17.7 against 19.6 and 23.3 against 25.7; FP16 mixed CG
-// iteration 78 against 67 us at 65536.
-#ifndef LYM_HOP_MAX
-#define LYM_HOP_MAX 32768
-#endif
-#ifndef LYM_HOP_MAX_LOWP_HALF
-#define LYM_HOP_MAX_LOWP_HALF 49152
-#endif
-
-// The launch geometry of that form: sites per workgroup and site blocks per
-// parity; returns the number of workgroups, or 0 when the launch takes another.
-static int plan_hop(DslashParams& a) {
-    const int par = a.parity >= 0 ? 1 : 2;
-    const long lanes = (long)a.g.Vh * a.nr * par;
-    if (LYM_T_SLOW || a.mfma || a.nr > 64 || lanes > (par == 1 && a.prec ? LYM_HOP_MAX_LOWP_HALF : LYM_HOP_MAX)) return 0;
-    a.spb = 64 / a.nr;
-    // tiny launches: fewer sites per workgroup, so that more CUs share the loads
-    while (a.spb > 1 && a.spb * a.nr > 16 && (a.g.Vh + a.spb - 1) / a.spb * par < 256) a.spb = (a.spb + 1) / 2;
-    a.nblocks_per_parity = (a.g.Vh + a.spb - 1) / a.spb;
-    a.inv_ext[0] = 1.0 / a.g.L[1];
-    a.inv_ext[1] = 1.0 / a.g.L[2];
-    a.inv_ext[2] = 1.0 / a.g.Lth;
-    return a.nblocks_per_parity * par;
-}
-
-// FP64 launches of one field that a sweep would spread badly run one wave to a
-// workgroup instead of four.  A CU's time is that of the waves it gets: with n
-// workgroups of four waves, 4 ceil(n / 256), some CUs a workgroup more than others;
-// with single waves ceil(4 n / 256).  Where that is at most 0.8 of the other (more
-// than it costs that fewer z neighbours are in the block's own copy): SU(3) clover
-// 16^3x20 31.4 -> 24.6 us, 16^3x24 33.6 -> 30.1, 14^4 16.3 -> 15.1, 17x15x13x21
-// 31.7 -> 24.4, Schur complement 16x20^2x24 81.0 -> 68.6.  Above it the four waves are as
-// fast or faster: at 7 against 8 (16^3x28) 35.4 and 36.4, at 4 against 4 (15^4) 18.1 and
-// 18.7.  Returns the workgroups, or 0 when the launch keeps workgroups of four.
-static int plan_waves(DslashParams& a) {
-    if (a.prec != 0 || LYM_DSLASH_THREADS != 256) return 0;
-    const int par = a.parity >= 0 ? 1 : 2;
-    const int n4 = a.nblocks_per_parity * par, nb = (a.g.Vh + 63) / 64, n1 = nb * par;
-    if (!over_lanes(a)) {
-        if (n4 > LYM_SWEEP_MAX_BLOCKS || 5 * ((n1 + 255) / 256) > 16 * ((n4 + 255) / 256)) return 0;
-        if (a.fmode && n1 > FOLD_MAX) return 0;  // a fold more would take what it gains
-    }
-    a.spb = 64;
-    a.nblocks_per_parity = nb;
-    const int xs = a.g.Vh / a.g.L[0];
-    a.xslice_blocks = xs % 64 == 0 ? xs / 64 : 0;
-    return n1;
-}
-
 int launch_dslash(DslashParams a, int link_kind, int diag, bool inv, hipStream_t st) {
-    const int threads = (a.threads > 0 && a.threads <= LYM_DSLASH_THREADS) ? a.threads : LYM_DSLASH_THREADS;
-    if (a.nr < 1) a.nr = 1;
-    if (a.prec == 0) a.threads = 0;
-    const int hop_blocks = plan_hop(a);
-    int nblocks = hop_blocks ? hop_blocks : plan_dslash(a);
-    if (!hop_blocks)
-        if (const int n = plan_waves(a)) nblocks = n;
-    a.grid1 = nblocks;
-    // output norm partials: low precision only, one per workgroup, and only
-    // when the caller's buffer holds one per workgroup of this launch
-    // (the workgroup sum shuffles over whole 64-lane waves)
-    const bool whole_waves = hop_blocks || threads % 64 == 0;
-    if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || !whole_waves || nblocks > a.norm_max)
-        a.norm_partials = nullptr;
-    // the fused update: under the same conditions (the caller checks the return
-    // value and runs the separate update when it is 0)
-    if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || a.lane_ops || !whole_waves ||
-        nblocks > a.norm_max || a.norm_partials)
-        if (!a.fmode) a.upd_state = nullptr;
-    // the FP64 solvers' fused steps: one RHS, a diagonal and no R^-1, and room for
-    // one partial per workgroup
-    if (a.prec != 0 || diag == 0 || inv || a.lanes > 1 || a.lane_flags || a.lane_ops || nblocks > a.part_stride)
-        a.fmode = F64_STORE;
-    const bool fused = a.norm_partials || a.upd_state || a.fmode;
-    if (hop_blocks) {
-        launch_dslash_hop(a, link_kind, diag, inv, nblocks, st);
-        return fused ? nblocks : 0;
+    const LaunchPlan L = plan_launch(a, link_kind, diag, inv);
+    if (L.form == LYM_FORM_HOP) {
+        launch_dslash_hop(a, link_kind, diag, inv, L.nblocks, st);
+        return L.partials;
     }
     switch (a.prec) {
-        case 0: launch_pr<0>(a, link_kind, diag, inv, nblocks, st); break;
-        case 1: launch_pr<1>(a, link_kind, diag, inv, nblocks, st); break;
-        default: launch_pr<2>(a, link_kind, diag, inv, nblocks, st); break;
+        case 0: launch_pr<0>(a, link_kind, diag, inv, L.nblocks, st); break;
+        case 1: launch_pr<1>(a, link_kind, diag, inv, L.nblocks, st); break;
+        default: launch_pr<2>(a, link_kind, diag, inv, L.nblocks, st); break;
     }
-    return fused ? nblocks : 0;
+    return L.partials;
 }
 
 }  // namespace lym
-
-// ---------------------------------------------------------------- launch plan (host)
-#include <cstring>
-
-#include "../../include/lym.h"
-
-namespace lym_internal {
-int fail(int code, const char* fmt, ...);
-}
-
-extern "C" int lym_launch_plan(const int dims[4], int parity, int nr, int threads, int lowp, int* grid, int* spb,
-                               int* nbpp, int* xslice_blocks, int* visits, long visits_len, int* branches) {
-    using lym_internal::fail;
-    if (!dims || !grid || !spb || !nbpp || !xslice_blocks) return fail(LYM_ERR_INVALID, "null argument");
-    for (int i = 0; i < 4; ++i)
-        if (dims[i] < 2) return fail(LYM_ERR_INVALID, "lattice extent %d must be >= 2", dims[i]);
-    // the context's layout: even-odd when all extents are even, else one class
-    // (whose launches are parity 0)
-    const int tsh = (dims[0] | dims[1] | dims[2] | dims[3]) % 2 == 0 ? 1 : 0;
-    if (parity < -1 || parity > 1 || nr < 1 || nr > 16 || threads < 0 || threads > LYM_DSLASH_THREADS ||
-        (!tsh && parity != 0))
-        return fail(LYM_ERR_INVALID, "bad launch arguments");
-    const long V = (long)dims[0] * dims[1] * dims[2] * dims[3];
-    if ((V >> tsh) > (1L << 27) - 64) return fail(LYM_ERR_INVALID, "lattice too large");
-    lym::DslashParams a;
-    std::memset(&a, 0, sizeof(a));
-    for (int i = 0; i < 4; ++i) a.g.L[i] = dims[i];
-    a.g.tsh = tsh;
-    a.g.Lth = dims[3] >> tsh;
-    a.g.Lxh = dims[0] >> tsh;
-    a.g.Vh = (int)(V >> tsh);
-    a.g.stride = (int)(((V >> tsh) + 63) / 64 * 64);
-    a.g.bc_t = -1;
-    a.nr = nr;
-    a.threads = threads;
-    a.parity = parity;
-    a.prec = lowp ? 2 : 0;
-    a.allow_split = lowp ? 1 : 0;
-    const int gdim = lym::plan_dslash(a);
-    *grid = gdim;
-    *spb = a.spb;
-    *nbpp = a.nblocks_per_parity;
-    *xslice_blocks = a.xslice_blocks;
-    if (visits && visits_len < 2L * a.nblocks_per_parity) return fail(LYM_ERR_INVALID, "visits array too short");
-    if (visits) std::memset(visits, 0, sizeof(int) * 2 * (size_t)a.nblocks_per_parity);
-    if (branches) branches[0] = branches[1] = branches[2] = 0;
-    for (int bx = 0; bx < gdim; ++bx) {
-        const lym::BlockSweep b = lym::block_sweep_at(a, bx, gdim);
-        for (int lb = b.lo + b.k; lb < b.hi; lb += b.nphys) {
-            int p = 0, bi = 0;
-            const int br = lym::block_of_at(a, b, lb, bx, p, bi);
-            if (p < 0 || p > 1 || bi < 0 || bi >= a.nblocks_per_parity)
-                return fail(LYM_ERR_INVALID, "workgroup %d maps block %d to (%d, %d), outside the lattice", bx, lb, p,
-                            bi);
-            if (visits) ++visits[p * a.nblocks_per_parity + bi];
-            if (branches) ++branches[br];
-        }
-    }
-    return LYM_OK;
-}

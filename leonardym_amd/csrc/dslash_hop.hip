@@ -25,10 +25,6 @@
 
 namespace lym {
 
-constexpr int HOP_LANES = 64;
-constexpr int HOP_WAVES = 4;  // one per direction, and two chirality waves
-constexpr int HOP_THREADS = HOP_LANES * (HOP_WAVES + 2);
-
 // n / d for 0 <= n < 2^27 by the reciprocal: (n + 1/2) / d lies at least
 // 1 / (2 d) from an integer, far more than the rounding of the product
 __device__ __forceinline__ int div_by(int n, double inv) { return (int)fma((double)n, inv, 0.5 * inv); }

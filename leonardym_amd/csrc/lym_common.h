@@ -195,7 +195,7 @@ __device__ __forceinline__ int site_parity(const Geom& g, const int c[4]) { retu
 // XCD-aware block order: MI355X deals workgroups round-robin over its 8 XCDs;
 // remapping gives each XCD a contiguous range of sites, so neighbour spinors
 // and links fetched by one XCD are reused from that XCD's own L2.
-__device__ __forceinline__ int xcd_block(int b, int nb) {
+__host__ __device__ __forceinline__ int xcd_block(int b, int nb) {
     const int nx = 8;
     int q = nb / nx, r = nb % nx;
     int xcd = b % nx, k = b / nx;

@@ -203,7 +203,7 @@ __device__ __forceinline__ void f64_step(const DslashParams& a, int p, int k, un
 // neighbour spinors and links of that slab are reused from its L2.  A
 // workgroup holds `spb` sites x `nr` right-hand sides, rhs fastest.
 // (The mapping functions take the workgroup index and grid size as arguments so
-// that the host can evaluate the same mapping: lym_launch_plan below.)
+// that the host can evaluate the same mapping: lym_launch_form.)
 struct BlockSweep {
     int lo, hi, k, nphys;
 };
@@ -230,7 +230,7 @@ __host__ __device__ __forceinline__ BlockSweep block_sweep_at(const DslashParams
     return b;
 }
 
-// Which renumbering block_of_at applied (reported by lym_launch_plan)
+// Which renumbering block_of_at applied (reported by lym_launch_form)
 enum { MAP_PLAIN = 0, MAP_XSLICE = 1, MAP_XCD_PAIRS = 2 };
 
 // logical block lb of the sweep of workgroup bx -> parity p and site block bi
@@ -277,15 +277,15 @@ __host__ __device__ __forceinline__ int block_of_at(const DslashParams& a, const
 
 // Workgroups of an FP64 launch over lanes, nw of them to a workgroup (a wave each): the
 // lanes of one site block follow one another on its XCD (links and blocks that one
-// lane reads are then in the L2 for the next).  Launcher: the grid; device: the
-// site block's workgroup bx of gd and the lane of wave w, false when there is nothing
-// to do.
+// lane reads are then in the L2 for the next).  Launcher: the grid; lane_of_block_at:
+// the site block's workgroup bx of gd and the lane of wave w, from the launch's
+// workgroup bx of gd; false when there is none; lane_of_block: also false when the
+// lane has nothing to do.
 static inline int lane_grid(const DslashParams& a, int nblocks, int nw) {
     return a.lanes > nw ? (nblocks + 7) / 8 * 8 * (a.lanes / nw) : nblocks;
 }
-__device__ __forceinline__ bool lane_of_block(const DslashParams& a, int nw, int w, int& bx, int& gd, int& lane) {
-    bx = (int)blockIdx.x;
-    gd = (int)gridDim.x;
+__host__ __device__ __forceinline__ bool lane_of_block_at(const DslashParams& a, int nw, int w, int& bx, int& gd,
+                                                          int& lane) {
     lane = w;
     if (a.lanes > nw) {
         const int t = bx >> 3, ng = a.lanes / nw, u = t / ng;
@@ -294,8 +294,20 @@ __device__ __forceinline__ bool lane_of_block(const DslashParams& a, int nw, int
         gd = a.grid1;
         if (bx >= gd) return false;
     }
+    return true;
+}
+__device__ __forceinline__ bool lane_of_block(const DslashParams& a, int nw, int w, int& bx, int& gd, int& lane) {
+    bx = (int)blockIdx.x;
+    gd = (int)gridDim.x;
+    if (!lane_of_block_at(a, nw, w, bx, gd, lane)) return false;
     return !(a.lane_flags && a.lane_flags[lane] == a.lane_skip_value);
 }
+
+// the one-wave-per-direction form (dslash_hop.hip): up to HOP_LANES (site, RHS) lanes,
+// HOP_WAVES direction waves over them and two chirality waves
+constexpr int HOP_LANES = 64;
+constexpr int HOP_WAVES = 4;
+constexpr int HOP_THREADS = HOP_LANES * (HOP_WAVES + 2);
 
 __device__ __forceinline__ BlockSweep block_sweep(const DslashParams& a) {
     return block_sweep_at(a, (int)blockIdx.x, (int)gridDim.x);

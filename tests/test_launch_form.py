@@ -1,0 +1,99 @@
+"""What the stencil's launches run, chosen on the host by the library's own selection
+(lym_launch_form; no GPU): every form visits every site block once per right-hand
+side, and the lattices that the GPU tests name for a form and a block order take them.
+"""
+import itertools
+
+import numpy as np
+import pytest
+
+import leonardym_amd as lym
+
+# (dims, parity, form, orders with blocks in them: plain, x-slice fastest, XCD pairs)
+FP64_FIELD = [
+    # four waves to a workgroup, each order: all workgroups at once, and sweeping
+    ((4, 14, 22, 40), -1, lym.FORM_STAGED, (1, 0, 0)),
+    ((16, 4, 28, 32), -1, lym.FORM_STAGED, (0, 1, 0)),
+    ((8, 8, 28, 32), -1, lym.FORM_STAGED, (0, 0, 1)),
+    ((4, 22, 28, 40), -1, lym.FORM_STAGED, (1, 0, 0)),
+    ((40, 4, 16, 40), -1, lym.FORM_STAGED, (0, 1, 0)),
+    ((8, 16, 26, 32), -1, lym.FORM_STAGED, (0, 0, 1)),
+    # ranges that split x-slices
+    ((98, 4, 4, 32), -1, lym.FORM_STAGED, (1, 1, 0)),
+    ((194, 4, 4, 32), -1, lym.FORM_STAGED, (1, 1, 0)),
+    ((98, 4, 8, 32), 1, lym.FORM_STAGED, (1, 1, 0)),
+    ((4, 22, 28, 40), 1, lym.FORM_STAGED, (1, 0, 0)),
+    ((40, 4, 16, 40), 1, lym.FORM_STAGED, (0, 1, 0)),
+    ((8, 16, 26, 32), 1, lym.FORM_STAGED, (0, 0, 1)),
+    # one wave to a workgroup
+    ((10, 10, 10, 40), -1, lym.FORM_WAVE, (1, 0, 0)),
+    ((16, 4, 14, 48), -1, lym.FORM_WAVE, (0, 1, 0)),
+    ((8, 4, 32, 40), -1, lym.FORM_WAVE, (0, 0, 1)),
+    ((6, 14, 28, 28), 1, lym.FORM_WAVE, (1, 0, 0)),
+    ((40, 4, 16, 26), 1, lym.FORM_WAVE, (0, 1, 0)),
+    ((8, 8, 22, 48), 1, lym.FORM_WAVE, (0, 0, 1)),
+    ((17, 15, 13, 21), 0, lym.FORM_WAVE, (1, 0, 0)),
+    ((14, 14, 14, 14), -1, lym.FORM_WAVE, (1, 0, 0)),
+    # the benchmark's apply and the largest lattice
+    ((16, 16, 16, 32), -1, lym.FORM_STAGED, (0, 0, 1)),
+    ((32, 32, 32, 64), -1, lym.FORM_STAGED, (0, 0, 1)),
+]
+
+
+@pytest.mark.parametrize("dims,parity,form,orders", FP64_FIELD, ids=lambda v: str(v).replace(", ", "x"))
+def test_fp64_field(dims, parity, form, orders):
+    r = lym.launch_form(dims, parity)
+    assert (r["form"], tuple(int(b > 0) for b in r["branches"])) == (form, orders), r["branches"]
+
+
+@pytest.mark.parametrize("dims,parity,prec,nrhs,form", [
+    # FP64: 32768 lanes of one field, whichever the parities
+    ((16, 16, 16, 16), 0, 0, 1, lym.FORM_HOP), ((16, 16, 16, 8), -1, 0, 1, lym.FORM_HOP),
+    ((16, 16, 16, 18), 0, 0, 1, lym.FORM_WAVE), ((16, 16, 16, 10), -1, 0, 1, lym.FORM_WAVE),
+    ((16, 16, 16, 24), 0, 0, 1, lym.FORM_WAVE),
+    # low precision: 49152 of one parity, 32768 of both, over the right-hand sides
+    ((16, 16, 16, 24), 0, 1, 1, lym.FORM_HOP), ((16, 16, 16, 24), 0, 2, 1, lym.FORM_HOP),
+    ((16, 16, 16, 26), 0, 1, 1, lym.FORM_SPLIT), ((16, 16, 16, 26), 0, 2, 1, lym.FORM_SPLIT),
+    ((16, 16, 16, 8), -1, 2, 1, lym.FORM_HOP), ((16, 16, 16, 10), -1, 2, 1, lym.FORM_SPLIT),
+    ((12, 12, 12, 12), 0, 2, 4, lym.FORM_HOP), ((12, 12, 12, 12), 0, 2, 6, lym.FORM_SITE),
+    # two threads per site up to 131072 sites of a parity
+    ((16, 16, 32, 32), 0, 1, 1, lym.FORM_SPLIT), ((16, 18, 32, 32), 0, 1, 1, lym.FORM_SITE),
+])
+def test_limits(dims, parity, prec, nrhs, form):
+    assert lym.launch_form(dims, parity, prec, nrhs, single=nrhs == 1)["form"] == form
+
+
+def test_matrix_cores():
+    for nrhs in (2, 4, 8):
+        assert lym.launch_form((8, 8, 8, 8), 0, 2, nrhs, matrix_cores=True)["form"] == lym.FORM_MFMA
+    for prec, nrhs in ((2, 3), (2, 16), (1, 4)):
+        assert lym.launch_form((8, 8, 8, 8), 0, prec, nrhs, matrix_cores=True)["form"] == lym.FORM_SITE
+
+
+def test_every_block_once():
+    seen = set()
+    lattices = [(4, 4, 4, 4), (6, 6, 6, 8), (4, 6, 2, 8), (12, 12, 12, 12), (18, 4, 4, 32), (14, 14, 14, 14),
+                (16, 16, 16, 32), (10, 12, 14, 22), (98, 4, 4, 32), (24, 24, 24, 32), (5, 7, 3, 6), (17, 15, 13, 21)]
+    options = [dict(nrhs=1), dict(nrhs=1, single=True), dict(nrhs=1, lane_ops=True), dict(nrhs=2),
+               dict(nrhs=2, matrix_cores=True), dict(nrhs=3), dict(nrhs=4, lane_ops=True), dict(nrhs=6, threads=192),
+               dict(nrhs=8, threads=64), dict(nrhs=12), dict(nrhs=16)]
+    for dims, parity, prec, kw in itertools.product(lattices, (-1, 0, 1), (0, 1, 2), options):
+        odd = any(d % 2 for d in dims)
+        if odd and (parity or kw["nrhs"] > 1 or prec):
+            continue  # one site class, FP64 launches of one field
+        r = lym.launch_form(dims, parity, prec, **kw)
+        want = np.zeros_like(r["visits"])
+        want[[0, 1] if parity < 0 else [parity]] = 1 if prec else kw["nrhs"]
+        assert np.array_equal(r["visits"], want), (dims, parity, prec, kw)
+        per_class = int(np.prod(dims)) // (1 if odd else 2)
+        assert r["spb"] * r["nbpp"] >= per_class > r["spb"] * (r["nbpp"] - 1)
+        assert r["threads"] <= 512 and r["partials"] == 0
+        seen.add(r["form"])
+    assert seen == set(range(7))
+
+
+def test_bad_arguments():
+    for kw in (dict(prec=3), dict(nrhs=0), dict(nrhs=17), dict(threads=-1), dict(threads=1024), dict(part_max=-1),
+               dict(parity=2), dict(dims=(1, 4, 4, 4)), dict(dims=(5, 4, 4, 4), parity=1)):
+        with pytest.raises(lym.LymError):
+            lym.launch_form(**{"dims": (4, 4, 4, 4), **kw})
