@@ -164,7 +164,8 @@ int lym_op_multiply_sloppy(lym_op* op, int prec, lym_spinor* out, const lym_spin
  * (no counterpart in the reference; the sloppy operator of the batched
  * solver): nrhs one of 1, 2, 3, 4, 6, 8, 12, 16.  matrix_cores = 1 runs the
  * FP16 SU(3) stencil's link products on the MFMA units (nrhs 2, 4 or 8;
- * LYM_ERR_UNSUPPORTED otherwise). */
+ * LYM_ERR_UNSUPPORTED otherwise), on lattices of up to 7456540 sites per parity;
+ * larger ones run the vector form. */
 int lym_op_multiply_sloppy_batch(lym_op* op, int prec, int matrix_cores, unsigned nrhs, lym_spinor* const* outs,
                                  const lym_spinor* const* ins);
 /* multiplyAdd (DiracOperator.h:99): out = Op v1 + alpha v2 */

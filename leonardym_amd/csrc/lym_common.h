@@ -43,6 +43,17 @@ __host__ __device__ constexpr int link_bytes(int prec, bool real, int rows) {
     return (3 * rows * (real ? 1 : 2) * (prec == 1 ? 4 : 2) + 3) / 4 * 4;
 }
 
+// Bytes from its wave-uniform base that a buffer instruction of the field access
+// (lym_device.h) reaches: loads past them return zero
+constexpr long BUF_RANGE = 0x7fffffff;
+
+// Whether the lanes of the matrix-core stencil reach all they load at this stride: any
+// entry of the packed FP16 links from the field's base, any component of an
+// interleaved FP16 spinor of nr right-hand sides from its site's
+constexpr bool mfma_reach(long stride, int nr) {
+    return 8 * stride * link_bytes(2, false, 3) <= BUF_RANGE && (32 * stride + 16) * nr <= BUF_RANGE;
+}
+
 // Device site order.  0: t fastest (the reference's lexicographic order; the
 // even-odd split needs Lt even).  1: t slowest, x fastest (needs Lx even): the
 // contiguous site range each XCD works on is then a slab of whole t-slices,

@@ -135,7 +135,7 @@ __device__ __forceinline__ E* lane_at(E* ubase, unsigned lane_elems) {
 #if LYM_BUFFER_LOADS
 // raw buffer resource for gfx9-family (gfx950): stride 0, 2 GiB range
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, 0x7fffffff, 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)BUF_RANGE, 0x00020000);
 }
 // cache policy bits of the buffer instructions: 2 = non-temporal
 template <class E, int AUX = 0>

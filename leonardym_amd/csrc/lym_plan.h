@@ -51,11 +51,11 @@ inline int lane_waves(const DslashParams& a) {
     return 1;
 }
 
-// The matrix-core form: FP16 SU(3) batches of 2, 4 or 8 RHS in whole waves (its
-// lanes address the links by 32-bit byte offsets)
+// The matrix-core form: FP16 SU(3) batches of 2, 4 or 8 RHS in whole waves, on lattices
+// whose links its lanes reach
 inline bool takes_mfma(const DslashParams& a) {
-    return a.mfma && !a.bmode && 8L * a.g.stride * link_bytes(2, false, 3) < (1L << 32) &&
-           (a.nr == 2 || a.nr == 4 || a.nr == 8) && (a.spb * a.nr) % 64 == 0;
+    return a.mfma && !a.bmode && mfma_reach(a.g.stride, a.nr) && (a.nr == 2 || a.nr == 4 || a.nr == 8) &&
+           (a.spb * a.nr) % 64 == 0;
 }
 
 // Launch geometry: sites per workgroup, the split form, site blocks per parity

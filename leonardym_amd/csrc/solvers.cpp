@@ -820,7 +820,7 @@ int autotune_batch(lym_solver* s, lym_op* op, bool half, int prec, unsigned nrhs
         if (nr > maxnr) continue;
         double best = 1e300;
         for (int form = 0; form < 2; ++form) {
-            if (form == 1 && !(mfma_ok && (nr == 4 || nr == 8))) continue;
+            if (form == 1 && !(mfma_ok && (nr == 4 || nr == 8) && lym::mfma_reach(c->g.stride, nr))) continue;
             for (int thr : {64, 128, 256}) {
                 if (thr < nr) continue;
                 BatchOp B{op, half, 1, 1, nr, thr, s->bsv[2], s->bsvsc[2], s->bsv[3], s->bsvsc[3]};
@@ -1178,6 +1178,7 @@ int lym_solver_solve_batch(lym_solver* s, lym_op* op, unsigned nrhs, const lym_s
         s->tuned_nr = nr;
         s->tuned_threads = thr;
     }
+    mfma = mfma && lym::mfma_reach(c->g.stride, nr);
     s->tuned_mfma = mfma;
     HIPCHECK(hipEventRecord(c->ev_start, c->stream));
     for (unsigned q0 = 0; q0 < nrhs; q0 += nr) {

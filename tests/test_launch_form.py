@@ -97,3 +97,17 @@ def test_bad_arguments():
                dict(parity=2), dict(dims=(1, 4, 4, 4)), dict(dims=(5, 4, 4, 4), parity=1)):
         with pytest.raises(lym.LymError):
             lym.launch_form(**{"dims": (4, 4, 4, 4), **kw})
+
+
+@pytest.mark.parametrize("dims,nrhs,form", [
+    # the lanes of the matrix-core form reach a link entry at 288 bytes a site of a parity,
+    # a spinor component at 32 bytes a (site, right-hand side), and a buffer holds 2^31 - 1
+    ((60, 60, 64, 64), 2, lym.FORM_MFMA), ((60, 60, 64, 64), 8, lym.FORM_MFMA),
+    ((60, 62, 64, 64), 2, lym.FORM_SITE), ((60, 62, 64, 64), 8, lym.FORM_SITE), ((64, 64, 64, 64), 4, lym.FORM_SITE),
+])
+def test_matrix_cores_within_a_buffer(dims, nrhs, form):
+    for parity in (-1, 0):
+        r = lym.launch_form(dims, parity, 2, nrhs, matrix_cores=True)
+        assert r["form"] == form and np.all(r["visits"][0] == 1)
+    sites = int(np.prod(dims)) // 2
+    assert (288 * sites <= 0x7fffffff and 32 * sites * nrhs <= 0x7fffffff) == (form == lym.FORM_MFMA)
