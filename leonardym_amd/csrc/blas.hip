@@ -459,9 +459,11 @@ void launch_bicg_setup(zd* r, zd* rh, zd* p, zd* nu, const zd* b, const zd* Ax, 
 
 // Each of the p, s and x/r updates below folds the partial sums of the step
 // before it in every workgroup (a fixed order, so all get the same value);
-// workgroup 0 writes the state, and no workgroup reads what it writes except
-// `done` at the start (read once per workgroup: after a stop decided there a
-// vector may be left partly updated, which nothing reads).
+// workgroup 0 writes the state.  No other workgroup reads what it writes, but for
+// two members: `done` (once per workgroup, at the start: a workgroup that starts
+// after a stop returns at once and leaves its part of a vector as it was, so a
+// kernel whose vector is still to be read never sets it), and `step` in the p
+// update, which changes there only when every workgroup returns without updating.
 #define BICG_STOP_CHECK()                        \
     __shared__ int stop_;                        \
     if (threadIdx.x == 0) stop_ = s->done;      \
@@ -493,6 +495,10 @@ __global__ __launch_bounds__(RB_THREADS) void k_bicg_p(BiCGState* s, zd* __restr
                                                        int stride, int npart) {
     BICG_STOP_CHECK();
     const bool wr = blockIdx.x == 0 && threadIdx.x == 0;
+    if (s->copy_b) {  // the last update copied the source into x: the solve is over
+        if (wr) s->done = 1;
+        return;
+    }
     const int phase = s->phase, step = s->step;
     double pl[3];
     fold_load<3>(partials, stride, npart, pl);
@@ -568,8 +574,7 @@ __global__ __launch_bounds__(RB_THREADS) void k_bicg_update(BiCGState* s, zd* __
     fold_block<3>(pl, out);
     if (out[2] == 0.0) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
-            s->copy_b = 1;
-            s->done = 1;
+            s->copy_b = 1;  // (`done` by the next p update or launch_bicg_check)
             s->converged = 1;
         }
         GRID_LOOP(i, n) { x[i] = b[i]; }
@@ -601,6 +606,10 @@ void launch_bicg_update(BiCGState* s, zd* x, zd* r, const zd* rh, const zd* p, c
 __global__ __launch_bounds__(RB_THREADS) void k_bicg_check(BiCGState* s, const double* partials, int stride,
                                                            int npart) {
     if (s->done || s->phase != BICG_FOLD) return;
+    if (s->copy_b) {
+        if (threadIdx.x == 0) s->done = 1;
+        return;
+    }
     double pl[3], out[3];
     fold_load<3>(partials, stride, npart, pl);
     fold_block<3>(pl, out);
