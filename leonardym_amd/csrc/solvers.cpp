@@ -934,7 +934,7 @@ int run_batch(lym_solver* s, lym_op* op, bool eo, bool half, int nr, int thr, in
     unsigned queued = 0;
     // steps are queued in chunks; those queued after the last RHS stopped exit at once
     Key key;
-    key << 4 << s << nr << thr << prec << eo << half << g5 << pw << x << r << b << Ax << mid << tmp << a.xs << a.rs
+    key << 4 << s << nr << thr << mfma << prec << eo << half << g5 << pw << x << r << b << Ax << mid << tmp << a.xs << a.rs
         << a.p << a.Ap << a.p_sc << a.Ap_sc << a.nsites << HS.mid << HS.tmp << HS.mid_sc << HS.tmp_sc;
     key_op(key, op);
     // The even-odd sloppy Qhat^2 p with the CG's two sums fused into its
