@@ -396,8 +396,8 @@ int lym_launch_plan(const int dims[4], int parity, int nr, int threads, int lowp
  * right-hand sides (FP64: fields of their own); parity and threads as above;
  * options: LYM_LAUNCH_SINGLE for the low-precision applies of one right-hand side
  * (not of a batch), LYM_LAUNCH_MATRIX_CORES, LYM_LAUNCH_LANE_OPS for a kappa per
- * right-hand side; step 1: a launch that also leaves partial sums, part_max of
- * them at most.  SU(3) links of three rows.
+ * right-hand side; step 1: a launch that also leaves partial sums of its output, 2:
+ * one that runs the conjugate gradient's update, part_max partial sums at most.  SU(3) links of three rows.
  * visits (2 * nbpp ints, or NULL) counts how often each (parity, block) is
  * visited: once per right-hand side of an FP64 launch, else once. */
 enum {
@@ -416,7 +416,7 @@ typedef struct {
     int threads;     /* threads per workgroup */
     int spb;         /* sites per workgroup (LYM_FORM_LANES: per wave) */
     int nbpp;        /* site blocks per parity */
-    int partials;    /* partial sums left (0: step 0, or more than part_max) */
+    int partials;    /* partial sums left (0: step 0, or the launch does not take the step) */
     int branches[3]; /* blocks in plain order, x-slice fastest, XCD pairs */
 } lym_launch_info;
 int lym_launch_form(const int dims[4], int parity, int prec, int nrhs, int threads, int options, int step,

@@ -192,7 +192,7 @@ class LaunchInfo(ctypes.Structure):
 
 
 def launch_form(dims, parity=-1, prec=0, nrhs=1, threads=0, single=False, matrix_cores=False, lane_ops=False,
-                step=False, part_max=0):
+                step=0, part_max=0):
     """The form, workgroups and block order one stencil launch takes, chosen on
     the host by the library's own selection (no device needed): dict with form
     (FORM_*), grid, threads, spb, nbpp, partials, branches (plain, x-slice, XCD

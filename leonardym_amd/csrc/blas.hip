@@ -457,6 +457,20 @@ void launch_bicg_setup(zd* r, zd* rh, zd* p, zd* nu, const zd* b, const zd* Ax, 
                        stride);
 }
 
+__global__ __launch_bounds__(RB_THREADS) void k_bicg_dot(const BiCGState* s, const zd* __restrict__ w,
+                                                         const zd* __restrict__ v, long n, double* partials,
+                                                         int stride) {
+    if (s->done) return;
+    double t[3] = {0, 0, 0};
+    GRID_LOOP(i, n) { bicg_terms(w[i], v[i], t); }
+    block_store<3>(t, partials, stride);
+}
+
+void launch_bicg_dot(const BiCGState* s, const zd* w, const zd* v, long n, double* partials, int stride,
+                     hipStream_t st) {
+    hipLaunchKernelGGL(k_bicg_dot, dim3(RED_BLOCKS), dim3(RB_THREADS), 0, st, s, w, v, n, partials, stride);
+}
+
 // Each of the p, s and x/r updates below folds the partial sums of the step
 // before it in every workgroup (a fixed order, so all get the same value);
 // workgroup 0 writes the state.  No other workgroup reads what it writes, but for

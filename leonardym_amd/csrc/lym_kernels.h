@@ -192,10 +192,12 @@ void launch_cg_init(CGState* s, const zd* r, long n, double* partials, double ep
 // The steps of an iteration that are not fused into the stencil fold npart
 // partial sums of the step before (sum k of workgroup b at part[k * stride + b]).
 // launch_fold folds more than FOLD_MAX of them into one; npart and part then
-// describe the result.
+// describe the result.  A stencil launch that does not take its fused step leaves
+// none, and the caller runs the step by itself: launch_bicg_dot, or launch_cg_alpha and
+// launch_cg_update.
 constexpr int FOLD_MAX = 2048;
 void launch_fold(int nv, const double*& part, int stride, int& npart, double* out, const int* skip, hipStream_t st);
-// one CG iteration after Ap = A p, for maps whose <p, Ap> is not |Q p|^2: <p, Ap>
+// one CG iteration after Ap = A p, where it is not fused into the stencil: <p, Ap>
 // partials (slots 0, 1 of partials), the update folding them into alpha (|r|^2
 // partials into slot 2)
 void launch_cg_alpha(CGState* s, const zd* p, const zd* Ap, long n, double* partials, hipStream_t st);
@@ -218,6 +220,9 @@ void launch_bicg_s(BiCGState* s, zd* sv, const zd* r, const zd* nu, long n, cons
                    hipStream_t st);
 void launch_bicg_update(BiCGState* s, zd* x, zd* r, const zd* rh, const zd* p, const zd* sv, const zd* t, const zd* b,
                         long n, const double* part, int stride, int npart, double* partials, hipStream_t st);
+// <w, v> and |v|^2 into RED_BLOCKS partials, for a stencil launch that did not
+void launch_bicg_dot(const BiCGState* s, const zd* w, const zd* v, long n, double* partials, int stride,
+                     hipStream_t st);
 // the stopping rule of the last update, before the host reads the state
 void launch_bicg_check(BiCGState* s, const double* partials, int stride, hipStream_t st);
 

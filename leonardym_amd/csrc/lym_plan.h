@@ -166,15 +166,18 @@ inline LaunchPlan plan_launch(DslashParams& a, int link_kind, int diag, bool inv
     const bool whole_waves = L.form == LYM_FORM_HOP || threads % 64 == 0;
     if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || !whole_waves || L.nblocks > a.norm_max)
         a.norm_partials = nullptr;
-    // the fused update: under the same conditions (the caller checks the return
-    // value and runs the separate update when it is 0)
-    if (a.prec == 0 || diag == 0 || inv || a.nr != 1 || a.lane_flags || a.lane_ops || !whole_waves ||
-        L.nblocks > a.norm_max || a.norm_partials)
-        if (!a.fmode) a.upd_state = nullptr;
     // the FP64 solvers' fused steps: one RHS, a diagonal and no R^-1, and room for
-    // one partial per workgroup
+    // one partial per workgroup (the caller checks the return value and runs the
+    // separate step when it is 0)
     if (a.prec != 0 || diag == 0 || inv || a.lanes > 1 || a.lane_flags || a.lane_ops || L.nblocks > a.part_stride)
         a.fmode = F64_STORE;
+    // the fused update: FP64 F64_CG; low precision under the same conditions
+    if (a.prec == 0) {
+        if (a.fmode != F64_CG) a.upd_state = nullptr;
+    } else if (diag == 0 || inv || a.nr != 1 || a.lane_flags || a.lane_ops || !whole_waves ||
+               L.nblocks > a.norm_max || a.norm_partials) {
+        a.upd_state = nullptr;
+    }
     L.partials = a.norm_partials || a.upd_state || a.fmode ? L.nblocks : 0;
     return L;
 }

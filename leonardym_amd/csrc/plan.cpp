@@ -70,7 +70,7 @@ extern "C" int lym_launch_form(const int dims[4], int parity, int prec, int nrhs
     using lym_internal::fail;
     if (!dims || !info) return fail(LYM_ERR_INVALID, "null argument");
     if (prec < 0 || prec > 2 || nrhs < 1 || nrhs > 16 || threads < 0 || threads > LYM_DSLASH_THREADS || step < 0 ||
-        step > 1 || part_max < 0 || (options & ~(LYM_LAUNCH_SINGLE | LYM_LAUNCH_MATRIX_CORES | LYM_LAUNCH_LANE_OPS)))
+        step > 2 || part_max < 0 || (options & ~(LYM_LAUNCH_SINGLE | LYM_LAUNCH_MATRIX_CORES | LYM_LAUNCH_LANE_OPS)))
         return fail(LYM_ERR_INVALID, "bad launch arguments");
     lym::DslashParams a;
     if (const int rc = plan_geometry(dims, parity, a)) return rc;
@@ -81,9 +81,10 @@ extern "C" int lym_launch_form(const int dims[4], int parity, int prec, int nrhs
     a.allow_split = prec && (options & LYM_LAUNCH_SINGLE);
     a.mfma = (options & LYM_LAUNCH_MATRIX_CORES) ? 1 : 0;
     a.lane_ops = (options & LYM_LAUNCH_LANE_OPS) ? 1 : 0;
-    double part;  // (its address only: partials are asked for)
-    if (step && prec == 0) a.fmode = lym::F64_NORM;
-    if (step && prec) a.norm_partials = &part;
+    double part;  // (its address only: the step is asked for)
+    if (step && prec == 0) a.fmode = step == 2 ? lym::F64_CG : lym::F64_NORM;
+    if (step == 1 && prec) a.norm_partials = &part;
+    if (step == 2) a.upd_state = &part;
     a.part_stride = a.norm_max = part_max;
     const lym::LaunchPlan L = lym::plan_launch(a, 0, 1, false);
     std::memset(info, 0, sizeof(*info));

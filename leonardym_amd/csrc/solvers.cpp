@@ -345,6 +345,14 @@ double read_norm2(lym_ctx* c, const zd* v, long n) {
     return out;
 }
 
+// LYM_FUSED_FP64=0: no room for the partial sums of the FP64 solvers' steps fused into
+// the stencil, so that every launch leaves them to launches of their own (for
+// comparison)
+int fused64_room(const lym_solver* s) {
+    const char* e = std::getenv("LYM_FUSED_FP64");
+    return e && e[0] == '0' ? 0 : s->dot_stride;
+}
+
 // CG on L (ConjugateGradient.cpp:10-74): vectors of length n
 int run_cg(lym_solver* s, const LinOp& L, const zd* b, zd* xout, const zd* x0, long n, lym_solve_info* info) {
     lym_ctx* c = s->ctx;
@@ -370,22 +378,27 @@ int run_cg(lym_solver* s, const LinOp& L, const zd* b, zd* xout, const zd* x0, l
     // A p, which then does not store it
     const bool fused = L.power == 2 && L.gamma5 && !L.shifted();
     const int* done = &S->done;
+    const int ds = s->dot_stride, room = fused64_room(s);
+    key << room;
     auto body = [&](unsigned) {
         const double* part = c->red_partials + 2 * lym::RED_BLOCKS;
-        int npart = lym::RED_BLOCKS;
+        int npart = 0;
         if (fused) {
-            lym::Fuse64 f{lym::F64_NORM, s->dot_part, s->dot_stride};
+            lym::Fuse64 f{lym::F64_NORM, s->dot_part, room};
             int nd = L.first(p, done, &f);
             const double* dot = s->dot_part;
-            lym::launch_fold(1, dot, s->dot_stride, nd, s->dot_part + 3 * (size_t)s->dot_stride, done, st);
-            f = {lym::F64_CG, s->dot_part + s->dot_stride, s->dot_stride, nullptr, S, dot, nd, p, x, r};
-            npart = L.second(Ap, p, done, &f);
-            part = f.part;
-            lym::launch_fold(1, part, s->dot_stride, npart, s->dot_part + 4 * (size_t)s->dot_stride, done, st);
+            lym::launch_fold(1, dot, ds, nd, s->dot_part + 3 * (size_t)ds, done, st);
+            f = {lym::F64_CG, s->dot_part + ds, room, nullptr, S, dot, nd, p, x, r};
+            npart = L.second(Ap, p, done, nd ? &f : nullptr);
+            if (npart) part = f.part;
+            lym::launch_fold(1, part, ds, npart, s->dot_part + 4 * (size_t)ds, done, st);
         } else {
             L.apply(Ap, p, done);
+        }
+        if (!npart) {
             lym::launch_cg_alpha(S, p, Ap, n, c->red_partials, st);
             lym::launch_cg_update(S, x, r, p, Ap, n, c->red_partials, st);
+            npart = lym::RED_BLOCKS;
         }
         lym::launch_cg_p(S, p, r, n, part, npart, st);
     };
@@ -441,18 +454,28 @@ int run_bicgstab(lym_solver* s, const LinOp& L, const zd* b, zd* xout, const zd*
     key_op(key, L.op);
     key << L.half << L.gamma5 << L.power << L.scratch << L.shift.re << L.shift.im;
     const int* done = &S->done;
-    auto body = [&](unsigned) {
-        lym::launch_bicg_p(S, p, r, nu, n, part, ds, st);
-        // <rh, nu>, then <s, t> and |t|^2, summed by the launches that write nu and t
-        lym::Fuse64 f{lym::F64_DOT, s->dot_part, ds, rh};
-        const double* dot = s->dot_part;
-        int nd = L.apply(nu, p, done, &f);
-        lym::launch_fold(3, dot, ds, nd, s->dot_part + 3 * (size_t)ds, done, st);
-        lym::launch_bicg_s(S, sv, r, nu, n, dot, ds, nd, st);
-        f.w = sv;
+    const int room = fused64_room(s);
+    key << room;
+    // out = A in with <w, out> and |out|^2 summed by the launch that writes out (or by
+    // one of their own); dot, nd: the partials to fold
+    auto apply_dot = [&](zd* out, const zd* in, const zd* w, const double*& dot, int& nd) {
+        // (the sums' stride is the room where the launch takes the step)
+        const lym::Fuse64 f{lym::F64_DOT, s->dot_part, room, w};
         dot = s->dot_part;
-        nd = L.apply(t, sv, done, &f);
+        nd = L.apply(out, in, done, &f);
+        if (!nd) {
+            lym::launch_bicg_dot(S, w, out, n, s->dot_part, ds, st);
+            nd = lym::RED_BLOCKS;
+        }
         lym::launch_fold(3, dot, ds, nd, s->dot_part + 3 * (size_t)ds, done, st);
+    };
+    auto body = [&](unsigned) {
+        const double* dot;
+        int nd;
+        lym::launch_bicg_p(S, p, r, nu, n, part, ds, st);
+        apply_dot(nu, p, rh, dot, nd);
+        lym::launch_bicg_s(S, sv, r, nu, n, dot, ds, nd, st);
+        apply_dot(t, sv, sv, dot, nd);
         lym::launch_bicg_update(S, x, r, rh, p, sv, t, b, n, dot, ds, nd, part, st);
     };
     while (!H->done && queued <= s->max_steps) {

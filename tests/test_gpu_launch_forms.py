@@ -65,6 +65,30 @@ def test_fused_steps(dims, swept, method, power):
         assert np.linalg.norm(x.download() - ref) < 1e-11 * np.linalg.norm(ref), steps
 
 
+@pytest.mark.parametrize("method,kind,power", [("cg", "wilson", 2), ("bicgstab", "clover", 1), ("cg", "eo", 2),
+                                               ("bicgstab", "eo", 2)])
+@pytest.mark.parametrize("dims", [(6, 4, 4, 6), (12, 12, 12, 24)])
+def test_steps_not_fused(dims, method, kind, power, monkeypatch):
+    """The iterates where the stencil launches do not take the steps are those where they do
+    (rounding of the sums, carried over 9 steps)."""
+    V = int(np.prod(dims))
+    ctx = lym.Context(dims)
+    g = lym.Gauge(ctx, fold_bc(dims, lym.gen_su3_links(dims, 0.5, 61)), folded=True)
+    lkind = {"wilson": lym.OP_WILSON, "clover": lym.OP_CLOVER, "eo": lym.OP_EO_CLOVER}[kind]
+    op = lym.Operator(ctx, lkind, power, 0.12, 1.0, method == "cg" or power == 2, gauge=g)
+    b = lym.Spinor(ctx, lym.gaussian_spinor(V, 62))
+    s = lym.Solver(ctx, lym.SOLVER_CG if method == "cg" else lym.SOLVER_BICGSTAB, precision=1e-30, max_steps=9)
+    got = []
+    for on in ("1", "0", "1"):
+        print("steps fused", on, dims, method, kind, flush=True)
+        monkeypatch.setenv("LYM_FUSED_FP64", on)
+        x = lym.Spinor(ctx)
+        assert s.solve(op, b, x).steps == 9
+        got.append(x.download())
+    assert np.array_equal(got[0], got[2])
+    assert np.linalg.norm(got[1] - got[0]) < 1e-11 * np.linalg.norm(got[0])
+
+
 @pytest.mark.parametrize("prec", [lym.PREC_SINGLE, lym.PREC_HALF], ids=["fp32", "fp16"])
 def test_low_precision_half_lattice_at_the_limit(prec):
     dims = (16, 16, 16, 24)

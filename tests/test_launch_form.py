@@ -111,3 +111,33 @@ def test_matrix_cores_within_a_buffer(dims, nrhs, form):
         assert r["form"] == form and np.all(r["visits"][0] == 1)
     sites = int(np.prod(dims)) // 2
     assert (288 * sites <= 0x7fffffff and 32 * sites * nrhs <= 0x7fffffff) == (form == lym.FORM_MFMA)
+
+
+@pytest.mark.parametrize("prec", [0, 1, 2])
+@pytest.mark.parametrize("step", [1, 2])
+def test_a_step_without_room_is_not_taken(prec, step):
+    """A launch with more workgroups than the partial sums hold runs without the step and
+    says so; with room it leaves one per workgroup."""
+    for dims in ((4, 4, 4, 4), (12, 12, 12, 24), (16, 16, 16, 32), (24, 24, 24, 32)):
+        r = lym.launch_form(dims, -1, prec, single=True, step=step, part_max=1 << 20)
+        assert r["partials"] == r["grid"] > 1
+        assert lym.launch_form(dims, -1, prec, single=True, step=step, part_max=r["grid"])["partials"] == r["grid"]
+        assert lym.launch_form(dims, -1, prec, single=True, step=step, part_max=r["grid"] - 1)["partials"] == 0
+    # several right-hand sides, or a kappa each: never
+    assert lym.launch_form((8, 8, 8, 8), -1, prec, nrhs=2, step=step, part_max=1 << 20)["partials"] == 0
+    if step == 2 or prec == 0:
+        assert lym.launch_form((8, 8, 8, 8), -1, prec, lane_ops=True, step=step, part_max=1 << 20)["partials"] == 0
+
+
+def test_room_of_the_fp64_solvers():
+    """The FP64 solvers' partial sums (8192, or one per 256 sites of a lattice) hold those of
+    any launch of theirs."""
+    r = np.random.default_rng(5)
+    dims = [tuple(int(v) for v in r.integers(2, 40, 4)) for _ in range(150)]
+    dims += [(64, 64, 64, 64), (32, 32, 32, 64), (2, 2, 2, 2), (3, 3, 3, 3), (48, 48, 48, 96)]
+    for d in dims:
+        odd = any(x % 2 for x in d)
+        vh = int(np.prod(d)) // (1 if odd else 2)
+        for parity in (0,) if odd else (-1, 0, 1):
+            q = lym.launch_form(d, parity, step=2, part_max=max(8192, 2 * ((vh + 255) // 256)))
+            assert q["partials"] == q["grid"], (d, parity)
