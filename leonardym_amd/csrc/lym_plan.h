@@ -123,12 +123,14 @@ inline int plan_hop(DslashParams& a) {
 // 16^3x20 31.4 -> 24.6 us, 16^3x24 33.6 -> 30.1, 14^4 16.3 -> 15.1, 17x15x13x21
 // 31.7 -> 24.4, Schur complement 16x20^2x24 81.0 -> 68.6.  Above it the four waves are as
 // fast or faster: at 7 against 8 (16^3x28) 35.4 and 36.4, at 4 against 4 (15^4) 18.1 and
-// 18.7.  Returns the workgroups, or 0 when the launch keeps workgroups of four.
+// 18.7.  Launches over lanes always hold blocks of 64 sites, a wave each.  Returns the
+// workgroups (of one lane), or 0 when the launch keeps workgroups of four.
 inline int plan_waves(DslashParams& a) {
-    if (a.prec != 0 || LYM_DSLASH_THREADS != 256) return 0;
+    if (a.prec != 0) return 0;
     const int par = a.parity >= 0 ? 1 : 2;
     const int n4 = a.nblocks_per_parity * par, nb = (a.g.Vh + 63) / 64, n1 = nb * par;
     if (!over_lanes(a)) {
+        if (LYM_DSLASH_THREADS != 256) return 0;  // (the rule counts workgroups of four waves)
         if (n4 > LYM_SWEEP_MAX_BLOCKS || 5 * ((n1 + 255) / 256) > 16 * ((n4 + 255) / 256)) return 0;
         if (a.fmode && n1 > FOLD_MAX) return 0;  // a fold more would take what it gains
     }

@@ -2,10 +2,16 @@
 (lym_launch_form; no GPU): every form visits every site block once per right-hand
 side, and the lattices that the GPU tests name for a form and a block order take them.
 """
+import ctypes
 import itertools
+import os
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
+
+from helpers import ROOT
 
 import leonardym_amd as lym
 
@@ -141,3 +147,30 @@ def test_room_of_the_fp64_solvers():
         for parity in (0,) if odd else (-1, 0, 1):
             q = lym.launch_form(d, parity, step=2, part_max=max(8192, 2 * ((vh + 255) // 256)))
             assert q["partials"] == q["grid"], (d, parity)
+
+
+@pytest.mark.parametrize("width", [64, 128, 512])
+def test_other_workgroup_sizes(width, tmp_path):
+    """LYM_DSLASH_THREADS is a build option: with another value every form still visits
+    every block once per right-hand side (the selection alone, built with it)."""
+    stub, so = tmp_path / "fail.cpp", tmp_path / "plan.so"
+    stub.write_text("namespace lym_internal { int fail(int code, const char*, ...) { return code; } }\n")
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    subprocess.check_call([hipcc, "-x", "hip", "--offload-host-only", "-std=c++17", "-fPIC", "-shared", "-w",
+                           "-DLYM_DSLASH_THREADS=%d" % width,
+                           os.path.join(ROOT, "leonardym_amd", "csrc", "plan.cpp"), str(stub), "-o", str(so)])
+    call = ctypes.CDLL(str(so)).lym_launch_form
+    call.argtypes = lym.SIGNATURES["lym_launch_form"][1]
+    for dims, parity, prec, nrhs in itertools.product([(4, 4, 4, 4), (12, 12, 12, 24), (16, 16, 16, 32), (10, 12, 14, 22)],
+                                                      (-1, 0, 1), (0, 1, 2), (1, 2, 3, 4, 6, 8, 12, 16)):
+        info = lym.LaunchInfo()
+        args = (np.array(dims, np.int32).ctypes.data, parity, prec, nrhs, 0, 0, 0, 0, ctypes.byref(info))
+        assert call(*args, None, 0) == 0
+        visits = np.zeros((2, info.nbpp), np.int32)
+        assert call(*args, visits.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), visits.size) == 0
+        want = np.zeros_like(visits)
+        want[[0, 1] if parity < 0 else [parity]] = 1 if prec else nrhs
+        assert np.array_equal(visits, want), (dims, parity, prec, nrhs)
+        assert info.spb * info.nbpp >= int(np.prod(dims)) // 2
+        if info.form == lym.FORM_LANES:
+            assert info.spb == 64  # what k_dslash_lanes covers, a wave
