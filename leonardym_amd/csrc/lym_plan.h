@@ -85,26 +85,41 @@ inline int plan_dslash(DslashParams& a) {
 
 // Launches of at most this many (site, RHS) lanes take the one-wave-per-direction
 // form (dslash_hop.hip); low-precision launches of one parity, whose other form
-// waits longest, more of them.  Measured, that form against the other: FP64 even-odd
+// waits longest, more of them, and FP64 launches over several lanes fewer: their other
+// form has a wave per lane for every 64 sites, which hide each other's waits.  Measured, that form against the other: FP64 even-odd
 // CG iteration 83 against 91 us at 32768 lanes, Schur complement 39.0 against 38.4 at
 // 40960 and 43.0 against 41.9 at 49152; full applies 10.2 against 13.6 us at 20736
 // lanes (clover), 14.3 against 12.5 us at 41472 (Wilson).  Low-precision Schur
 // complement at 41472 lanes of two RHS 14.2 against 21.9 us (FP16), 18.8 against 22.5
 // (FP32), at 49152 lanes of one 17.7 against 19.6 and 23.3 against 25.7; FP16 mixed CG
-// iteration 78 against 67 us at 65536.
+// iteration 78 against 67 us at 65536.  FP64 over lanes, by whole batched FP16 solves of
+// as many right-hand sides: four and more at 8192 lanes 3.13 against 3.24 ms (8^4, 4),
+// at 16384 4.37 against 4.20 (8^3x16, 4) and 3.56 against 3.47 (8^4, 8), at 82944 7.7
+// against 7.1 (12^4, 8), at 393216 21.1 against 19.1 (16^4, 12); two, whose other form
+// has half the waves, at 41472 4.99 against 5.02 (12^3x24; adjoint 4.58 and 4.67), at
+// 54880 6.51 against 6.37 (14^3x20), at 65536 6.74 against 6.50 (16^4).
 #ifndef LYM_HOP_MAX
 #define LYM_HOP_MAX 32768
 #endif
 #ifndef LYM_HOP_MAX_LOWP_HALF
 #define LYM_HOP_MAX_LOWP_HALF 49152
 #endif
+#ifndef LYM_HOP_MAX_FP64_LANES
+#define LYM_HOP_MAX_FP64_LANES 8192
+#endif
+#ifndef LYM_HOP_MAX_FP64_PAIR
+#define LYM_HOP_MAX_FP64_PAIR 49152
+#endif
 
 // The launch geometry of that form: sites per workgroup and site blocks per
 // parity; returns the number of workgroups, or 0 when the launch takes another.
 inline int plan_hop(DslashParams& a) {
     const int par = a.parity >= 0 ? 1 : 2;
-    const long lanes = (long)a.g.Vh * a.nr * par;
-    if (LYM_T_SLOW || a.mfma || a.nr > 64 || lanes > (par == 1 && a.prec ? LYM_HOP_MAX_LOWP_HALF : LYM_HOP_MAX)) return 0;
+    const int rhs = a.prec == 0 && a.lanes > 1 ? a.lanes : a.nr;
+    const long lanes = (long)a.g.Vh * par * rhs;
+    const long most = a.prec ? (par == 1 ? LYM_HOP_MAX_LOWP_HALF : LYM_HOP_MAX)
+                             : (rhs > 2 ? LYM_HOP_MAX_FP64_LANES : rhs == 2 ? LYM_HOP_MAX_FP64_PAIR : LYM_HOP_MAX);
+    if (LYM_T_SLOW || a.mfma || a.nr > 64 || lanes > most) return 0;
     a.spb = 64 / a.nr;
     // tiny launches: fewer sites per workgroup, so that more CUs share the loads
     while (a.spb > 1 && a.spb * a.nr > 16 && (a.g.Vh + a.spb - 1) / a.spb * par < 256) a.spb = (a.spb + 1) / 2;

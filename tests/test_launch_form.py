@@ -57,6 +57,11 @@ def test_fp64_field(dims, parity, form, orders):
     ((16, 16, 16, 16), 0, 0, 1, lym.FORM_HOP), ((16, 16, 16, 8), -1, 0, 1, lym.FORM_HOP),
     ((16, 16, 16, 18), 0, 0, 1, lym.FORM_WAVE), ((16, 16, 16, 10), -1, 0, 1, lym.FORM_WAVE),
     ((16, 16, 16, 24), 0, 0, 1, lym.FORM_WAVE),
+    # over several lanes 8192, over two 49152
+    ((8, 8, 8, 8), 0, 0, 4, lym.FORM_HOP), ((8, 8, 8, 8), 1, 0, 6, lym.FORM_LANES),
+    ((8, 8, 8, 16), 0, 0, 3, lym.FORM_LANES), ((16, 16, 16, 12), 1, 0, 2, lym.FORM_HOP),
+    ((12, 12, 12, 24), -1, 0, 2, lym.FORM_LANES), ((16, 16, 16, 14), 0, 0, 2, lym.FORM_LANES),
+    ((12, 12, 12, 24), 0, 0, 12, lym.FORM_LANES), ((4, 4, 4, 4), -1, 0, 16, lym.FORM_HOP),
     # low precision: 49152 of one parity, 32768 of both, over the right-hand sides
     ((16, 16, 16, 24), 0, 1, 1, lym.FORM_HOP), ((16, 16, 16, 24), 0, 2, 1, lym.FORM_HOP),
     ((16, 16, 16, 26), 0, 1, 1, lym.FORM_SPLIT), ((16, 16, 16, 26), 0, 2, 1, lym.FORM_SPLIT),
