@@ -11,9 +11,10 @@
 // time: every load of a site is in flight at once, one wait instead of five.
 // The direction waves leave their two colour vectors per hop in LDS; the
 // chirality waves sum the eight hops in the order of dslash.hip's accumulator and
-// finish spins 0, 1 and 2, 3 (the clover blocks and R^-1 are chiral).  The
-// operations and their order are those of the one-thread form, so both give the
-// same bits.  A fused update (x_s, r_s) is spread over all six waves.
+// finish spins 0, 1 and 2, 3 (the clover blocks and R^-1 are chiral).  A site's
+// operations and their order are those of the one-thread form, so outputs and a
+// batch's fused steps have the same bits in both (a single launch's norms and update
+// are summed in another order).  A fused update (x_s, r_s) is spread over all six waves.
 //
 // Measured (MI355X, against the one- or two-thread form): FP64 Wilson apply on
 // 8^4 9.1 -> 5.8 us, on 8^3x16 clover 12.0 -> 6.3 us; FP64 even-odd CG iteration

@@ -257,8 +257,8 @@ struct lym_op {
     double* dev_kappa;  // kappa in device memory, read by the stencil (captured launches stay valid across kappa changes)
     int gamma5;
     const lym_gauge* gauge;
-    double2* A;        // [2][36][stride] site-diagonal blocks of D (1 + kappa csw gamma5 B)
-    double2* Ainv;     // [36][stride] inverse blocks on even sites
+    double2* A;        // site-diagonal blocks of D without the 1 (kappa csw gamma5 B; BLK_A, BLK_A_REAL)
+    double2* Ainv;     // inverse blocks on even sites (BLK_INV, BLK_INV_REAL)
     int diag_dirty;
     double2* tmp;      // full-spinor scratch for squared operators
     double2* tmp2;     // half-spinor scratch for the Schur operator
@@ -268,9 +268,9 @@ struct lym_op {
     int sloppy_lk;     // link kind of the low-precision links
     void* Usf;         // all rows of the links in low precision (multi-RHS applies), when Us holds rows 0, 1
     void* Us;          // links
-    void* As;          // [2][36][stride] blocks
+    void* As;          // blocks, as A
     float* As_sc;      // [2][stride]
-    void* Ainvs;       // [36][stride]
+    void* Ainvs;       // inverse blocks, as Ainv
     float* Ainvs_sc;   // [stride]
     // spinor fields of lym_op_multiply_sloppy (in, out, Q^2 intermediate, even
     // Schur intermediate), sized for FP32 storage; allocated on first use

@@ -1,7 +1,13 @@
 // lym_stencil.h -- the hop arithmetic and the workgroup -> site-block mapping shared
 // by the stencil kernels (dslash.hip: one or two threads per site; dslash_hop.hip:
-// one wave per hop).  Every form runs the same operations in the same order on a
-// site, so a result does not depend on the form a launch takes.
+// one wave per direction).  The forms that launches of one kind choose between by size
+// run the same operations in the same order on a site, so that an FP64 apply and a
+// right-hand side of a batch have the same bits in any of them: k_dslash_stg,
+// k_dslash_lanes and k_dslash_hop in FP64; k_dslash (its batch steps included) and
+// k_dslash_hop in FP32 and FP16.  Others differ by rounding: k_dslash_split adds the
+// x and y hops and the z and t hops apart, k_dslash_mfma sums in the matrix cores, and
+// the fused update and the norms of single low-precision launches are formed and summed
+// as each form does it, so a single mixed-precision solve depends on the form.
 #pragma once
 
 #include "lym_device.h"
