@@ -7,7 +7,7 @@ eps = 0.5 from a seeded generator, Gaussian complex<double> spinors.  A step
 is one full-lattice FP64 clover apply Q psi = gamma5 (A psi - kappa H psi)
 (DiracOperator::multiply of ImprovedDiracWilsonOperator).  Inputs are resident
 in HBM; ROTATE independent (links, clover, in, out) sets are cycled so the
-working set (~604 MB) exceeds the 256 MB Infinity Cache.
+working set (~547 MB) exceeds the 256 MB Infinity Cache.
 
 value = algorithmic bytes / time, with 1536 B per site
   (4 links x 18 reals + spinor in 24 + out 24 + clover 72 reals, FP64), the

@@ -40,7 +40,7 @@ __device__ __forceinline__ void chunk_store(double v, double* partials, long nch
 // t + 512, then 256, ... 1.  All lanes (in groups of FG) load at once, and wave q of
 // the block runs lane q's tree, the steps down to 64 in registers and the rest by
 // shuffles (one lane after the other, with a barrier a step, 8 lanes of 16384 chunks
-// took 45 us and 4 lanes of small lattices 8 to 11, now below 10 and 3.5 to 4).
+// took 45 us and 4 lanes of small lattices 8 to 11, now 18 and 3.5 to 4).
 constexpr int FG = 8;
 template <int NR>
 __device__ __forceinline__ void final_sums(const double* partials, long nchunks, double* tot) {
