@@ -66,6 +66,7 @@ int dmalloc(lym_ctx* c, void** p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError();  // (reported here, not by the next launch)
         return fail(LYM_ERR_NOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
     }
     e = hipMemsetAsync(*p, 0, bytes, c->stream);

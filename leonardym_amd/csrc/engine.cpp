@@ -114,6 +114,7 @@ namespace {
 int ealloc(LaneEngine* e, void** p, size_t bytes) {
     if (hipMalloc(p, bytes) != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError();  // (reported here, not by the next launch)
         return fail(LYM_ERR_NOMEM, "serving engine: hipMalloc of %zu bytes", bytes);
     }
     e->allocs.push_back(*p);

@@ -177,20 +177,33 @@ struct LinOp {
     }
 };
 
-int ensure_work(lym_solver* s) {
-    if (s->w[0]) return LYM_OK;
-    const size_t bytes = sizeof(zd) * full_n(s->ctx);
-    for (int i = 0; i < 8; ++i) {
-        if (hipMalloc((void**)&s->w[i], bytes) != hipSuccess) return fail(LYM_ERR_NOMEM, "solver work vectors");
-        if (hipMemsetAsync(s->w[i], 0, bytes, s->ctx->stream) != hipSuccess) return fail(LYM_ERR_DEVICE, "hipMemsetAsync");
+// A zeroed device buffer, unless *p is there already.  An allocation that fails leaves
+// *p null, so that a later call, with memory free again, makes it.
+int dzalloc(lym_ctx* c, void** p, size_t bytes) {
+    if (*p) return LYM_OK;
+    if (hipMalloc(p, bytes) != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();  // (reported here, not by the next launch)
+        return fail(LYM_ERR_NOMEM, "solver buffer of %zu bytes", bytes);
     }
+    if (hipMemsetAsync(*p, 0, bytes, c->stream) != hipSuccess) return fail(LYM_ERR_DEVICE, "hipMemsetAsync");
+    return LYM_OK;
+}
+
+int ensure_work(lym_solver* s) {
+    if (s->host_state) return LYM_OK;  // the last of them
+    lym_ctx* c = s->ctx;
+    int rc = LYM_OK;
+    for (int i = 0; i < 8; ++i)
+        if ((rc = dzalloc(c, (void**)&s->w[i], sizeof(zd) * full_n(c)))) return rc;
     // one partial per workgroup of a stencil launch of both parities, however split
-    s->dot_stride = (int)std::max<long>(8192, 2 * (((long)s->ctx->g.Vh + 255) / 256));
-    if (hipMalloc((void**)&s->dot_part, 9 * sizeof(double) * (size_t)s->dot_stride) != hipSuccess)
-        return fail(LYM_ERR_NOMEM, "solver partials");
-    if (hipMalloc(&s->state, 256) != hipSuccess) return fail(LYM_ERR_NOMEM, "solver state");
-    if (hipHostMalloc(&s->host_state, 256, hipHostMallocDefault) != hipSuccess)
+    s->dot_stride = (int)std::max<long>(8192, 2 * (((long)c->g.Vh + 255) / 256));
+    if ((rc = dzalloc(c, (void**)&s->dot_part, 9 * sizeof(double) * (size_t)s->dot_stride))) return rc;
+    if ((rc = dzalloc(c, &s->state, 256))) return rc;
+    if (hipHostMalloc(&s->host_state, 256, hipHostMallocDefault) != hipSuccess) {
+        s->host_state = nullptr;
         return fail(LYM_ERR_DEVICE, "hipHostMalloc");
+    }
     return LYM_OK;
 }
 
@@ -501,6 +514,7 @@ int run_bicgstab(lym_solver* s, const LinOp& L, const zd* b, zd* xout, const zd*
 int ensure_mixed_work(lym_solver* s, int prec) {
     if (s->mixed_prec_alloc == prec) return LYM_OK;
     lym_ctx* c = s->ctx;
+    s->mixed_prec_alloc = 0;
     for (int i = 0; i < 4; ++i) {
         if (s->sv[i]) (void)hipFree(s->sv[i]);
         if (s->svsc[i]) (void)hipFree(s->svsc[i]);
@@ -512,20 +526,14 @@ int ensure_mixed_work(lym_solver* s, int prec) {
     s->xs = s->rs = nullptr;
     const size_t S = c->g.stride;
     const size_t es = prec == 1 ? 8 : 4;
+    int rc = LYM_OK;
     for (int i = 0; i < 4; ++i) {
-        if (hipMalloc(&s->sv[i], 24 * S * es) != hipSuccess) return fail(LYM_ERR_NOMEM, "sloppy vectors");
-        if (hipMalloc((void**)&s->svsc[i], 2 * S * sizeof(float)) != hipSuccess) return fail(LYM_ERR_NOMEM, "scales");
-        if (hipMemsetAsync(s->sv[i], 0, 24 * S * es, c->stream) != hipSuccess ||
-            hipMemsetAsync(s->svsc[i], 0, 2 * S * sizeof(float), c->stream) != hipSuccess)
-            return fail(LYM_ERR_DEVICE, "hipMemsetAsync");
+        if ((rc = dzalloc(c, &s->sv[i], 24 * S * es))) return rc;
+        if ((rc = dzalloc(c, (void**)&s->svsc[i], 2 * S * sizeof(float)))) return rc;
     }
-    if (hipMalloc((void**)&s->xs, 24 * S * 8) != hipSuccess || hipMalloc((void**)&s->rs, 24 * S * 8) != hipSuccess)
-        return fail(LYM_ERR_NOMEM, "FP32 vectors");
-    if (!s->upd_part && hipMalloc((void**)&s->upd_part, sizeof(double) * lym::NORM_FOLD_MAX) != hipSuccess)
-        return fail(LYM_ERR_NOMEM, "update partials");
-    if (hipMemsetAsync(s->xs, 0, 24 * S * 8, c->stream) != hipSuccess ||
-        hipMemsetAsync(s->rs, 0, 24 * S * 8, c->stream) != hipSuccess)
-        return fail(LYM_ERR_DEVICE, "hipMemsetAsync");
+    if ((rc = dzalloc(c, (void**)&s->xs, 24 * S * 8))) return rc;
+    if ((rc = dzalloc(c, (void**)&s->rs, 24 * S * 8))) return rc;
+    if ((rc = dzalloc(c, (void**)&s->upd_part, sizeof(double) * lym::NORM_FOLD_MAX))) return rc;
     s->mixed_prec_alloc = prec;
     return LYM_OK;
 }
@@ -671,27 +679,19 @@ void free_batch(lym_solver* s) {
     s->bdom = 0;
 }
 
-int dzalloc(lym_ctx* c, void** p, size_t bytes) {
-    if (hipMalloc(p, bytes) != hipSuccess) {
-        *p = nullptr;
-        return fail(LYM_ERR_NOMEM, "batch buffer of %zu bytes", bytes);
-    }
-    if (hipMemsetAsync(*p, 0, bytes, c->stream) != hipSuccess) return fail(LYM_ERR_DEVICE, "hipMemsetAsync");
-    return LYM_OK;
-}
-
 // buffers for batches of nr RHS over `dom` parities (1: even-odd, 2: full)
 int ensure_batch(lym_solver* s, int nr, int dom, int prec) {
     lym_ctx* c = s->ctx;
     int rc;
-    if (!s->bpartials) {
+    if (!s->bzero) {  // the last of them
         const size_t nch = (2 * (size_t)c->g.stride + lym::BATCH_CHUNK - 1) / lym::BATCH_CHUNK;
         if ((rc = dzalloc(c, (void**)&s->bpartials, sizeof(double) * lym::BMAX * nch))) return rc;
         if ((rc = dzalloc(c, &s->bstate, sizeof(lym::BState)))) return rc;
-        if (hipHostMalloc(&s->bhost, sizeof(lym::BState), hipHostMallocDefault) != hipSuccess)
+        if (!s->bhost && hipHostMalloc(&s->bhost, sizeof(lym::BState), hipHostMallocDefault) != hipSuccess)
             return fail(LYM_ERR_DEVICE, "hipHostMalloc");
         if ((rc = dzalloc(c, (void**)&s->bptr_dev, sizeof(zd*) * lym::BMAX))) return rc;
-        if (hipHostMalloc((void**)&s->bptr_host, sizeof(zd*) * lym::BMAX, hipHostMallocDefault) != hipSuccess)
+        if (!s->bptr_host &&
+            hipHostMalloc((void**)&s->bptr_host, sizeof(zd*) * lym::BMAX, hipHostMallocDefault) != hipSuccess)
             return fail(LYM_ERR_DEVICE, "hipHostMalloc");
         if ((rc = dzalloc(c, (void**)&s->bzero, sizeof(zd) * full_n(c)))) return rc;
     }
